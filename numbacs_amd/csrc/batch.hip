@@ -89,7 +89,8 @@ int launch_batch_queue(nbx_batch* b, const Flow& f, const LaunchCfg& cfg, hipStr
     const int block = cfg.block;
     if (cfg.persistent == 0) {
         if (b->total_slots == 0) return 0;
-        k_flowmap_tiles<Flow, R, G><<<blocks_for(b->total_slots * G, block), block, 0, s>>>(
+        k_flowmap_tiles<Flow, R, G><<<blocks_for(b->total_slots * G, block), block,
+                                    solve_lds_bytes<Flow, R, G>(block), s>>>(
             f, b->d_table, b->d_slot_off, b->nreq, b->total_slots, b->rtol, b->atol, b->nmax);
         NBX_LAUNCHED("flowmap_tiles (batch)");
         return 0;
@@ -101,7 +102,7 @@ int launch_batch_queue(nbx_batch* b, const Flow& f, const LaunchCfg& cfg, hipStr
     const unsigned long long ring = chunk_ring(ntiles);
     const size_t state_off = ring * sizeof(unsigned long long) + 256;
     NBX_REQUIRE(b->d_chunk != nullptr &&
-                    b->chunk_bytes >= state_off + sizeof(Dop853State<R>) * b->total_slots,
+                    b->chunk_bytes >= state_off + (solve_state_bytes<R, G>()) * b->total_slots,
                 "the batch's queue buffers are not allocated for this launch configuration");
     char* w = b->d_chunk;
     const ChunkQueue q{reinterpret_cast<unsigned long long*>(w),
@@ -114,9 +115,10 @@ int launch_batch_queue(nbx_batch* b, const Flow& f, const LaunchCfg& cfg, hipStr
     const int64_t want = (ntiles * 64 + block - 1) / block;
     const int64_t grid =
         std::max<int64_t>(1, std::min<int64_t>(want, static_cast<int64_t>(cus) * cfg.persistent));
-    k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(grid), block, 0, s>>>(
+    k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(grid), block,
+                                 solve_lds_bytes<Flow, R, G>(block), s>>>(
         f, ReqDev{}, b->d_table, b->d_slot_off, b->nreq, q,
-        reinterpret_cast<Dop853State<R>*>(w + state_off), b->rtol, b->atol, b->nmax);
+        reinterpret_cast<decltype(Solve<Flow, R, G>::s)*>(w + state_off), b->rtol, b->atol, b->nmax);
     NBX_LAUNCHED("flowmap_chunks (batch)");
     return 0;
 }
@@ -131,7 +133,8 @@ int ensure_chunk_buffers(nbx_batch* b) {
     const int64_t ntiles = b->total_slots / (64 / G);
     NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
     const size_t need = chunk_ring(ntiles) * sizeof(unsigned long long) + 256 +
-                        sizeof(Dop853State<double>) * static_cast<size_t>(b->total_slots);
+                        std::max(solve_state_bytes<double, 1>(), solve_state_bytes<double, 4>()) *
+                            static_cast<size_t>(b->total_slots);
     if (b->chunk_bytes >= need) return 0;
     if (b->d_chunk) (void)hipFree(b->d_chunk);
     b->d_chunk = nullptr;

@@ -25,6 +25,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
+
+#include "lanes.h"
 
 namespace nbx {
 namespace dop {
@@ -193,8 +196,8 @@ __device__ __forceinline__ void dop853_init(const Flow& f, Dop853State<R>& s, do
 // The head of one attempted step: the step budget and underflow checks and
 // the clipping of the last step to xend.  Sets s.idid != 0 and returns false
 // when the solve ends here; otherwise s.h is the step about to be taken.
-template <class R>
-__device__ __forceinline__ bool dop853_step_begin(Dop853State<R>& s, long long nmax) {
+template <class State>
+__device__ __forceinline__ bool dop853_step_begin(State& s, long long nmax) {
     using namespace dop;
     if (s.nstep > nmax) {
         s.idid = -2;
@@ -342,6 +345,244 @@ __device__ __forceinline__ bool dop853_step(const Flow& f, Dop853State<R>& s, do
                                             double atol, long long nmax) {
     if (!dop853_step_begin(s, nmax)) return false;
     return dop853_step_body(f, s, rtol, atol);
+}
+
+// ---------------------------------------------------------------------------
+// Component-per-lane form, for G = 2 or 4 lanes per particle: even lanes
+// hold x, odd lanes y (a 4-lane group holds each component twice), so a stage
+// sum is one chain of FMAs instead of two and a lane keeps ten stage values
+// instead of twenty.  A lane's flow evaluation takes its own coordinate and
+// returns its own velocity component; the functor exchanges what it needs
+// inside the group (Flow::component).  The error norms combine the two
+// components with one DPP exchange.  Every value is formed by the operations
+// of dop853_step_body in their order and as the compiler contracts them there
+// (written out as fma here: of each sum's first pair the second product is
+// rounded, but in stage 11 the first), so the two forms agree bit for bit.
+
+// x*x + y*y of a pair's components: the even lane forms fma(x, x, y*y), as
+// the two-component form's contracted sum, and both lanes take its result
+__device__ __forceinline__ double pair_sumsq(double e) {
+    return quad_move<kPairEven>(fma(e, e, quad_move<kPairOdd>(e * e)));
+}
+
+template <class R>
+struct Dop853Lane {
+    double x, xend, h, hmax, posneg;
+    double y;  // the lane's coordinate
+    R k1;
+    int nstep;
+    bool last, reject;
+    int idid;  // as Dop853State
+};
+
+template <class R, class Flow>
+__device__ __forceinline__ void dop853_init(const Flow& f, Dop853Lane<R>& s, double x,
+                                            double xend, double p0, double rtol, double atol) {
+    s.x = x;
+    s.xend = xend;
+    s.posneg = (xend - x) >= 0 ? 1.0 : -1.0;
+    s.hmax = fabs(xend - x);
+    s.last = false;
+    s.reject = false;
+    s.nstep = 0;
+    s.idid = 0;
+    s.y = p0;
+    s.k1 = f.component(x, p0, [] {});
+    const double f0 = static_cast<double>(s.k1);
+    const double sk = atol + rtol * fabs(p0);
+    const double dnf = pair_sumsq(f0 / sk);
+    const double dny = pair_sumsq(p0 / sk);
+    double h = (dnf <= 1.0e-10 || dny <= 1.0e-10) ? 1.0e-6 : sqrt(dny / dnf) * 0.01;
+    h = fmin(h, s.hmax);
+    h = s.posneg >= 0 ? fabs(h) : -fabs(h);
+    const double df = f.component_change(x + h, p0 + h * f0, f0);
+    const double der2 = sqrt(pair_sumsq(df / sk)) / h;
+    const double der12 = fmax(fabs(der2), sqrt(dnf));
+    const double h1 =
+        der12 <= 1.0e-15 ? fmax(1.0e-6, fabs(h) * 1.0e-3) : dop::root8(0.01 / der12);
+    h = fmin(fmin(100 * fabs(h), h1), s.hmax);
+    s.h = s.posneg >= 0 ? h : -h;
+}
+
+// Where a lane keeps its ten stage values (index 0..9: stages 1, 4..10, 11 and
+// 12; stages 2 and 3 are used once, at once).
+struct StageRegs {
+    double k[10];
+    __device__ __forceinline__ void put(int i, double v) { k[i] = v; }
+    __device__ __forceinline__ double get(int i) const { return k[i]; }
+};
+// In LDS, 512 bytes a stage and wavefront (kStageLdsBytes a wavefront, the
+// launch's dynamic LDS): each value is written once and read back where a sum
+// needs it, so the 20 vector registers it would hold stay free.  volatile, or
+// the compiler forwards the stores and keeps the registers.
+constexpr unsigned kStageLdsBytes = 10 * 64 * sizeof(double);
+extern __shared__ double stage_lds[];
+struct StageLds {
+    // (an LDS pointer: volatile accesses through a generic one stay flat)
+    using Slot = __attribute__((address_space(3))) volatile double;
+    Slot* at;
+    __device__ __forceinline__ StageLds()
+        : at((Slot*)stage_lds + (threadIdx.x >> 6) * 640 + (threadIdx.x & 63)) {}
+    __device__ __forceinline__ void put(int i, double v) const { at[64 * i] = v; }
+    __device__ __forceinline__ double get(int i) const { return at[64 * i]; }
+};
+
+// A stage's evaluation and, in the time its gathers are in flight, the part
+// of the next stage's sum that does not need it (`ahead`).
+template <class R, class Stages, class Flow>
+__device__ __forceinline__ bool dop853_step_body(const Flow& f, Dop853Lane<R>& s, Stages& ks,
+                                                 double rtol, double atol) {
+    using namespace dop;
+    ++s.nstep;
+    const double x = s.x, h = s.h, y = s.y;
+    auto F = [&](double t, double q, auto&& ahead) {
+        return static_cast<double>(f.component(t, q, ahead));
+    };
+    auto none = [] {};
+    double P;  // the next stage's sum but for its last term
+    const double K1 = static_cast<double>(s.k1);
+    ks.put(0, K1);
+    double K = F(x + c2 * h, fma(h * a21, K1, y), none);
+    K = F(x + c3 * h, fma(h, fma(a31, K1, a32 * K), y), none);
+    K = F(x + c4 * h, fma(h, fma(a41, K1, a43 * K), y), [&, K3 = K] { P = fma(a51, K1, a53 * K3); });
+    ks.put(1, K);
+    K = F(x + c5 * h, fma(h, fma(a54, K, P), y),
+          [&] { P = fma(a61, ks.get(0), a64 * ks.get(1)); });
+    ks.put(2, K);
+    K = F(x + c6 * h, fma(h, fma(a65, K, P), y),
+          [&] { P = fma(a75, ks.get(2), fma(a71, ks.get(0), a74 * ks.get(1))); });
+    ks.put(3, K);
+    K = F(x + c7 * h, fma(h, fma(a76, K, P), y), [&] {
+        P = fma(a86, ks.get(3),
+                fma(a85, ks.get(2), fma(a81, ks.get(0), a84 * ks.get(1))));
+    });
+    ks.put(4, K);
+    K = F(x + c8 * h, fma(h, fma(a87, K, P), y), [&] {
+        P = fma(a97, ks.get(4),
+                fma(a96, ks.get(3),
+                    fma(a95, ks.get(2), fma(a91, ks.get(0), a94 * ks.get(1)))));
+    });
+    ks.put(5, K);
+    K = F(x + c9 * h, fma(h, fma(a98, K, P), y), [&] {
+        P = fma(a108, ks.get(5),
+                fma(a107, ks.get(4),
+                    fma(a106, ks.get(3),
+                        fma(a105, ks.get(2), fma(a101, ks.get(0), a104 * ks.get(1))))));
+    });
+    ks.put(6, K);
+    K = F(x + c10 * h, fma(h, fma(a109, K, P), y), [&] {
+        P = fma(a119, ks.get(6),
+                fma(a118, ks.get(5),
+                    fma(a117, ks.get(4),
+                        fma(a116, ks.get(3), fma(a115, ks.get(2), fma(a114, ks.get(1), a111 * ks.get(0)))))));
+    });
+    ks.put(7, K);
+    K = F(x + c11 * h, fma(h, fma(a1110, K, P), y), [&] {
+        P = fma(a1210, ks.get(7),
+                fma(a129, ks.get(6),
+                    fma(a128, ks.get(5),
+                        fma(a127, ks.get(4),
+                            fma(a126, ks.get(3),
+                                fma(a125, ks.get(2),
+                                    fma(a121, ks.get(0), a124 * ks.get(1))))))));
+    });
+    ks.put(8, K);
+    const double xph = x + h;
+    double B, E;  // the update's and the fifth-order error's sums but for the last term
+    K = F(xph, fma(h, fma(a1211, K, P), y), [&] {
+        const double k1 = ks.get(0), k6 = ks.get(3), k7 = ks.get(4), k8 = ks.get(5),
+                     k9 = ks.get(6), k10 = ks.get(7), k11 = ks.get(8);
+        B = fma(b11, k11,
+                fma(b10, k10, fma(b9, k9, fma(b8, k8, fma(b7, k7, fma(b1, k1, b6 * k6))))));
+        E = fma(er11, k11,
+                fma(er10, k10,
+                    fma(er9, k9, fma(er8, k8, fma(er7, k7, fma(er1, k1, er6 * k6))))));
+    });
+    const double k4n = fma(b12, K, B);
+    const double pn = fma(h, k4n, y);
+    const double sk = fma(rtol, fmax(fabs(y), fabs(pn)), atol);
+    const double rsk = div_recip(sk);
+    const double e2 = div_with(
+        fma(-bhh3, K, fma(-bhh2, ks.get(6), fma(-bhh1, ks.get(0), k4n))), sk, rsk);
+    const double e5 = div_with(fma(er12, K, E), sk, rsk);
+    const double err2 = pair_sumsq(e2);
+    double err = pair_sumsq(e5);
+    double deno = fma(0.01, err2, err);
+    if (deno <= 0.0) deno = 1.0;
+    err = fabs(h) * err * sqrt(1.0 / (2 * deno));
+    const double fac = dop::root8(err) / safe;
+    const bool accept = err <= 1.0;
+    double hnew = h / (accept ? fmax(facc2, fmin(facc1, fac)) : fmin(facc1, fac));
+    if (accept) {
+        s.y = pn;
+        s.k1 = f.component(xph, pn, none);
+        s.x = xph;
+        if (s.last) {
+            s.idid = 1;
+            return false;
+        }
+        if (fabs(hnew) > s.hmax) hnew = s.posneg * s.hmax;
+        if (s.reject) hnew = s.posneg * fmin(fabs(hnew), fabs(h));
+        s.reject = false;
+    } else {
+        s.reject = true;
+        s.last = false;
+    }
+    s.h = hnew;
+    return true;
+}
+
+
+// The solver of a group of G lanes, as the launches use it: one lane holds
+// both components, two or four lanes one component each.
+template <class Flow, class R, int G>
+struct Solve {
+    static constexpr int kStates = 2;  // states a group hands on (one per component)
+    static constexpr unsigned kLdsBytes = Flow::kStagesInLds ? kStageLdsBytes : 0;  // a wavefront
+    Dop853Lane<R> s;
+    std::conditional_t<Flow::kStagesInLds, StageLds, StageRegs> ks;
+    __device__ __forceinline__ void init(const Flow& f, double x, double xend, double px,
+                                         double py, double rtol, double atol) {
+        dop853_init(f, s, x, xend, (__lane_id() & 1) ? py : px, rtol, atol);
+    }
+    __device__ __forceinline__ bool body(const Flow& f, double rtol, double atol) {
+        return dop853_step_body(f, s, ks, rtol, atol);
+    }
+    // one attempted step: false when the solve has ended (s.idid says how)
+    __device__ __forceinline__ bool step(const Flow& f, double rtol, double atol, long long nmax) {
+        return dop853_step_begin(s, nmax) && body(f, rtol, atol);
+    }
+    // the group's final position: lanes 0 and 1 write x and y
+    __device__ __forceinline__ void store(double2* out) const {
+        const unsigned g = __lane_id() & (G - 1);
+        if (g < 2) reinterpret_cast<double*>(out)[g] = s.y;
+    }
+};
+template <class Flow, class R>
+struct Solve<Flow, R, 1> {
+    static constexpr int kStates = 1;
+    static constexpr unsigned kLdsBytes = 0;
+    Dop853State<R> s;
+    __device__ __forceinline__ void init(const Flow& f, double x, double xend, double px,
+                                         double py, double rtol, double atol) {
+        dop853_init(f, s, x, xend, px, py, rtol, atol);
+    }
+    __device__ __forceinline__ bool step(const Flow& f, double rtol, double atol, long long nmax) {
+        return dop853_step(f, s, rtol, atol, nmax);
+    }
+    __device__ __forceinline__ void store(double2* out) const {
+        *out = make_double2(s.px(), s.py());
+    }
+};
+// dynamic LDS of a launch with `block` threads a block
+template <class Flow, class R, int G>
+constexpr unsigned solve_lds_bytes(int block) {
+    return block / 64 * Solve<Flow, R, G>::kLdsBytes;
+}
+// what the launches' hand-over buffers hold per particle slot
+template <class R, int G>
+constexpr size_t solve_state_bytes() {
+    return G == 1 ? sizeof(Dop853State<R>) : 2 * sizeof(Dop853Lane<R>);
 }
 
 }  // namespace nbx

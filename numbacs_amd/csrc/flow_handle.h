@@ -54,10 +54,13 @@ Spline3<R, 1, L> make_spline(const nbx_flow* fl, double p0) {
         const int n = static_cast<int>(fl->grid9[3 * d + 2]);
         s.dinv[d] = (n - 1) / (s.hi[d] - s.lo[d]);
         s.nm2[d] = n - 2;
+        s.nm2d[d] = n - 2;
     }
     const int nx = static_cast<int>(fl->grid9[5]), ny = static_cast<int>(fl->grid9[8]);
     s.sx = ny + 2;
     s.st = (nx + 2) * (ny + 2);
+    s.sxd = s.sx;
+    s.std_ = s.st;
     s.spherical = fl->spherical;
     s.extrap = fl->extrap;
     s.r = fl->r;
@@ -94,9 +97,12 @@ Spline3<R, G, false, S> regroup(const Spline3<R, 1, false>& a) {
         s.hi[d] = a.hi[d];
         s.dinv[d] = a.dinv[d];
         s.nm2[d] = a.nm2[d];
+        s.nm2d[d] = a.nm2d[d];
     }
     s.sx = a.sx;
     s.st = a.st;
+    s.sxd = a.sxd;
+    s.std_ = a.std_;
     s.cbytes = a.cbytes;
     s.spherical = a.spherical;
     s.extrap = a.extrap;

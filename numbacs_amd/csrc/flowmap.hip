@@ -281,12 +281,10 @@ struct AuxSource {
 // One solve per group of G lanes (G = 1 for analytic flows); the group's
 // lanes run identical solver arithmetic and split the spline gathers.
 template <class Flow, class R, int G, class Src>
-__global__ __launch_bounds__(256, NBX_FLOWMAP_MIN_WAVES) void k_flowmap(Flow f, Src src, int64_t P, double s0, double s1,
-                                                 double rtol, double atol,
-                                                 const uint8_t* __restrict__ mask, long long nmax,
-                                                 double2* __restrict__ out,
-                                                 int32_t* __restrict__ status,
-                                                 int32_t* __restrict__ nsteps) {
+__global__ __launch_bounds__(256, (flowmap_min_waves<Flow, R, G>())) void k_flowmap(
+    Flow f, Src src, int64_t P, double s0, double s1, double rtol, double atol,
+    const uint8_t* __restrict__ mask, long long nmax, double2* __restrict__ out,
+    int32_t* __restrict__ status, int32_t* __restrict__ nsteps) {
     f.prepare();
     const unsigned bid = xcd_block<Flow>();
     const int64_t tid = bid * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -307,12 +305,13 @@ __global__ __launch_bounds__(256, NBX_FLOWMAP_MIN_WAVES) void k_flowmap(Flow f, 
         }
         return;
     }
-    Dop853State<R> s;
-    dop853_init(f, s, s0, s1, px, py, rtol, atol);
-    while (dop853_step(f, s, rtol, atol, nmax)) {
+    Solve<Flow, R, G> sv;
+    auto& s = sv.s;
+    sv.init(f, s0, s1, px, py, rtol, atol);
+    while (sv.step(f, rtol, atol, nmax)) {
     }
+    sv.store(out + p);
     if (lead) {
-        out[p] = make_double2(s.px(), s.py());
         if (status) status[p] = s.idid;
         if (nsteps) nsteps[p] = s.nstep;
     }
@@ -379,15 +378,16 @@ __global__ __launch_bounds__(64) void k_flowmap_staged(
     }
     f.box.lds = stage;
     f.box.on = false;
-    Dop853State<R> s;
+    Solve<Spline3<R, 4, false, true>, R, 4> sv;
+    auto& s = sv.s;
     if (running) {
         double px, py;
         src.pos(p, px, py);
-        dop853_init(f, s, s0, s1, px, py, rtol, atol);
+        sv.init(f, s0, s1, px, py, rtol, atol);
     }
     auto finish = [&]() {
+        sv.store(out + p);
         if (lead) {
-            out[p] = make_double2(s.px(), s.py());
             if (status) status[p] = s.idid;
             if (nsteps) nsteps[p] = s.nstep;
         }
@@ -409,10 +409,10 @@ __global__ __launch_bounds__(64) void k_flowmap_staged(
             const double t0 = f.p0 * s.x, t1 = f.p0 * (s.x + s.h);
             tlo = fmin(t0, t1);
             thi = fmax(t0, t1);
-            const double ex = s.h * static_cast<double>(s.k1x);
-            const double ey = s.h * static_cast<double>(s.k1y);
+            const double e = s.h * static_cast<double>(s.k1);
+            const double ex = quad_move<kPairEven>(e), ey = quad_move<kPairOdd>(e);
             const double m = 0.5 * (fabs(ex) + fabs(ey));
-            const double px = s.px(), py = s.py();
+            const double px = quad_move<kPairEven>(s.y), py = quad_move<kPairOdd>(s.y);
             const double a = f.lookup_x(px + fmin(0.0, ex) - m);
             const double b = f.lookup_x(px + fmax(0.0, ex) + m);
             if (a <= b) {
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(64) void k_flowmap_staged(
         }
         __syncthreads();
         if (stepping) {
-            running = dop853_step_body(f, s, rtol, atol);
+            running = sv.body(f, rtol, atol);
             if (!running) finish();
         }
         __syncthreads();  // every read of the box is done before the next copy
@@ -552,7 +552,7 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
             const unsigned long long ring = chunk_ring(ntiles);
             const size_t state_off = ring * sizeof(unsigned long long) + 256;
-            Workspace ws(s, 3, state_off + sizeof(Dop853State<R>) * static_cast<size_t>(slots));
+            Workspace ws(s, 3, state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots));
             if (ws.error()) return ws.error();
             char* w = ws.get();
             const ChunkQueue q{reinterpret_cast<unsigned long long*>(w),
@@ -564,16 +564,18 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             NBX_LAUNCHED("chunk_init");
             const int64_t want = (ntiles * 64 + block - 1) / block;
             const int64_t grid = std::min<int64_t>(want, static_cast<int64_t>(cus) * cfg.persistent);
-            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(grid), block, 0, s>>>(
+            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(grid), block,
+                                         solve_lds_bytes<Flow, R, G>(block), s>>>(
                 f, single_request(src, a), nullptr, nullptr, 1, q,
-                reinterpret_cast<Dop853State<R>*>(w + state_off), a.rtol, a.atol, a.nmax);
+                reinterpret_cast<decltype(Solve<Flow, R, G>::s)*>(w + state_off), a.rtol, a.atol, a.nmax);
             NBX_LAUNCHED("flowmap_chunks");
             return 0;
         }
     }
     int64_t slots = a.P;
     if constexpr (std::is_same<Src, GridSource>::value) slots = src.slots();
-    k_flowmap<Flow, R, G, Src><<<blocks_for(slots * G, block), block, 0, s>>>(
+    k_flowmap<Flow, R, G, Src><<<blocks_for(slots * G, block), block,
+                                 solve_lds_bytes<Flow, R, G>(block), s>>>(
         f, src, slots, a.s0, a.s1, a.rtol, a.atol, a.mask, a.nmax, a.out, a.status, a.nsteps);
     NBX_LAUNCHED("flowmap");
     return 0;

@@ -13,6 +13,8 @@
 #include <cmath>
 #include <type_traits>
 
+#include "lanes.h"
+
 namespace nbx {
 
 constexpr double kPi = 3.141592653589793;
@@ -157,6 +159,19 @@ __device__ __forceinline__ double py_mod(double a, double m) {
     return r;
 }
 
+// py_mod out of line, for arguments a period or more away
+__device__ __attribute__((noinline)) static double py_mod_far(double a, double m) {
+    return py_mod(a, m);
+}
+
+// py_mod(a, 360): within a period the sum needs no branch (a zero keeps the
+// divisor's sign, as copysign gives it: -0.0 + 0.0 is +0.0)
+__device__ __forceinline__ double wrap360(double a) {
+    double r = a + (a < 0 ? 360.0 : 0.0);
+    if (__builtin_expect(!(fabs(a) < 360.0), 0)) r = py_mod_far(a, 360.0);
+    return r;
+}
+
 // Degrees to radians as the reference writes it, (deg * pi) / 180: the
 // quotient by 180 is the product with the rounded reciprocal plus one FMA
 // correction (Markstein), which is the correctly rounded quotient -- equal
@@ -193,11 +208,15 @@ __device__ __forceinline__ double fma_coef(double a, double b, double c) {
 #endif
 }
 
+// The library cosine, out of line: inlined into the flow-map kernels, its
+// polynomial constants were held in 18 vector registers through the whole
+// solve for a path that no latitude takes.
+__device__ __attribute__((noinline)) static double cos_far(double x) { return cos(x); }
+
 __device__ __forceinline__ double cos_lat(double x) {
     constexpr double pio2_hi = 1.5707963267948966;      // double nearest pi/2
     constexpr double pio2_lo = 6.123233995736766e-17;   // pi/2 - pio2_hi
     const double ax = fabs(x);
-    if (ax > 2 * pio2_hi) return cos(x);
     const double u = (pio2_hi - ax) + pio2_lo;
     const double s = u * u;
     double p = 1.0 / 15511210043330985984000000.0;      // 1/25!
@@ -212,7 +231,9 @@ __device__ __forceinline__ double cos_lat(double x) {
     p = fma_coef(p, s, -1.0 / 5040.0);                       // -1/7!
     p = fma_coef(p, s, 1.0 / 120.0);                         // 1/5!
     p = fma_coef(p, s, -1.0 / 6.0);                          // -1/3!
-    return fma(u * s, p, u);
+    double r = fma(u * s, p, u);
+    if (__builtin_expect(ax > 2 * pio2_hi, 0)) r = cos_far(x);
+    return r;
 }
 
 // The float form's latitude cosine: the same reduction in float, Taylor to
@@ -242,42 +263,22 @@ template <class R> struct CoefPair;
 template <> struct CoefPair<double> { using type = double2; };
 template <> struct CoefPair<float> { using type = float4; };
 
-// Sum of a value over the G lanes of an aligned lane group, with a butterfly
-// of DPP quad permutations, so every lane of the group ends with the same
-// bits (the additions are commutative pairwise, and each level combines the
-// same two partial sums in every lane).  The empty asm materialises v first:
-// otherwise the compiler may fuse the multiply that produced v into the
-// first add (fma(a, b, other lane's rounded a*b)), and the lanes of a group
-// would then round differently and take different step-size decisions.
-template <int G>
-__device__ __forceinline__ float group_sum(float v) {
+// Sums of u and of v over the G lanes of an aligned lane group, the sum of u
+// left in the even lanes and that of v in the odd ones (a reduce-scatter of
+// DPP quad permutations: each lane keeps the component it integrates and sends
+// the other).  Every lane of a parity ends with the same bits: the additions
+// are commutative pairwise, and each level combines the same two partial sums.
+// The empty asm materialises u and v first: otherwise the compiler may fuse
+// the multiply that produced them into the first add (fma(a, b, other lane's
+// rounded a*b)), and the lanes of a group would then round differently and
+// take different step-size decisions.
+template <int G, class R>
+__device__ __forceinline__ R group_component(R u, R v, bool odd) {
+    asm volatile("" : "+v"(u));
     asm volatile("" : "+v"(v));
-    if constexpr (G >= 2)
-        v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-    if constexpr (G >= 4)
-        v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, false));
-    return v;
-}
-
-template <int G>
-__device__ __forceinline__ double group_sum(double v) {
-    auto xchg = [](double a, int ctrl) {
-        const long long b = __double_as_longlong(a);
-        int lo = static_cast<int>(b & 0xffffffffll), hi = static_cast<int>(b >> 32);
-        if (ctrl == 0xB1) {
-            lo = __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xF, 0xF, false);
-            hi = __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xF, 0xF, false);
-        } else {
-            lo = __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xF, 0xF, false);
-            hi = __builtin_amdgcn_mov_dpp(hi, 0x4E, 0xF, 0xF, false);
-        }
-        return __longlong_as_double((static_cast<long long>(hi) << 32) |
-                                    static_cast<unsigned int>(lo));
-    };
-    asm volatile("" : "+v"(v));
-    if constexpr (G >= 2) v += xchg(v, 0xB1);
-    if constexpr (G >= 4) v += xchg(v, 0x4E);
-    return v;
+    R s = (odd ? v : u) + quad_move<kPairSwap>(odd ? u : v);
+    if constexpr (G == 4) s += quad_move<kQuadCross>(s);
+    return s;
 }
 
 // Tricubic natural B-spline velocity on a uniform (t, x, y) grid (the
@@ -285,7 +286,7 @@ __device__ __forceinline__ double group_sum(double v) {
 // C holds (nt+2, nx+2, ny+2) (u, v) pairs, y fastest.  R is the coefficient
 // and evaluation precision (double for the plain path, float for the
 // FP32-displacement form).  G lanes (1, 2 or 4, aligned in the wavefront)
-// share one evaluation and combine partial sums with group_sum:
+// share one evaluation and combine partial sums with group_component:
 //   G = 2: lane g gathers the t-slices a with a % 2 == g (whole 4-pair rows);
 //   G = 4: lane g gathers y-coefficient g of all 16 rows, so one load
 //          instruction covers one contiguous row per particle -- a third of
@@ -314,6 +315,31 @@ __device__ __forceinline__ double in_vgpr(double x) {
     return y;
 }
 
+// Bare minimum and maximum: fmin and fmax first quiet each operand whose
+// origin the compiler cannot see (a v_max_f64 apiece).  Same values, NaN
+// included: a quiet NaN yields the other operand.
+__device__ __forceinline__ double raw_min(double a, double b) {
+#if __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmin(a, b);
+#endif
+}
+__device__ __forceinline__ double raw_max(double a, double b) {
+#if __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmax(a, b);
+#endif
+}
+__device__ __forceinline__ double clamped(double q, double lo, double hi) {
+    return raw_min(raw_max(q, lo), hi);
+}
+
 // A box of coefficient elements copied to LDS by a one-wavefront block for
 // the stencils of one DOP853 step (cells it0.., ix0.., iy0.. of the
 // coefficient array, bt x bx x by elements, y fastest): a stencil whose 4 x 4
@@ -339,6 +365,7 @@ struct Spline3 {
     std::conditional_t<S, StageBox<P>, NoStageBox> box;
     double lo[3], hi[3], dinv[3];
     int nm2[3];   // n - 2 per axis: the largest cell index
+    double nm2d[3], sxd, std_;  // nm2, sx and st as doubles (the held form's cells)
     int sx, st;   // strides (in pairs) of the x and t axes
     int spherical, extrap;
     double r;     // sphere radius (km) for spherical = 1, 2
@@ -349,9 +376,12 @@ struct Spline3 {
     // the same cell as the particle's previous one reads registers instead
     // of the cache hierarchy (the kernel's own copy of the functor holds it)
     static constexpr bool kReuse = (G == 4) && !S;
+    // the FP64 form has no vector registers left for the solver's stages (at
+    // three wavefronts per SIMD)
+    static constexpr bool kStagesInLds = kReuse && sizeof(R) == sizeof(double);
     static constexpr int kRows = sizeof(R) == sizeof(double) ? 16 : 8;
     mutable P cst[kReuse ? kRows : 1];
-    mutable long ckey = -1;
+    mutable double ckey = -1;
     // bytes of C (the 4-lane form's buffer loads: under 4 GiB, checked by
     // the dispatcher)
     unsigned cbytes = 0;
@@ -380,6 +410,74 @@ struct Spline3 {
         k = k < 0 ? 0 : k;
         i = k;
         s = static_cast<R>(u - k);
+    }
+
+    // position u in cells of coordinate d, clamped into the box (so u >= 0 and
+    // truncation is floor), and its cell k as a whole double: no conversions
+    // to and from integers
+    __device__ __forceinline__ void locate(int d, double q, double& u, double& k) const {
+        u = (q - lo[d]) * dinv[d];
+        k = raw_min(trunc(u), nm2d[d]);
+    }
+
+    // kReuse: have the lane hold its y-column of the stencil at element `key`
+    // (a whole double, below 2^28)
+    __device__ __forceinline__ void hold(double key, bool skip) const {
+        if (skip | (key == ckey)) return;
+        ckey = key;
+        // buffer loads: the lane's origin is the vector offset, each row's
+        // offset a scalar one (no per-load address arithmetic, and no 64-bit
+        // row pointers held in scalar registers)
+        const int g = static_cast<int>(__lane_id() & 3);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<P*>(C), 0, static_cast<int>(cbytes), 0x00020000);
+        // (time slices step the vector offset, x rows are the scalar offsets:
+        // three live scalars, not sixteen)
+        const int vo = (static_cast<int>(key) + g) * static_cast<int>(sizeof(P));
+        const int tstep =
+            (sizeof(R) == sizeof(double) ? 1 : 2) * st * static_cast<int>(sizeof(P));
+        const int xstep = sx * static_cast<int>(sizeof(P));
+#pragma unroll
+        for (int a = 0; a < kRows / 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const auto raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, vo + a * tstep,
+                                                                       b * xstep, 0);
+                __builtin_memcpy(&cst[a * 4 + b], &raw, sizeof(P));
+            }
+    }
+
+    // the lane's component of the stencil sum over the held column: the sums
+    // of column_sums, the y-weight applied last
+    __device__ __forceinline__ R held_sum(const double u[3], const double k[3], bool odd) const {
+        R wt[4], wx[4], wy[4];
+        bspline_weights6(static_cast<R>(u[0] - k[0]), wt);
+        bspline_weights6(static_cast<R>(u[1] - k[1]), wx);
+        bspline_weights6(static_cast<R>(u[2] - k[2]), wy);
+        R au = 0, av = 0;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            R ru = 0, rv = 0;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                R cu, cv;
+                if constexpr (sizeof(R) == sizeof(double)) {
+                    const P e = cst[a * 4 + b];
+                    cu = e.x;
+                    cv = e.y;
+                } else {
+                    const P e = cst[(a >> 1) * 4 + b];
+                    cu = (a & 1) ? e.z : e.x;
+                    cv = (a & 1) ? e.w : e.y;
+                }
+                ru = fma(wx[b], cu, ru);
+                rv = fma(wx[b], cv, rv);
+            }
+            au = fma(wt[a], ru, au);
+            av = fma(wt[a], rv, av);
+        }
+        const R wc = pick4(wy, static_cast<int>(__lane_id() & 3)) * R(1.0 / 216.0);
+        return group_component<G>(au * wc, av * wc, odd);
     }
 
     // (u, v) of stencil time slice a (0..3), x row b, y column c, relative
@@ -440,7 +538,8 @@ struct Spline3 {
         }
     }
 
-    // (u, v) at an in-box point
+    // (u, v) at an in-box point; in a lane group the lane's own component
+    // (u in even lanes, v in odd ones), as su
     __device__ __forceinline__ void eval_in(double qt, double qx, double qy, R& su,
                                             R& sv) const {
         int it, ix, iy;
@@ -487,53 +586,6 @@ struct Spline3 {
                                   (iy - box.iy0) + g;
                     column_sums(lb, box.bx * box.by, box.by, wt, wx, au, av);
                 }
-            } else if constexpr (kReuse) {
-                const long key = static_cast<long>(it) * st + static_cast<long>(ix) * sx + iy;
-                if (key != ckey) {
-                    ckey = key;
-                    // buffer loads: the lane's origin is the vector offset,
-                    // each row's offset a scalar one (no per-load address
-                    // arithmetic, and no 64-bit row pointers held in
-                    // scalar registers)
-                    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-                        const_cast<P*>(C), 0, static_cast<int>(cbytes), 0x00020000);
-                    // (time slices step the vector offset, x rows are the
-                    // scalar offsets: three live scalars, not sixteen)
-                    const int vo = static_cast<int>((key + g) * static_cast<long>(sizeof(P)));
-                    const int tstep = (sizeof(R) == sizeof(double) ? 1 : 2) * st *
-                                      static_cast<int>(sizeof(P));
-                    const int xstep = sx * static_cast<int>(sizeof(P));
-#pragma unroll
-                    for (int a = 0; a < kRows / 4; ++a)
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) {
-                            const auto raw = __builtin_amdgcn_raw_buffer_load_b128(
-                                rsrc, vo + a * tstep, b * xstep, 0);
-                            __builtin_memcpy(&cst[a * 4 + b], &raw, sizeof(P));
-                        }
-                }
-                // the same sums as column_sums over the held rows
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    R ru = 0, rv = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        R cu, cv;
-                        if constexpr (sizeof(R) == sizeof(double)) {
-                            const P e = cst[a * 4 + b];
-                            cu = e.x;
-                            cv = e.y;
-                        } else {
-                            const P e = cst[(a >> 1) * 4 + b];
-                            cu = (a & 1) ? e.z : e.x;
-                            cv = (a & 1) ? e.w : e.y;
-                        }
-                        ru = fma(wx[b], cu, ru);
-                        rv = fma(wx[b], cv, rv);
-                    }
-                    au = fma(wt[a], ru, au);
-                    av = fma(wt[a], rv, av);
-                }
             } else {
                 column_sums(base + g, st, sx, wt, wx, au, av);
             }
@@ -559,8 +611,13 @@ struct Spline3 {
                 }
             }
         }
-        su = group_sum<G>(au);
-        sv = group_sum<G>(av);
+        if constexpr (G == 1) {
+            su = au;
+            sv = av;
+        } else {
+            su = group_component<G>(au, av, __lane_id() & 1);
+            sv = 0;
+        }
     }
 
     // value and gradient (d/dt, d/dx, d/dy) at an in-box point; every lane
@@ -641,9 +698,86 @@ struct Spline3 {
     // the x lookup coordinate of a position: the longitude wrapped into
     // [-180, 180) (spherical=1) or [0, 360) (spherical=2), else itself
     __device__ __forceinline__ double lookup_x(double y0) const {
-        if (spherical == 1) return py_mod(y0 - 180, 360) - 180;
-        if (spherical != 0) return py_mod(y0, 360);
+        if (spherical == 1) return wrap360(y0 - 180) - 180;
+        if (spherical != 0) return wrap360(y0);
         return y0;
+    }
+
+    // the latitude's cosine, in R
+    __device__ __forceinline__ static R lat_cos(double y) {
+        if constexpr (sizeof(R) == sizeof(double)) return cos_lat(deg_to_rad(y));
+        else return cos_lat(static_cast<float>(y) * static_cast<float>(kPi / 180));
+    }
+
+    // What a lane of a group of 2 or 4 brings to its component of the
+    // right-hand side at time t (yc: the lane's coordinate): the spline sum s
+    // and the divisor of the degree conversion (one for the meridional
+    // component, which is exact) with its reciprocal.  By the operations of
+    // operator().  In the held form everything that does not need the
+    // stencil -- the caller's `ahead`, the cosine, the reciprocal -- stands
+    // between the gathers and the sums.
+    struct Parts {
+        R s, den;
+        double recip;
+    };
+    template <class Ahead>
+    __device__ __forceinline__ Parts parts(double t, double yc, Ahead&& ahead) const {
+        static_assert(G > 1 && !L, "one lane holds both components");
+        const bool odd = __lane_id() & 1;
+        const double y1 = quad_move<kPairOdd>(yc);
+        const double tt = p0 * t, xx = lookup_x(quad_move<kPairEven>(yc));
+        Parts r;
+        if constexpr (kReuse) {
+            const double ct = clamped(tt, lo[0], hi[0]);
+            const double cx = clamped(xx, lo[1], hi[1]);
+            const double cy = clamped(y1, lo[2], hi[2]);
+            const bool zero = extrap != 2 && !((ct == tt) & (cx == xx) & (cy == y1));
+            double u[3], k[3];
+            locate(0, ct, u[0], k[0]);
+            locate(1, cx, u[1], k[1]);
+            locate(2, cy, u[2], k[2]);
+            hold(fma(k[0], std_, fma(k[1], sxd, k[2])), zero);
+            ahead();
+            if (spherical != 0) divide_by(odd, y1, r);
+            // (outside the box the sums run on the held column and are
+            // dropped: a branch around them costs more than they do)
+            const R v = held_sum(u, k, odd);
+            r.s = zero ? R(0) : v;
+        } else {
+            R unused;
+            eval(tt, xx, y1, r.s, unused);
+            ahead();
+            if (spherical != 0) divide_by(odd, y1, r);
+        }
+        return r;
+    }
+    __device__ __forceinline__ void divide_by(bool odd, double y1, Parts& r) const {
+        const R c = lat_cos(y1);
+        r.den = odd ? R(1) : c;
+        if constexpr (sizeof(R) == sizeof(double)) r.recip = div_recip(r.den);
+    }
+    __device__ __forceinline__ R degrees(const Parts& r) const {
+        if constexpr (sizeof(R) == sizeof(double)) return div_with(kdeg * r.s, r.den, r.recip);
+        else return (static_cast<float>(kdeg) * r.s) / r.den;
+    }
+
+    // the lane's component of the right-hand side
+    template <class Ahead>
+    __device__ __forceinline__ R component(double t, double yc, Ahead&& ahead) const {
+        const Parts r = parts(t, yc, ahead);
+        if (spherical == 0) return static_cast<R>(p0 * static_cast<double>(r.s));
+        return degrees(r);
+    }
+    // component(t, yc) - f0, rounded as operator()'s result is where the
+    // solver's initial step subtracts it in place (the meridional product
+    // contracted with the subtraction)
+    __device__ __forceinline__ double component_change(double t, double yc, double f0) const {
+        const Parts r = parts(t, yc, [] {});
+        if (spherical == 0) return static_cast<double>(static_cast<R>(p0 * static_cast<double>(r.s))) - f0;
+        const double d = static_cast<double>(degrees(r)) - f0;
+        if constexpr (sizeof(R) == sizeof(double))
+            return (__lane_id() & 1) ? fma(kdeg, r.s, -f0) : d;
+        return d;
     }
 
     __device__ __forceinline__ void operator()(double t, double y0, double y1, R& f0,

@@ -39,12 +39,6 @@
 #include "dop853.h"
 #include "flows.h"
 
-// Minimum wavefronts per SIMD requested from the compiler for the flow-map
-// kernels (caps their VGPR budget at 512 / n registers).
-#ifndef NBX_FLOWMAP_MIN_WAVES
-#define NBX_FLOWMAP_MIN_WAVES 1
-#endif
-
 namespace nbx {
 
 // Particle order of the one-solve-per-group grid launch: 8 x 8 tiles of the
@@ -89,6 +83,17 @@ template <class T>
 struct IsSpline3 : std::false_type {};
 template <class R, int G, bool L, bool S>
 struct IsSpline3<Spline3<R, G, L, S>> : std::true_type {};
+
+// Minimum wavefronts per SIMD asked of the compiler for a flow-map kernel
+// (it caps the vector registers at 512 / n).  The 4-lane spline forms hold
+// their stencil column in registers and wait on its gathers, so a further
+// wavefront is worth a few spilled bytes: float, 4 wavefronts at 128 registers,
+// batched time series 4.97 -> 4.24 ms; FP64, 3 at 168 (natural 175), gridded
+// flow map, FTLE and ridges 1.77 -> 1.67 ms (676 x 251 particles).
+template <class Flow, class R, int G>
+constexpr int flowmap_min_waves() {
+    return IsSpline3<Flow>::value && G == 4 ? (sizeof(R) == 4 ? 4 : 3) : 1;
+}
 
 // The work block of this block in a tile launch over a spline flow.
 // Consecutive blocks go to the eight XCDs in turn; XCD x is given the work
@@ -223,10 +228,10 @@ int device_cu_count();
 // solver state per slot.  Masked particles are written at their tile's first
 // chunk; a particle's outputs are written when its solve ends.
 template <class Flow, class R, int G>
-__global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : NBX_FLOWMAP_MIN_WAVES) void k_flowmap_chunks(
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 1) void k_flowmap_chunks(
     Flow f, ReqDev single, const ReqDev* __restrict__ table, const int64_t* __restrict__ slot_off,
-    int nreq, ChunkQueue q, Dop853State<R>* __restrict__ state, double rtol, double atol,
-    long long nmax) {
+    int nreq, ChunkQueue q, decltype(Solve<Flow, R, G>::s)* __restrict__ state, double rtol,
+    double atol, long long nmax) {
     constexpr int kSlots = 64 / G;
     // (only the factors, in FP64: this kernel's solver state, tile
     // bookkeeping and handoff leave no vector registers for the box and
@@ -255,11 +260,14 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : NBX_FLOWMAP_MIN_WAVES) vo
         const ReqDev& Rq = table == nullptr ? single : table[r];
         const int64_t p =
             tile_particle(slot - (table == nullptr ? 0 : slot_off[r]), Rq.nx, Rq.ny);
-        Dop853State<R> s;
+        Solve<Flow, R, G> sv;
+        auto& s = sv.s;
+        // a group's states: one, or one per component
+        auto* const held = state + slot * Solve<Flow, R, G>::kStates + (G > 1 ? lane & 1 : 0);
         bool active = false;
         if (p >= 0) {
             if (resume) {
-                s = coherent_load(state + slot);
+                s = coherent_load(held);
                 active = s.idid == 0;
             } else if (Rq.mask != nullptr && Rq.mask[p]) {
                 if (lead) {
@@ -270,14 +278,14 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : NBX_FLOWMAP_MIN_WAVES) vo
                 s.idid = 1;  // nothing left to do if the tile comes back
             } else {
                 const int64_t i = p / Rq.ny;
-                dop853_init(f, s, Rq.s0, Rq.s1, Rq.xs[i], Rq.ys[p - i * Rq.ny], rtol, atol);
+                sv.init(f, Rq.s0, Rq.s1, Rq.xs[i], Rq.ys[p - i * Rq.ny], rtol, atol);
                 active = true;
             }
         }
         for (int n = 0; active && n < kChunkSteps; ++n) {
-            if (!dop853_step(f, s, rtol, atol, nmax)) {
+            if (!sv.step(f, rtol, atol, nmax)) {
+                sv.store(Rq.out + p);
                 if (lead) {
-                    Rq.out[p] = make_double2(s.px(), s.py());
                     if (Rq.status) Rq.status[p] = s.idid;
                     if (Rq.nsteps) Rq.nsteps[p] = s.nstep;
                 }
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : NBX_FLOWMAP_MIN_WAVES) vo
             }
         }
         if (__ballot(active) != 0ull) {
-            if (lead && p >= 0) coherent_store(state + slot, s);
+            if ((lane & (G - 1)) < Solve<Flow, R, G>::kStates && p >= 0) coherent_store(held, s);
             // the states complete before the entry that hands them on
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             if (lane == 0) chunk_push(q, u | kResume);
@@ -303,7 +311,7 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : NBX_FLOWMAP_MIN_WAVES) vo
 // locality is worth more than the queue's refills (the autotuner times
 // both: persistent occupancy 0 selects this kernel).
 template <class Flow, class R, int G>
-__global__ __launch_bounds__(256, NBX_FLOWMAP_MIN_WAVES) void k_flowmap_tiles(
+__global__ __launch_bounds__(256, (flowmap_min_waves<Flow, R, G>())) void k_flowmap_tiles(
     Flow f, const ReqDev* __restrict__ table, const int64_t* __restrict__ slot_off, int nreq,
     int64_t total_slots, double rtol, double atol, long long nmax) {
     f.prepare();
@@ -329,12 +337,13 @@ __global__ __launch_bounds__(256, NBX_FLOWMAP_MIN_WAVES) void k_flowmap_tiles(
         return;
     }
     const int64_t i = p / Rq.ny;
-    Dop853State<R> s;
-    dop853_init(f, s, Rq.s0, Rq.s1, Rq.xs[i], Rq.ys[p - i * Rq.ny], rtol, atol);
-    while (dop853_step(f, s, rtol, atol, nmax)) {
+    Solve<Flow, R, G> sv;
+    auto& s = sv.s;
+    sv.init(f, Rq.s0, Rq.s1, Rq.xs[i], Rq.ys[p - i * Rq.ny], rtol, atol);
+    while (sv.step(f, rtol, atol, nmax)) {
     }
+    sv.store(Rq.out + p);
     if (lead) {
-        Rq.out[p] = make_double2(s.px(), s.py());
         if (Rq.status) Rq.status[p] = s.idid;
         if (Rq.nsteps) Rq.nsteps[p] = s.nstep;
     }
