@@ -72,95 +72,6 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes) {
     ptr_ = static_cast<char*>(e->ptr);
 }
 
-// ---------------------------------------------------------------------------
-// Spline prefilter: natural cubic B-spline, one thread per line.
-// Per axis n samples -> n+2 coefficients c[-1..n]: (c[i-1] + 4c[i] + c[i+1])/6
-// = f[i], zero second derivative at both ends, i.e. c[0] = f[0],
-// c[n-1] = f[n-1], interior by the Thomas algorithm, then
-// c[-1] = 2c[0]-c[1], c[n] = 2c[n-1]-c[n-2].
-
-__device__ void prefilter_line(double* p, long stride, int n) {
-    auto C = [&](int k) -> double& { return p[(static_cast<long>(k) + 1) * stride]; };
-    if (n == 1) {
-        C(-1) = C(0);
-        C(1) = C(0);
-        return;
-    }
-    if (n > 2) {
-        // forward sweep; the modified super-diagonal cp[k] = 1/(4 - cp[k-1])
-        // is recomputed on the way back instead of stored
-        const int m = n - 2;
-        double cp = 0.0, prev_d = 0.0;
-        for (int k = 0; k < m; ++k) {
-            const int i = k + 1;
-            double rhs = 6.0 * C(i);
-            if (i == 1) rhs -= C(0);
-            if (i == n - 2) rhs -= C(n - 1);
-            const double denom = 4.0 - (k > 0 ? cp : 0.0);
-            cp = 1.0 / denom;
-            const double d = (rhs - (k > 0 ? prev_d : 0.0)) / denom;
-            C(i) = d;
-            prev_d = d;
-        }
-        // back substitution needs cp[k] for k = m-2 .. 0.  The recurrence
-        // cp[k] = 1/(4 - cp[k-1]) reaches its double-precision fixed point
-        // (2 - sqrt(3)) by k = 13 and stays there, so 32 stored terms give
-        // every cp[k] exactly.
-        constexpr int kLocal = 32;
-        double cps[kLocal];
-        double c = 0.0;
-        for (int k = 0; k < kLocal; ++k) {
-            c = 1.0 / (4.0 - (k > 0 ? c : 0.0));
-            cps[k] = c;
-        }
-        for (int k = m - 2; k >= 0; --k)
-            C(k + 1) = C(k + 1) - cps[k < kLocal ? k : kLocal - 1] * C(k + 2);
-    }
-    C(-1) = 2 * C(0) - C(1);
-    C(n) = 2 * C(n - 1) - C(n - 2);
-}
-
-__global__ void k_prefilter_scatter(const double* __restrict__ U, int nt, int nx, int ny,
-                                    double* __restrict__ C) {
-    const long n2 = ny + 2, n1 = static_cast<long>(nx + 2) * n2;
-    const long total = static_cast<long>(nt + 2) * n1;
-    for (long k = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; k < total;
-         k += static_cast<long>(gridDim.x) * blockDim.x) {
-        const int a = static_cast<int>(k / n1);
-        const int b = static_cast<int>((k / n2) % (nx + 2));
-        const int c = static_cast<int>(k % n2);
-        double v = 0.0;
-        if (a >= 1 && a <= nt && b >= 1 && b <= nx && c >= 1 && c <= ny)
-            v = U[(static_cast<long>(a - 1) * nx + (b - 1)) * ny + (c - 1)];
-        C[k] = v;
-    }
-}
-
-// axis: 2 = y lines (a in 1..nt, b in 1..nx), 1 = x lines (a in 1..nt,
-// c in 0..ny+1), 0 = t lines (b in 0..nx+1, c in 0..ny+1)
-__global__ void k_prefilter_axis(double* __restrict__ C, int nt, int nx, int ny, int axis) {
-    const long n2 = ny + 2, n1 = static_cast<long>(nx + 2) * n2;
-    long lines, stride;
-    int n;
-    if (axis == 2) { lines = static_cast<long>(nt) * nx; stride = 1; n = ny; }
-    else if (axis == 1) { lines = static_cast<long>(nt) * (ny + 2); stride = n2; n = nx; }
-    else { lines = static_cast<long>(nx + 2) * (ny + 2); stride = n1; n = nt; }
-    const long L = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-    if (L >= lines) return;
-    double* p;
-    if (axis == 2) {
-        const long a = 1 + L / nx, b = 1 + L % nx;
-        p = C + a * n1 + b * n2;
-    } else if (axis == 1) {
-        const long a = 1 + L / (ny + 2), c = L % (ny + 2);
-        p = C + a * n1 + c;
-    } else {
-        const long b = L / (ny + 2), c = L % (ny + 2);
-        p = C + b * n2 + c;
-    }
-    prefilter_line(p, stride, n);
-}
-
 // (u, v) pairs in FP64, and FP32 elements pairing time index t with t + 1
 // (slab = one time slice of coefficients; the last slice repeats itself).
 __global__ void k_interleave(const double* __restrict__ u, const double* __restrict__ v, int64_t n,
@@ -899,26 +810,6 @@ void nbx_flow_destroy(nbx_flow* fl) {
     if (fl->coef) (void)hipFree(fl->coef);
     if (fl->coef32) (void)hipFree(fl->coef32);
     delete fl;
-}
-
-int nbx_prefilter3(const double* U, int nt, int nx, int ny, double* C, nbx_stream stream) {
-    NBX_REQUIRE(U != nullptr && C != nullptr, "NULL argument");
-    NBX_REQUIRE(nt >= 1 && nx >= 1 && ny >= 1, "empty grid");
-    hipStream_t s = as_stream(stream);
-    const long total = static_cast<long>(nt + 2) * (nx + 2) * (ny + 2);
-    const unsigned nb = blocks_for(total, 256) < 8192 ? blocks_for(total, 256) : 8192;
-    k_prefilter_scatter<<<nb, 256, 0, s>>>(U, nt, nx, ny, C);
-    NBX_LAUNCHED("prefilter_scatter");
-    const long lines2 = static_cast<long>(nt) * nx;
-    k_prefilter_axis<<<blocks_for(lines2, 128), 128, 0, s>>>(C, nt, nx, ny, 2);
-    NBX_LAUNCHED("prefilter_axis_y");
-    const long lines1 = static_cast<long>(nt) * (ny + 2);
-    k_prefilter_axis<<<blocks_for(lines1, 128), 128, 0, s>>>(C, nt, nx, ny, 1);
-    NBX_LAUNCHED("prefilter_axis_x");
-    const long lines0 = static_cast<long>(nx + 2) * (ny + 2);
-    k_prefilter_axis<<<blocks_for(lines0, 128), 128, 0, s>>>(C, nt, nx, ny, 0);
-    NBX_LAUNCHED("prefilter_axis_t");
-    return 0;
 }
 
 int nbx_flow_eval(const nbx_flow* fl, const double* params, int np, const double* t,
