@@ -14,6 +14,8 @@ struct nbx_flow {
     double2* coef = nullptr;  // spline: (nt+2, nx+2, ny+2) interleaved (u, v) coefficients;
                               // trilinear: (nt, nx, ny) interleaved samples; device
     float4* coef32 = nullptr; // FP32 copy, time-paired, for the FP32-displacement path
+    size_t coef_bytes = 0, coef32_bytes = 0;  // of the arrays, as allocated
+    int dev = -1;             // device of the arrays (-1: none)
     int64_t ncoef = 0;
     double grid9[9] = {0};
     int spherical = 0;

@@ -10,12 +10,14 @@
 #include <cmath>
 #include <cstring>
 #include <algorithm>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <tuple>
 #include <type_traits>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -71,6 +73,91 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes) {
     }
     ptr_ = static_cast<char*>(e->ptr);
 }
+
+// Device memory of flow handles.  A program that follows a data set replaces
+// its flow over and over (the next handle made, then the old one closed), and
+// hipFree and hipMalloc of the 2 x 44 MB of a 96-frame field cost 330 us of a
+// 550 us set-up.  So a closed flow's arrays wait here for the next one -- at
+// most kHeldBytes per device, and only while the device still has another
+// flow: the last handle to close gives everything back.  As hipFree does, a
+// close waits for the device's work first, so held memory is idle whatever
+// streams used it; an allocation that fails gives the held blocks back and is
+// tried again.
+namespace {
+constexpr size_t kHeldBytes = size_t(1) << 30;
+struct FlowBlocks {
+    std::vector<std::pair<void*, size_t>> held;
+    size_t bytes = 0;
+    int flows = 0;  // live gridded flows
+    void give_back() {
+        for (auto& b : held) (void)hipFree(b.first);
+        held.clear();
+        bytes = 0;
+    }
+};
+std::mutex g_blocks_mutex;
+std::map<int, FlowBlocks> g_blocks;  // per device
+
+// a held block of at least `bytes` and at most an eighth more, or a new one;
+// `bytes` becomes the block's size
+void* flow_alloc(int dev, size_t& bytes) {
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    FlowBlocks& fb = g_blocks[dev];
+    for (size_t i = 0; i < fb.held.size(); ++i) {
+        const auto b = fb.held[i];
+        if (b.second < bytes || b.second > bytes + bytes / 8) continue;
+        fb.held.erase(fb.held.begin() + i);
+        fb.bytes -= b.second;
+        bytes = b.second;
+        return b.first;
+    }
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    if (fb.held.empty()) return nullptr;
+    fb.give_back();
+    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+}
+
+// the arrays of a closing flow (sizes as allocated; null entries allowed)
+void flow_release(int dev, std::initializer_list<std::pair<void*, size_t>> blocks) {
+    int cur = dev;
+    (void)hipGetDevice(&cur);
+    if (cur != dev) (void)hipSetDevice(dev);
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        FlowBlocks& fb = g_blocks[dev];
+        --fb.flows;
+        for (const auto& b : blocks) {
+            if (b.first == nullptr) continue;
+            if (idle && fb.flows > 0 && fb.bytes + b.second <= kHeldBytes) {
+                fb.held.push_back(b);
+                fb.bytes += b.second;
+            } else {
+                (void)hipFree(b.first);
+            }
+        }
+        if (fb.flows <= 0) fb.give_back();
+    }
+    if (cur != dev) (void)hipSetDevice(cur);
+}
+
+// device and block sizes of a new gridded flow, counted among the live ones
+int flow_register(nbx_flow* fl) {
+    if (hipGetDevice(&fl->dev) != hipSuccess) return -1;
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    ++g_blocks[fl->dev].flows;
+    return 0;
+}
+template <class T>
+bool flow_array(const nbx_flow* fl, T** p, size_t* bytes) {
+    *bytes = sizeof(T) * static_cast<size_t>(fl->ncoef);
+    *p = static_cast<T*>(flow_alloc(fl->dev, *bytes));
+    return *p != nullptr;
+}
+}  // namespace
 
 // (u, v) pairs in FP64, and FP32 elements pairing time index t with t + 1
 // (slab = one time slice of coefficients; the last slice repeats itself).
@@ -730,8 +817,8 @@ int nbx_flow_create_spline3(const double* grid9_host, const double* Cu, const do
     fl->extrap = extrap;
     fl->r = r;
     fl->ncoef = ncoef;
-    if (hipMalloc(&fl->coef, sizeof(double2) * ncoef) != hipSuccess ||
-        hipMalloc(&fl->coef32, sizeof(float4) * ncoef) != hipSuccess) {
+    if (flow_register(fl) != 0 || !flow_array(fl, &fl->coef, &fl->coef_bytes) ||
+        !flow_array(fl, &fl->coef32, &fl->coef32_bytes)) {
         nbx_flow_destroy(fl);
         set_error("hipMalloc of spline coefficients failed");
         return -1;
@@ -771,7 +858,7 @@ int nbx_flow_create_linear3(const double* grid9_host, const double* U, const dou
     fl->extrap = extrap;
     fl->r = r;
     fl->ncoef = nval;
-    if (hipMalloc(&fl->coef, sizeof(double2) * nval) != hipSuccess) {
+    if (flow_register(fl) != 0 || !flow_array(fl, &fl->coef, &fl->coef_bytes)) {
         nbx_flow_destroy(fl);
         set_error("hipMalloc of velocity samples failed");
         return -1;
@@ -807,8 +894,8 @@ int nbx_ingest_xy(const double* U_xy, int nt, int ny, int nx, double scale, doub
 
 void nbx_flow_destroy(nbx_flow* fl) {
     if (!fl) return;
-    if (fl->coef) (void)hipFree(fl->coef);
-    if (fl->coef32) (void)hipFree(fl->coef32);
+    if (fl->dev >= 0)
+        flow_release(fl->dev, {{fl->coef, fl->coef_bytes}, {fl->coef32, fl->coef32_bytes}});
     delete fl;
 }
 

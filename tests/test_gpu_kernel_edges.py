@@ -29,3 +29,32 @@ def test_prefilter_line_groups(shape):
     C = _lib.to_host(prefilter3_device(U))
     assert C.shape == tuple(n + 2 for n in shape)
     assert relerr(C, oracle.prefilter3(U)) < 1e-13
+
+
+def test_flow_arrays_are_reused_safely():
+    """A flow made while others of its size come and go evaluates its own
+    coefficients: replaced handles, handles of near sizes, two alive at once,
+    and a fresh start after the last has closed."""
+    from numbacs_amd.flows import flow_velocity, get_flow_2D, get_flow_linear_2D
+
+    rng = np.random.default_rng(7)
+    pts, t = rng.uniform(0.1, 0.9, (50, 2)), rng.uniform(0.1, 0.9, 50)
+    p = np.array([1.0])
+
+    def make(k):
+        n = (9 + k % 2, 12, 11)  # near sizes share blocks
+        grid = tuple((0.0, 1.0, m) for m in n)
+        if k % 3 == 2:
+            return get_flow_linear_2D(grid, np.full(n, k + 1.0), np.full(n, -k - 1.0))
+        C = np.full(tuple(m + 2 for m in n), k + 1.0)  # constant coefficients: constant field
+        return get_flow_2D(grid, C, -C)
+
+    kept, current = make(100), None
+    for k in range(12):
+        current = make(k)  # the previous handle closes after this one is made
+        for f, v in ((current, k + 1.0), (kept, 101.0)):
+            got = flow_velocity(f, t, pts, p)
+            assert np.allclose(got[:, 0], v, rtol=1e-12) and np.allclose(got[:, 1], -v, rtol=1e-12)
+    kept.close()
+    current.close()
+    assert np.allclose(flow_velocity(make(3), t, pts, p)[:, 0], 4.0, rtol=1e-12)
