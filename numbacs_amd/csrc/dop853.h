@@ -387,7 +387,7 @@ __device__ __forceinline__ void dop853_init(const Flow& f, Dop853Lane<R>& s, dou
     s.nstep = 0;
     s.idid = 0;
     s.y = p0;
-    s.k1 = f.component(x, p0, [] {});
+    s.k1 = f.component(f.time_of(x), p0, [] {});
     const double f0 = static_cast<double>(s.k1);
     const double sk = atol + rtol * fabs(p0);
     const double dnf = pair_sumsq(f0 / sk);
@@ -395,7 +395,7 @@ __device__ __forceinline__ void dop853_init(const Flow& f, Dop853Lane<R>& s, dou
     double h = (dnf <= 1.0e-10 || dny <= 1.0e-10) ? 1.0e-6 : sqrt(dny / dnf) * 0.01;
     h = fmin(h, s.hmax);
     h = s.posneg >= 0 ? fabs(h) : -fabs(h);
-    const double df = f.component_change(x + h, p0 + h * f0, f0);
+    const double df = f.component_change(f.time_of(x + h), p0 + h * f0, f0);
     const double der2 = sqrt(pair_sumsq(df / sk)) / h;
     const double der12 = fmax(fabs(der2), sqrt(dnf));
     const double h1 =
@@ -427,6 +427,11 @@ struct StageLds {
     __device__ __forceinline__ double get(int i) const { return at[64 * i]; }
 };
 
+__device__ __forceinline__ double unfused_add(double a, double b) {
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 // A stage's evaluation and, in the time its gathers are in flight, the part
 // of the next stage's sum that does not need it (`ahead`).
 template <class R, class Stages, class Flow>
@@ -435,49 +440,57 @@ __device__ __forceinline__ bool dop853_step_body(const Flow& f, Dop853Lane<R>& s
     using namespace dop;
     ++s.nstep;
     const double x = s.x, h = s.h, y = s.y;
-    auto F = [&](double t, double q, auto&& ahead) {
+    auto F = [&](typename Flow::Time t, double q, auto&& ahead) {
         return static_cast<double>(f.component(t, q, ahead));
     };
     auto none = [] {};
     double P;  // the next stage's sum but for its last term
     const double K1 = static_cast<double>(s.k1);
     ks.put(0, K1);
-    double K = F(x + c2 * h, fma(h * a21, K1, y), none);
-    K = F(x + c3 * h, fma(h, fma(a31, K1, a32 * K), y), none);
-    K = F(x + c4 * h, fma(h, fma(a41, K1, a43 * K), y), [&, K3 = K] { P = fma(a51, K1, a53 * K3); });
+    typename Flow::Time ta, tb;  // of a pair of stages (a pair of lanes forms one each)
+    // (c2 = a21: gridded flows' kernels form h a21 once and add it to x)
+    const double ha = h * a21;
+    f.times_of(Flow::kFusedC2 ? fma(c2, h, x) : unfused_add(x, ha), fma(c3, h, x), ta, tb);
+    double K = F(ta, fma(ha, K1, y), none);
+    K = F(tb, fma(h, fma(a31, K1, a32 * K), y), none);
+    f.times_of(fma(c4, h, x), fma(c5, h, x), ta, tb);
+    K = F(ta, fma(h, fma(a41, K1, a43 * K), y), [&, K3 = K] { P = fma(a51, K1, a53 * K3); });
     ks.put(1, K);
-    K = F(x + c5 * h, fma(h, fma(a54, K, P), y),
+    K = F(tb, fma(h, fma(a54, K, P), y),
           [&] { P = fma(a61, ks.get(0), a64 * ks.get(1)); });
     ks.put(2, K);
-    K = F(x + c6 * h, fma(h, fma(a65, K, P), y),
+    f.times_of(fma(c6, h, x), fma(c7, h, x), ta, tb);
+    K = F(ta, fma(h, fma(a65, K, P), y),
           [&] { P = fma(a75, ks.get(2), fma(a71, ks.get(0), a74 * ks.get(1))); });
     ks.put(3, K);
-    K = F(x + c7 * h, fma(h, fma(a76, K, P), y), [&] {
+    K = F(tb, fma(h, fma(a76, K, P), y), [&] {
         P = fma(a86, ks.get(3),
                 fma(a85, ks.get(2), fma(a81, ks.get(0), a84 * ks.get(1))));
     });
     ks.put(4, K);
-    K = F(x + c8 * h, fma(h, fma(a87, K, P), y), [&] {
+    f.times_of(fma(c8, h, x), fma(c9, h, x), ta, tb);
+    K = F(ta, fma(h, fma(a87, K, P), y), [&] {
         P = fma(a97, ks.get(4),
                 fma(a96, ks.get(3),
                     fma(a95, ks.get(2), fma(a91, ks.get(0), a94 * ks.get(1)))));
     });
     ks.put(5, K);
-    K = F(x + c9 * h, fma(h, fma(a98, K, P), y), [&] {
+    K = F(tb, fma(h, fma(a98, K, P), y), [&] {
         P = fma(a108, ks.get(5),
                 fma(a107, ks.get(4),
                     fma(a106, ks.get(3),
                         fma(a105, ks.get(2), fma(a101, ks.get(0), a104 * ks.get(1))))));
     });
     ks.put(6, K);
-    K = F(x + c10 * h, fma(h, fma(a109, K, P), y), [&] {
+    f.times_of(fma(c10, h, x), fma(c11, h, x), ta, tb);
+    K = F(ta, fma(h, fma(a109, K, P), y), [&] {
         P = fma(a119, ks.get(6),
                 fma(a118, ks.get(5),
                     fma(a117, ks.get(4),
                         fma(a116, ks.get(3), fma(a115, ks.get(2), fma(a114, ks.get(1), a111 * ks.get(0)))))));
     });
     ks.put(7, K);
-    K = F(x + c11 * h, fma(h, fma(a1110, K, P), y), [&] {
+    K = F(tb, fma(h, fma(a1110, K, P), y), [&] {
         P = fma(a1210, ks.get(7),
                 fma(a129, ks.get(6),
                     fma(a128, ks.get(5),
@@ -488,8 +501,9 @@ __device__ __forceinline__ bool dop853_step_body(const Flow& f, Dop853Lane<R>& s
     });
     ks.put(8, K);
     const double xph = x + h;
+    const typename Flow::Time tn = f.time_of(xph);
     double B, E;  // the update's and the fifth-order error's sums but for the last term
-    K = F(xph, fma(h, fma(a1211, K, P), y), [&] {
+    K = F(tn, fma(h, fma(a1211, K, P), y), [&] {
         const double k1 = ks.get(0), k6 = ks.get(3), k7 = ks.get(4), k8 = ks.get(5),
                      k9 = ks.get(6), k10 = ks.get(7), k11 = ks.get(8);
         B = fma(b11, k11,
@@ -515,7 +529,7 @@ __device__ __forceinline__ bool dop853_step_body(const Flow& f, Dop853Lane<R>& s
     double hnew = h / (accept ? fmax(facc2, fmin(facc1, fac)) : fmin(facc1, fac));
     if (accept) {
         s.y = pn;
-        s.k1 = f.component(xph, pn, none);
+        s.k1 = f.component(tn, pn, none);
         s.x = xph;
         if (s.last) {
             s.idid = 1;

@@ -90,6 +90,14 @@ Linear3<R> make_linear(const nbx_flow* fl, double p0) {
     return s;
 }
 
+template <class R>
+Linear3Pair<R> pair_linear(const Linear3<R>& f) {
+    Linear3Pair<R> p;
+    p.f = f;
+    for (int d = 0; d < 3; ++d) p.rstep[d] = 1.0 / f.step[d];
+    return p;
+}
+
 template <int G, class R, bool S = false>
 Spline3<R, G, false, S> regroup(const Spline3<R, 1, false>& a) {
     Spline3<R, G, false, S> s;

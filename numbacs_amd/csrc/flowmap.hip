@@ -488,13 +488,18 @@ __global__ void k_flow_eval(Flow f, const double* __restrict__ t, const double2*
     out[k] = make_double2(static_cast<double>(a), static_cast<double>(b));
 }
 
-// defaults: the best shapes measured on the gridded-velocity and
-// double-gyre workloads (spline flows: 4 lanes per particle, 128-thread
-// blocks); the autotuner overrides them per workload
-LaunchCfg g_cfg[4][2] = {{{1, 256, 0}, {1, 256, 0}},
-                         {{1, 256, 0}, {1, 256, 0}},
+// defaults: the best shapes measured on the gridded-velocity, double-gyre
+// and Bickley workloads; the autotuner overrides them per workload.  One-wave
+// blocks let each wavefront's slot go to the next as it ends (double gyre,
+// 3,321 particles: 320 us with 256 threads, 187 with 64; 2 M: 2.87, 2.80 ms).
+// The Bickley jet's long trajectories leave a third of the grid launch idle
+// behind its last wavefronts, so it runs the tile queue at its kernels'
+// occupancy (2 and 3 wavefronts per SIMD): 401,401 particles 17.1 -> 14.0 ms,
+// float 10.0 -> 8.0; 1.6 M 49.6 -> 46.4 ms.
+LaunchCfg g_cfg[4][2] = {{{1, 64, 0}, {1, 64, 0}},
+                         {{1, 64, 8}, {1, 64, 12}},
                          {{4, 128, 0}, {4, 128, 0}},
-                         {{1, 128, 0}, {1, 128, 0}}};
+                         {{1, 64, 0}, {1, 64, 0}}};
 // edge-first tile order of the spline grid launch, per precision
 int g_edge_first[2] = {1, 1};
 std::mutex g_cfg_mutex;
@@ -536,6 +541,18 @@ inline ReqDev single_request(const GridSource& src, const SolveArgs& a) {
                   a.out, a.status, a.nsteps};
 }
 
+// One launch with a group of G lanes for every particle.
+template <class Flow, class R, int G, class Src>
+int launch_grid(const Flow& f, const Src& src, const SolveArgs& a, int block, hipStream_t s) {
+    int64_t slots = a.P;
+    if constexpr (std::is_same<Src, GridSource>::value) slots = src.slots();
+    k_flowmap<Flow, R, G, Src><<<blocks_for(slots * G, block), block,
+                                 solve_lds_bytes<Flow, R, G>(block), s>>>(
+        f, src, slots, a.s0, a.s1, a.rtol, a.atol, a.mask, a.nmax, a.out, a.status, a.nsteps);
+    NBX_LAUNCHED("flowmap");
+    return 0;
+}
+
 template <class Flow, class R, int G, class Src>
 int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const LaunchCfg& cfg,
                  hipStream_t s) {
@@ -548,6 +565,16 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             if (slots == 0) return 0;
             const int64_t ntiles = slots / (64 / G);
             NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
+            const int64_t want = (ntiles * 64 + block - 1) / block;
+            const int64_t most = static_cast<int64_t>(cus) * cfg.persistent;
+            // With a wavefront for every tile there is nothing to hand on; from
+            // 16 rounds of them the tail is a few percent and not worth the
+            // states' memory.  A stream under capture takes the grid launch too
+            // (the queue's workspace may have to be allocated).
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            (void)hipStreamIsCapturing(s, &capture);
+            if (want <= most || want > 16 * most || capture != hipStreamCaptureStatusNone)
+                return launch_grid<Flow, R, G>(f, src, a, block, s);
             const unsigned long long ring = chunk_ring(ntiles);
             const size_t state_off = ring * sizeof(unsigned long long) + 256;
             Workspace ws(s, 3, state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots));
@@ -560,23 +587,16 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
                                ring - 1, static_cast<unsigned long long>(ntiles)};
             k_chunk_init<<<blocks_for(static_cast<int64_t>(ring), 256), 256, 0, s>>>(q, ntiles);
             NBX_LAUNCHED("chunk_init");
-            const int64_t want = (ntiles * 64 + block - 1) / block;
-            const int64_t grid = std::min<int64_t>(want, static_cast<int64_t>(cus) * cfg.persistent);
-            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(grid), block,
-                                         solve_lds_bytes<Flow, R, G>(block), s>>>(
+            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(most), block,
+                                           solve_lds_bytes<Flow, R, G>(block), s>>>(
                 f, single_request(src, a), nullptr, nullptr, 1, q,
-                reinterpret_cast<decltype(Solve<Flow, R, G>::s)*>(w + state_off), a.rtol, a.atol, a.nmax);
+                reinterpret_cast<decltype(Solve<Flow, R, G>::s)*>(w + state_off), a.rtol, a.atol,
+                a.nmax);
             NBX_LAUNCHED("flowmap_chunks");
             return 0;
         }
     }
-    int64_t slots = a.P;
-    if constexpr (std::is_same<Src, GridSource>::value) slots = src.slots();
-    k_flowmap<Flow, R, G, Src><<<blocks_for(slots * G, block), block,
-                                 solve_lds_bytes<Flow, R, G>(block), s>>>(
-        f, src, slots, a.s0, a.s1, a.rtol, a.atol, a.mask, a.nmax, a.out, a.status, a.nsteps);
-    NBX_LAUNCHED("flowmap");
-    return 0;
+    return launch_grid<Flow, R, G>(f, src, a, block, s);
 }
 
 // Edge-first launch order of a grid's 4 x 4 particle tiles.  A particle
@@ -751,11 +771,19 @@ int dispatch_solve(const nbx_flow* fl, const double* params, int np, const Src& 
             return launch_solve<Spline3<R, 2>, R, 2>(regroup<2>(sp), run_src, a, cfg, s);
         return launch_solve<Spline3<R, 1>, R, 1>(sp, run_src, a, cfg, s);
     }
+    // (the auxiliary grid's one-lane kernels of these flows contract a few
+    // operations differently from the grid's: they stay, for the same results)
+    const bool pair = !std::is_same<Src, AuxSource>::value && pair_lanes<R>(fl, a.P);
     if (fl->kind == NBX_FLOW_LINEAR3)
-        return launch_solve<Linear3<R>, R, 1>(make_linear<R>(fl, params[0]), src, a, cfg, s);
+        return pair ? launch_solve<Linear3Pair<R>, R, 2>(
+                          pair_linear(make_linear<R>(fl, params[0])), src, a, cfg, s)
+                    : launch_solve<Linear3<R>, R, 1>(make_linear<R>(fl, params[0]), src, a, cfg,
+                                                     s);
     if (fl->kind == NBX_FLOW_DOUBLE_GYRE) {
         NBX_REQUIRE(np >= 6, "double_gyre needs 6 parameters [dir, A, eps, alpha, omega, psi]");
         const DoubleGyre<R> dg{params[0], params[1], params[2], params[3], params[4], params[5]};
+        if (pair)
+            return launch_solve<DoubleGyrePair<R>, R, 2>(DoubleGyrePair<R>{dg}, src, a, cfg, s);
         return launch_solve<DoubleGyre<R>, R, 1>(dg, src, a, cfg, s);
     }
     if (fl->kind == NBX_FLOW_BICKLEY_JET) {

@@ -62,6 +62,60 @@ struct DoubleGyre {
     }
 };
 
+// The double gyre on a pair of lanes (x in the even one, y in the odd one):
+// the even lane takes sin and cos of pi f, the odd lane of pi y, and each lane
+// the time factor eps sin(omega t + psi) of every other stage, so a lane runs
+// one and a half library calls an evaluation instead of three.  By the
+// operations of DoubleGyre.
+template <class R>
+struct DoubleGyrePair {
+    static constexpr bool kStagesInLds = false;
+    static constexpr bool kFusedC2 = true;
+    DoubleGyre<R> g;
+    __device__ __forceinline__ void prepare() {}
+    __device__ __forceinline__ void prepare_factors() {}
+
+    using Time = R;
+    __device__ __forceinline__ R time_of(double t) const {
+        const double tt = g.p0 * t;
+        return static_cast<R>(g.eps * sin(g.omega * tt + g.psi));
+    }
+    __device__ __forceinline__ void times_of(double ta, double tb, R& a, R& b) const {
+        const R v = time_of((__lane_id() & 1) ? tb : ta);
+        a = quad_move<kPairEven>(v);
+        b = quad_move<kPairOdd>(v);
+    }
+
+    // the lane's component but for the direction's factor
+    template <class Ahead>
+    __device__ __forceinline__ R undirected(R a, double yc, Ahead&& ahead) const {
+        const bool odd = __lane_id() & 1;
+        const R y = static_cast<R>(yc), y0 = quad_move<kPairEven>(y);
+        // (the contractions of DoubleGyre's expressions, written out)
+        const R b = fma(a, R(-2), R(1));
+        const R f = fma(a, y0 * y0, b * y0);
+        const R df = fma(2 * a, y0, b);
+        const R pi = static_cast<R>(kPi), A = static_cast<R>(g.A), alpha = static_cast<R>(g.alpha);
+        ahead();
+        R sn, cs;
+        if constexpr (sizeof(R) == sizeof(double)) sincos(pi * (odd ? y : f), &sn, &cs);
+        else sincosf(pi * (odd ? y : f), &sn, &cs);
+        const R other = quad_move<kPairSwap>(cs);  // cos(pi y) in the even lane, cos(pi f) in the odd
+        const R w = (odd ? pi * A * other : -pi * A) * sn;
+        return fma(w, odd ? df : other, -(alpha * y));
+    }
+    template <class Ahead>
+    __device__ __forceinline__ R component(R a, double yc, Ahead&& ahead) const {
+        return static_cast<R>(g.p0) * undirected(a, yc, ahead);
+    }
+    // component - f0 as the solver's initial step contracts it
+    __device__ __forceinline__ double component_change(R a, double yc, double f0) const {
+        if constexpr (sizeof(R) == sizeof(double))
+            return fma(g.p0, undirected(a, yc, [] {}), -f0);
+        return static_cast<double>(component(a, yc, [] {})) - f0;
+    }
+};
+
 // Bickley jet with three travelling modes, flows.py:1182-1213.
 // p = [dir, U0, L, A1, A2, A3, k1, k2, k3, c1, c2, c3].
 template <class R>
@@ -379,6 +433,7 @@ struct Spline3 {
     // the FP64 form has no vector registers left for the solver's stages (at
     // three wavefronts per SIMD)
     static constexpr bool kStagesInLds = kReuse && sizeof(R) == sizeof(double);
+    static constexpr bool kFusedC2 = false;
     static constexpr int kRows = sizeof(R) == sizeof(double) ? 16 : 8;
     mutable P cst[kReuse ? kRows : 1];
     mutable double ckey = -1;
@@ -761,6 +816,14 @@ struct Spline3 {
         else return (static_cast<float>(kdeg) * r.s) / r.den;
     }
 
+    // (a stage's time enters as it is)
+    using Time = double;
+    __device__ __forceinline__ double time_of(double t) const { return t; }
+    __device__ __forceinline__ void times_of(double ta, double tb, double& a, double& b) const {
+        a = ta;
+        b = tb;
+    }
+
     // the lane's component of the right-hand side
     template <class Ahead>
     __device__ __forceinline__ R component(double t, double yc, Ahead&& ahead) const {
@@ -881,6 +944,83 @@ struct Linear3 {
             f0 = static_cast<R>(((p0 * su) * 180) / (kPi * r * cos_lat(deg_to_rad(y1))));
             f1 = static_cast<R>(((p0 * sv) * 180) / (kPi * r));
         }
+    }
+};
+
+// The trilinear flow on a pair of lanes (x in the even one, y in the odd one):
+// the even lane gathers and sums time slice it, the odd lane slice it + 1 (four
+// samples each instead of eight), and each finishes its own component.  By the
+// operations of Linear3, its three quotients by the grid steps taken with
+// their reciprocals (div_with: an IEEE division's result).
+template <class R>
+struct Linear3Pair {
+    static constexpr bool kStagesInLds = false;
+    static constexpr bool kFusedC2 = false;
+    Linear3<R> f;
+    double rstep[3];  // 1 / step, correctly rounded
+    // the lane's four samples of the cell it read last and that cell: a step
+    // cut at a cell face makes most of its evaluations inside one cell
+    mutable double2 held[4];
+    mutable double hkey = -1;
+    __device__ __forceinline__ void prepare() {}
+    __device__ __forceinline__ void prepare_factors() {}
+
+    using Time = double;
+    __device__ __forceinline__ double time_of(double t) const { return t; }
+    __device__ __forceinline__ void times_of(double ta, double tb, double& a, double& b) const {
+        a = ta;
+        b = tb;
+    }
+
+    template <class Ahead>
+    __device__ __forceinline__ R component(double t, double yc, Ahead&& ahead) const {
+#pragma clang fp contract(off)
+        const bool odd = __lane_id() & 1;
+        const double y1 = quad_move<kPairOdd>(yc);
+        double xx = quad_move<kPairEven>(yc);
+        if (f.spherical == 1) xx = wrap360(xx - 180) - 180;
+        else if (f.spherical != 0) xx = wrap360(xx);
+        const double q[3] = {f.p0 * t, xx, y1};
+        bool out = false;
+        double k[3], w[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            out |= (q[d] < f.lo[d]) | (q[d] > f.hi[d]);
+            const double qq = f.extrap == 2 ? clamped(q[d], f.lo[d], f.hi[d]) : q[d];
+            const double u = div_with(qq - f.lo[d], f.step[d], rstep[d]);
+            k[d] = clamped(floor(u), 0.0, f.n[d] - 2);
+            w[d] = u - k[d];
+        }
+        // (out-of-box points read the boundary cell and are dropped)
+        const double key = fma(k[0], static_cast<double>(f.st),
+                               fma(k[1], static_cast<double>(f.sx), k[2]));
+        if (key != hkey) {
+            hkey = key;
+            const double2* c = f.V + (static_cast<unsigned>(key) + (odd ? f.st : 0));
+            held[0] = c[0];
+            held[1] = c[1];
+            held[2] = c[f.sx];
+            held[3] = c[f.sx + 1];
+        }
+        ahead();
+        double den = 1.0, recip = 1.0;
+        if (f.spherical != 0) {
+            const double pr = kPi * f.r, cl = cos_lat(deg_to_rad(y1));
+            den = odd ? pr : pr * cl;
+            recip = div_recip(den);
+        }
+        const double2 a00 = held[0], a01 = held[1], a10 = held[2], a11 = held[3];
+        const double w1 = w[1], w2 = w[2], w0 = w[0];
+        const double bu = (1 - w1) * ((1 - w2) * a00.x + w2 * a01.x) + w1 * ((1 - w2) * a10.x + w2 * a11.x);
+        const double bv = (1 - w1) * ((1 - w2) * a00.y + w2 * a01.y) + w1 * ((1 - w2) * a10.y + w2 * a11.y);
+        const double got = quad_move<kPairSwap>(odd ? bu : bv);
+        double s = (1 - w0) * (odd ? got : bu) + w0 * (odd ? bv : got);
+        if (out && f.extrap == 0) s = 0.0;
+        if (f.spherical == 0) return static_cast<R>(f.p0 * s);
+        return static_cast<R>(div_with((f.p0 * s) * 180, den, recip));
+    }
+    __device__ __forceinline__ double component_change(double t, double yc, double f0) const {
+        return static_cast<double>(component(t, yc, [] {})) - f0;
     }
 };
 

@@ -37,9 +37,13 @@
 #include <cstdint>
 
 #include "dop853.h"
+#include "flow_handle.h"
 #include "flows.h"
 
 namespace nbx {
+
+// Number of compute units of the current device (cached per device).
+int device_cu_count();
 
 // Particle order of the one-solve-per-group grid launch: 8 x 8 tiles of the
 // particle grid, each walked as its four 4 x 4 quadrants, so any run of 16,
@@ -83,6 +87,24 @@ template <class T>
 struct IsSpline3 : std::false_type {};
 template <class R, int G, bool L, bool S>
 struct IsSpline3<Spline3<R, G, L, S>> : std::true_type {};
+
+// Whether a double-gyre or trilinear flow map of P particles runs two lanes per
+// particle (one component each) rather than one.  What bounds these maps when
+// the machine is not full is one particle's serial chain -- a lone wavefront
+// issues an FP64 operation every 8 cycles -- and a pair halves the chain's
+// work.  Trilinear maps are bound by their longest trajectories (518 steps
+// against 112 on average) at every size: 1,768 particles 4.8 -> 3.1 ms,
+// 169,676 7.3 -> 6.5, 676,851 14.1 -> 12.6; their pair indexes samples with
+// 32 bits.  The double gyre's pair spends a fifth more instructions, so it
+// stays below two (float: four) wavefronts per SIMD of the one-lane form:
+// FP64 3,321 particles 187 -> 120 us, 80,601 289 -> 240, 180,901 376 -> 394;
+// float 80,601 220 -> 179, 180,901 289 -> 286, 721,801 857 -> 880.
+template <class R>
+inline bool pair_lanes(const nbx_flow* fl, int64_t P) {
+    if (fl->kind == NBX_FLOW_LINEAR3) return fl->ncoef < (int64_t(1) << 31);
+    return fl->kind == NBX_FLOW_DOUBLE_GYRE &&
+           P <= static_cast<int64_t>(device_cu_count()) * (sizeof(R) == 4 ? 1024 : 512);
+}
 
 // Minimum wavefronts per SIMD asked of the compiler for a flow-map kernel
 // (it caps the vector registers at 512 / n).  The 4-lane spline forms hold
@@ -217,9 +239,6 @@ __device__ __forceinline__ void chunk_push(const ChunkQueue& q, unsigned payload
     __hip_atomic_store(q.items + (r & q.mask), ((r & 0xffffffffull) << 32) | payload,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Number of compute units of the current device (cached per device).
-int device_cu_count();
 
 // The queue's tiles are the grid launch's wavefronts: 64 / G consecutive
 // slots in tile order (a 4 x 4 particle tile at G = 4).  Slots are numbered

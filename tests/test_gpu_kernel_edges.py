@@ -58,3 +58,68 @@ def test_flow_arrays_are_reused_safely():
     kept.close()
     current.close()
     assert np.allclose(flow_velocity(make(3), t, pts, p)[:, 0], 4.0, rtol=1e-12)
+
+
+@pytest.mark.parametrize("kind", ["double_gyre", "trilinear"])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 11), (33, 4), (8, 65)])
+def test_pair_lanes_equal_one_lane(kind, precision, shape):
+    """The two-lane solver runs the one-lane solver's operations: flow maps,
+    status and step counts equal bit for bit (the batch of a size above the
+    double gyre's pair limit, and a map's point list, as counterparts)."""
+    from numbacs_amd import _lib
+    from numbacs_amd.flows import get_flow_linear_2D, get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    rng = np.random.default_rng(3)
+    if kind == "double_gyre":
+        flow, p, _ = get_predefined_flow(kind, int_direction=-1.0)
+        p[3], box, t0, T = 0.02, ((0.0, 2.0), (0.0, 1.0)), 1.0, -7.0
+    else:
+        n = (9, 21, 17)
+        U, V = rng.standard_normal((2,) + n)
+        flow = get_flow_linear_2D(tuple((0.0, 1.0, m) for m in n), U, V)
+        p, box, t0, T = np.array([1.0]), ((-0.05, 1.05), (-0.05, 1.05)), 0.1, 0.8
+    nx, ny = shape
+    x, y = np.linspace(*box[0], nx), np.linspace(*box[1], ny)
+
+    def run(xs, ys):
+        st, ns = (_lib.empty((len(xs), len(ys)), "i32") for _ in range(2))
+        fm = flowmap_grid_2d_device(flow, t0, T, _lib.to_dev(xs), _lib.to_dev(ys), p,
+                                    precision=precision, status=st, nsteps=ns)
+        return [_lib.to_host(a) for a in (fm, st, ns)]
+
+    got = run(x, y)
+    assert (got[1] == 1).all()
+    # the same rows inside a map of 300,000 particles: one lane per particle
+    # for the double gyre
+    xs = np.concatenate([x, np.linspace(*box[0], 300000 // ny)])
+    for a, b in zip(got, run(xs, y)):
+        assert np.array_equal(a, b[:nx])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_bickley_queue_equals_grid_launch(precision):
+    """The default tile queue (more tiles than wavefronts) against the grid
+    launch, and a map small enough to take the grid launch by itself."""
+    from numbacs_amd import _lib, autotune
+    from numbacs_amd.flows import get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    flow, p, dom = get_predefined_flow("bickley_jet")
+    saved = autotune.get(1, precision)
+    assert saved[2] > 0
+
+    def run(nx, ny):
+        return _lib.to_host(flowmap_grid_2d_device(
+            flow, 0.0, 9.0, _lib.to_dev(np.linspace(*dom[0], nx)),
+            _lib.to_dev(np.linspace(*dom[1], ny)), p, precision=precision))
+
+    try:
+        got = [run(*n) for n in ((711, 333), (9, 33))]
+        autotune.set_config(1, precision, (1, 64, 0))
+        want = [run(*n) for n in ((711, 333), (9, 33))]
+    finally:
+        autotune.set_config(1, precision, saved)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
