@@ -321,17 +321,42 @@ __global__ void k_to_bf16(const float* __restrict__ x, int64_t n, uint16_t* __re
 // ---------------------------------------------------------------------------
 // Fused inference: Fourier features, the four hidden layers and the head in
 // one launch.  A 256-thread block takes 64 particles; their activations stay
-// in LDS (two 64 x 256 bf16 buffers, rows padded to 264 elements), each
-// wavefront computes a 64 x 64 quarter of a layer's output as 4 x 4 MFMA
-// 16x16x32 tiles, reading its weight fragments straight from global memory
-// (weights stored transposed, k contiguous, so a lane's 8 k-values are one
-// 16-byte load; the next k-step's fragments are loaded before the current
-// step's MFMAs).  Every step is the unfused path's arithmetic in its order:
-// the features of k_features, per layer the same k-steps of 32 accumulated
-// in order then bias + GELU + bf16 (k_gemm's epilogue), the head's
+// in LDS (64 x 256 bf16, each layer writing over its inputs once every
+// wavefront has read them), each wavefront computes a 64 x 64 quarter of a
+// layer's output as 4 x 4 MFMA 16x16x32 tiles.  Four blocks share a CU: 40 KiB
+// of LDS and 128 registers each.  Weights are stored transposed (k contiguous);
+// a wavefront reads 16 rows' 64 bytes with neighbouring lanes on one row and
+// turns them into fragments through its own 2 KiB of LDS, the next k-step's
+// loads in flight meanwhile (read as fragments straight from global memory,
+// neighbouring lanes on different rows, the same bytes cost four times the L1
+// accesses and bound the kernel: 2.97 ms).  The products run with the weights
+// as the first operand, so a lane receives four consecutive columns of one
+// particle: one 8-byte store each.  Every step is the unfused path's arithmetic
+// in its order: the features of k_features, per layer the same k-steps of 32
+// accumulated in order then bias + GELU + bf16 (k_gemm's epilogue), the head's
 // sequential fp32 sums of k_out_fwd and the output scaling -- so the result
 // equals the unfused forward pass bit for bit.
-constexpr int kInferRows = 64, kInferWidth = 256, kInferHalf = 64, kActLd = kInferWidth + 8;
+//
+// What bounds it is the VALU (some 70% of the issue slots, MFMA another 25%):
+// 1,024 GELUs and 128 sines a particle.  Both are kept to 8 bits only, so they
+// are first formed from the hardware's exp2, reciprocal, sine and cosine with a
+// bound on how far these can lie from the library's float value; only where a
+// rounding boundary to bf16 lies within that bound does the library function
+// itself decide (gelu_near: about one activation in a thousand near zero, all
+// below -4; sincos_near).  Those are listed per wavefront and evaluated 64 at a
+// time.  2701 x 1001 particles: 5.38 -> 2.15 ms (231 -> 577 TFLOP/s of products;
+// two 67 KB blocks a CU and the library's tanh, sin and cos throughout before).
+constexpr int kInferRows = 64, kInferWidth = 256, kInferHalf = 64;
+// bytes of a wavefront's own LDS: two weight fragments in the k-loop, else a
+// list of undecided activations, at the end the head's weights
+constexpr int kWaveBytes = 2048, kUndecided = kWaveBytes / 8;
+
+// element of act that holds column c of a row: the 16-byte chunks of a row are
+// permuted by the row's low bits, so 16 rows' chunks of one column lie in
+// different banks without padding
+__device__ __forceinline__ int act_at(int row, int c) {
+    return row * kInferWidth + (((c >> 3) ^ (row & 15)) << 3) + (c & 7);
+}
 
 struct MlpNetDev {
     const float* shift;
@@ -344,94 +369,233 @@ struct MlpNetDev {
     const float* out_scale;
 };
 
-__global__ __launch_bounds__(256) void k_mlp_infer(MlpNetDev net, const float* __restrict__ inp,
-                                                   int64_t n, float* __restrict__ out) {
-    __shared__ __attribute__((aligned(16))) uint16_t act[2][kInferRows][kActLd];
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// two floats to bf16 (round to nearest even), as f2bf rounds each
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    const bf16x2 v = __builtin_convertvector((f32x2{a, b}), bf16x2);
+    uint32_t r;
+    __builtin_memcpy(&r, &v, 4);
+    return r;
+}
+
+// gelu(a) = a / (1 + exp(-2 inner)) by the hardware's exp2 and reciprocal.
+// It differs from gelu(a) by less than (d + 6) units in its last float place,
+// d = 1 + exp(-2 inner) (the library form's own rounding grows with d: 1 + tanh
+// cancels), so undecided is set where a bf16 rounding boundary (low half
+// 0x8000) is that near.  Checked for every float: where undecided is not set,
+// both round to the same bf16.
+__device__ __forceinline__ float gelu_near(float a, bool& undecided) {
+    constexpr float c0 = -2.0f * 1.4426950408889634f * kGeluC, c1 = c0 * kGeluA;
+    const float d = 1.0f + __builtin_amdgcn_exp2f(a * fmaf(c1, a * a, c0));
+    const float g = a * __builtin_amdgcn_rcpf(d);
+    // the low half as a signed number lies at +-0x8000 on a boundary
+    const float low = static_cast<float>(static_cast<int16_t>(__float_as_uint(g)));
+    undecided = fabsf(low) + d >= 32768.0f - 6.0f;
+    return g;
+}
+
+// sine (x) and cosine (y) of 2 pi s to bf16 by the hardware's functions of a
+// revolution: both lie within delta of sinf / cosf of the rounded product, which
+// k_features takes (7e-7 |s| is that product's rounding, 5e-7 the hardware's
+// own error; largest seen over every float: 0.78 delta), so undecided is set
+// where the two ends of that interval round differently.
+__device__ __forceinline__ uint2 sincos_near(float s, bool& und_s, bool& und_c) {
+    const float f = __builtin_amdgcn_fractf(s), delta = fmaf(fabsf(s), 7e-7f, 5e-7f);
+    const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f);
+    const uint2 b = make_uint2(pack_bf16(sn - delta, sn + delta), pack_bf16(cs - delta, cs + delta));
+    const bool wide = !(fabsf(s) < 1e4f);
+    und_s = (b.x >> 16) != (b.x & 0xffffu) || wide;
+    und_c = (b.y >> 16) != (b.y & 0xffffu) || wide;
+    return b;
+}
+
+// position of the lane among those set in m
+__device__ __forceinline__ int rank_in(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
+}
+
+__global__ __launch_bounds__(256, 4) void k_mlp_infer(MlpNetDev net, const float* __restrict__ inp,
+                                                      int64_t n, float* __restrict__ out) {
+    __shared__ __attribute__((aligned(16))) uint16_t act[kInferRows * kInferWidth];
+    __shared__ __attribute__((aligned(16))) uint8_t own[4][kWaveBytes];
     const int t = threadIdx.x;
-    const int lane = t & 63, w = t >> 6;
+    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kInferRows;
-    // ---- Fourier features (k_features): thread -> row t/4, 16 frequencies
+    uint2* const undecided = reinterpret_cast<uint2*>(own[w]);  // (argument, element of act)
+    int held = 0;
+    // ---- Fourier features (k_features): a particle a lane, 16 frequencies a
+    // wavefront
     {
-        const int r = t >> 2, c0 = (t & 3) * 16;
-        const int64_t gr = r0 + r < n ? r0 + r : n - 1;
+        const int64_t gr = r0 + lane < n ? r0 + lane : n - 1;
         float u[4];
 #pragma unroll
         for (int d = 0; d < 4; ++d) u[d] = (inp[4 * gr + d] - net.shift[d]) / net.scale[d];
-#pragma unroll 4
+#pragma unroll 1
         for (int i = 0; i < 16; ++i) {
-            const int c = c0 + i;
+            const int c = 16 * w + i;
             float z = 0.f;
 #pragma unroll
             for (int d = 0; d < 4; ++d) z += u[d] * net.Bf[d * kInferHalf + c];
-            z *= 6.283185307179586f;
-            act[0][r][c] = f2bf(sinf(z));
-            act[0][r][kInferHalf + c] = f2bf(cosf(z));
+            bool und[2];
+            const uint2 g = sincos_near(z, und[0], und[1]);
+            const int at[2] = {act_at(lane, c), act_at(lane, kInferHalf + c)};
+            act[at[0]] = static_cast<uint16_t>(g.x);
+            act[at[1]] = static_cast<uint16_t>(g.y);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const uint64_t m = __ballot(und[q]);
+                if (und[q])
+                    undecided[held + rank_in(m)] =
+                        make_uint2(__float_as_uint(z), static_cast<uint32_t>(at[q]) | q << 31);
+                held += __popcll(m);
+            }
+            if (held <= kUndecided - 128 && i < 15) continue;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll 1
+            for (int first = lane; first < held; first += 64) {
+                const uint2 e = undecided[first];
+                float sn, cs;
+                sincosf(__uint_as_float(e.x) * 6.283185307179586f, &sn, &cs);
+                act[e.y & 0x7fffffffu] = f2bf(e.y >> 31 ? cs : sn);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            held = 0;
         }
     }
     __syncthreads();
     // ---- hidden layers
-    const int r16 = lane & 15, kk = 8 * (lane >> 4);
-    int cur = 0;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    bf16x8* const stage = reinterpret_cast<bf16x8*>(own[w]);
+    const bf16x8* const fragment =
+        reinterpret_cast<const bf16x8*>(own[w]) + 4 * r16 + (g4 ^ (r16 >> 2));
 #pragma unroll 1
     for (int l = 0; l < 4; ++l) {
         const int K = l == 0 ? 2 * kInferHalf : kInferWidth;
-        const uint16_t* __restrict__ WT = net.WT[l];
         f32x4 acc[4][4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        bf16x8 bnext[4];
+        const uint16_t* const wt =
+            net.WT[l] + (64 * w + (lane >> 2)) * K + 8 * ((lane & 3) ^ g4);
+        bf16x8 raw[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            bnext[j] = *reinterpret_cast<const bf16x8*>(
-                WT + static_cast<long>(64 * w + 16 * j + r16) * K + kk);
+        for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const bf16x8*>(wt + 16 * j * K);
 #pragma unroll 1
         for (int k0 = 0; k0 < K; k0 += 32) {
-            bf16x8 bcur[4];
+            const int next = k0 + 32 < K ? k0 + 32 : k0;
+            bf16x8 bf[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) bcur[j] = bnext[j];
-            if (k0 + 32 < K) {
+            for (int h = 0; h < 4; h += 2) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                stage[lane] = raw[h];
+                stage[64 + lane] = raw[h + 1];
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    bnext[j] = *reinterpret_cast<const bf16x8*>(
-                        WT + static_cast<long>(64 * w + 16 * j + r16) * K + k0 + 32 + kk);
+                for (int j = h; j < h + 2; ++j)
+                    raw[j] = *reinterpret_cast<const bf16x8*>(wt + 16 * j * K + next);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                bf[h] = fragment[0];
+                bf[h + 1] = fragment[64];
             }
-            bf16x8 af[4];
+            const int col = ((k0 >> 3) + g4) ^ r16;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                af[i] = *reinterpret_cast<const bf16x8*>(&act[cur][16 * i + r16][k0 + kk]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i) {
+                const bf16x8 af = *reinterpret_cast<const bf16x8*>(
+                    act + (16 * i + r16) * kInferWidth + 8 * col);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bcur[j], acc[i][j],
-                                                                        0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af, acc[i][j], 0, 0, 0);
+            }
         }
-        const int nxt = cur ^ 1;
-        const int rq = 4 * (lane >> 4);
-#pragma unroll
+        __syncthreads();  // every wavefront has read the layer's inputs
+#pragma unroll 1
         for (int j = 0; j < 4; ++j) {
-            const int nc = 64 * w + 16 * j + r16;
-            const float bias = net.b[l][nc];
+            const int nc = 64 * w + 16 * j + 4 * g4;
+            const int at0 = act_at(r16, nc);
+            float bias[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bias[q] = net.b[l][nc + q];
+            uint64_t open[4][4];
+            uint64_t any = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float g[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    bool und;
+                    g[q] = gelu_near(acc[i][0][q] + bias[q], und);
+                    open[i][q] = __ballot(und);
+                    any |= open[i][q];
+                }
+                *reinterpret_cast<uint2*>(act + at0 + 16 * i * kInferWidth) =
+                    make_uint2(pack_bf16(g[0], g[1]), pack_bf16(g[2], g[3]));
+            }
+            // list the undecided; evaluate where the list is full or complete
+            while (any != 0ull || (j == 3 && held > 0)) {
+                any = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint64_t m = open[i][q];
+                        const int count = __popcll(m);
+                        if (count == 0) continue;
+                        if (held + count > kUndecided) {
+                            any |= m;
+                            continue;
+                        }
+                        if (m >> lane & 1)
+                            undecided[held + rank_in(m)] =
+                                make_uint2(__float_as_uint(acc[i][0][q] + bias[q]),
+                                           at0 + 16 * i * kInferWidth + q);
+                        held += count;
+                        open[i][q] = 0;
+                    }
+                if (any == 0ull && j < 3) break;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll 1
+                for (int first = lane; first < held; first += 64) {
+                    const uint2 e = undecided[first];
+                    act[e.y] = f2bf(gelu(__uint_as_float(e.x)));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                held = 0;
+            }
+            // the next column of tiles (static registers: the loop stays rolled)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    act[nxt][16 * i + rq + q][nc] = f2bf(gelu(acc[i][j][q] + bias));
+                for (int c = 0; c < 3; ++c) acc[i][c] = acc[i][c + 1];
         }
         __syncthreads();
-        cur = nxt;
     }
-    // ---- head (k_out_fwd's sequential sums) and output scaling
-    if (t < 2 * kInferRows) {
-        const int r = t >> 1, c = t & 1;
-        if (r0 + r < n) {
-            float sum = 0.f;
-            for (int k = 0; k < kInferWidth; ++k) sum += bf2f(act[cur][r][k]) * bf2f(net.Wout[2 * k + c]);
-            out[2 * (r0 + r) + c] = (sum + net.bout[c]) * net.out_scale[c];
+    // ---- head (k_out_fwd's sequential sums) and output scaling: one wavefront,
+    // a particle a lane, the 512 weights as floats over the list's memory
+    static_assert(kWaveBytes >= 2 * kInferWidth * sizeof(float), "");
+    if (w != (blockIdx.x & 3)) return;
+    float* const wf = reinterpret_cast<float*>(own[w]);
+    {
+        const u16x8 h = *reinterpret_cast<const u16x8*>(net.Wout + 8 * lane);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) wf[8 * lane + q] = bf2f(h[q]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (r0 + lane >= n) return;
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll 4
+    for (int k8 = 0; k8 < kInferWidth; k8 += 8) {
+        const u16x8 h = *reinterpret_cast<const u16x8*>(act + act_at(lane, k8));
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            s0 += bf2f(h[q]) * wf[2 * (k8 + q)];
+            s1 += bf2f(h[q]) * wf[2 * (k8 + q) + 1];
         }
     }
+    out[2 * (r0 + lane)] = (s0 + net.bout[0]) * net.out_scale[0];
+    out[2 * (r0 + lane) + 1] = (s1 + net.bout[1]) * net.out_scale[1];
 }
 
 int check_gemm_shape(int M, int N, int K) {

@@ -123,3 +123,30 @@ def test_bickley_queue_equals_grid_launch(precision):
         autotune.set_config(1, precision, saved)
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("kind", ["plain", "wide", "negative", "nonfinite"])
+def test_fused_inference_where_rounding_is_undecided(n, kind):
+    """The fused kernel's short forms of GELU, sine and cosine hand over to the
+    library functions wherever these could round otherwise, so it equals the
+    layer-by-layer kernels bit for bit: ordinary particles, features of
+    thousands of revolutions, activations below -4 throughout (every one is
+    handed over, so the lists fill), and arguments that are not finite."""
+    import torch
+    from numbacs_amd.surrogate import MLPSurrogate
+
+    rng = np.random.default_rng(n)
+    net = MLPSurrogate([0.0] * 4, [1.0] * 4, out_scale=[10.0, 5.0], seed=n)
+    x = rng.uniform(-1, 1, (n, 4)).astype(np.float32)
+    if kind == "wide":
+        x *= rng.choice(np.float32([1e1, 1e3, 1e4, 1e7]), (n, 1))
+    if kind == "negative":
+        for b in net.b[:4]:
+            b.fill_(-6.0)
+    if kind == "nonfinite":
+        x[rng.integers(0, n, 3), rng.integers(0, 4, 3)] = [np.inf, -np.inf, np.nan]
+    inp = torch.tensor(x, device="cuda")
+    a, b = net.predict_device(inp), net.predict_device_unfused(inp)
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
