@@ -9,22 +9,24 @@
 // Device pipeline (with a percentile threshold no host round trip before the
 // end, the grouping stage being sized by a bound on the ridge-point count;
 // without one the count is read back to size it):
-//   percentile  : two radix selects (8 passes of 8 bits over order-preserving
-//                 64-bit keys, each pass's blocks first picking the previous
-//                 pass's digit) for the order statistics around the virtual
-//                 index, then numpy's two-sided lerp -- f_min stays in HBM;
+//   percentile  : two radix selects (6 passes of 11 or 10 bits over
+//                 order-preserving 64-bit keys, each pass's blocks first
+//                 picking the previous pass's digit) for the order statistics
+//                 around the virtual index, then numpy's two-sided lerp --
+//                 f_min stays in HBM;
 //   predicate   : one thread per grid point, the reference's central
 //                 differences and Steger sub-pixel test;
-//   compaction  : exclusive scan over the ridge flags (tile scans, then the
-//                 tile offsets, which consumers of the grouping path add
-//                 themselves), so points come out in raveled (i*ny+j) order;
-//   labelling   : lock-free union-find (atomicMin linking of the larger root
-//                 under the smaller) over the 4 raster-earlier neighbours,
-//                 then path flattening; every root is its component's
-//                 smallest raveled index, so ordering components by root is
+//   labelling   : union-find (the larger root linked under the smaller), in LDS
+//                 within 16 x 64 tiles by the predicate's blocks, then
+//                 lock-free (atomicMin) across the tiles' borders, then path
+//                 flattening; every root is its component's smallest raveled
+//                 index, so ordering components by root is
 //                 scipy.ndimage.label's raster order of first pixels;
-//   grouping    : bitonic sort of (root << 32 | index) keys, segment
-//                 boundaries, min_ridge_pts filter and a scatter.
+//   compaction  : counts of ridge points and roots a 1024-point tile, their
+//                 scan, then the points in raveled (i*ny+j) order and the
+//                 roots' ranks;
+//   grouping    : stable radix sort of the points by component, segment
+//                 starts, min_ridge_pts filter and a scatter.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -51,24 +53,35 @@ constexpr int kScanThreads = 256;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;  // 1024 flags per block
 
-constexpr int kSortThreads = 512;
-constexpr int kSortChunk = 2 * kSortThreads;  // keys per LDS chunk
-
 // Radix-select state.  The digit picked from pass p's histograms is
 // computed by every block of pass p+1 (and by the finishing kernel after the
 // last pass) instead of by a launch of its own, so the histograms rotate
 // over three buffers (pass p adds into hist[p % 3], reads hist[(p-1) % 3]
 // and clears hist[(p+1) % 3], which no block of p reads or writes) and the
 // digit state over two (pass p's blocks read the state of pass p-1's
-// search, block 0 stores the updated one for pass p+1).
+// search, block 0 stores the updated one for pass p+1).  While both searches
+// share a prefix only search 0's histogram is filled, for both.
+constexpr int kSelThreads = 1024, kSelPasses = 6, kSelBins = 2048;
+constexpr int kSelOwn = kSelBins / kSelThreads;  // bins a thread
+// keys kept once their first 22 bits are known (all later passes read these)
+constexpr int64_t kSelHeld = 65536;
+constexpr unsigned kSelStage = 1024;  // of them a block collects before one append
+
 struct SelState {
     unsigned long long prefix[2][2];  // [pass & 1][search]
     unsigned long long mask[2][2];
     long long k[2][2];
-    unsigned int hist[3][2][256];     // [pass % 3][search][bin]
+    unsigned int hist[3][2][kSelBins];  // [pass % 3][search][bin]
     unsigned int nan_count;
+    unsigned int held;  // keys offered to the list; past its room it is not used
     double result;
 };
+
+// digits of 11, 11, 11, 11, 10 and 10 bits from the top
+__host__ __device__ constexpr int sel_shift(int pass) {
+    return pass < 4 ? 53 - 11 * pass : 10 * (kSelPasses - 1 - pass);
+}
+__host__ __device__ constexpr unsigned sel_digit(int pass) { return pass < 4 ? 2047u : 1023u; }
 
 __device__ __forceinline__ unsigned long long order_key(double v) {
     const unsigned long long b = __double_as_longlong(v);
@@ -82,74 +95,105 @@ __device__ __forceinline__ double key_value(unsigned long long k) {
 
 __global__ void k_sel_init(SelState* st, long long k_lo, long long k_hi) {
     const int t = threadIdx.x;
-    if (t < 256) {
-        st->hist[0][0][t] = 0;
-        st->hist[0][1][t] = 0;
-    }
+    for (int b = t; b < kSelBins; b += blockDim.x) st->hist[0][0][b] = st->hist[0][1][b] = 0;
     if (t == 0) {
         st->prefix[0][0] = st->prefix[0][1] = 0;
         st->mask[0][0] = st->mask[0][1] = 0;
         st->k[0][0] = k_lo;
         st->k[0][1] = k_hi;
         st->nan_count = 0;
+        st->held = 0;
         st->result = 0.0;
     }
 }
 
-// Digit state of both searches after pass `prev` (digit at `shift`), into
-// LDS: an inclusive scan of the pass's 256-bin histograms, then the bin
-// whose cumulative count first exceeds k.  Called by all 256 threads; ends
-// with a barrier.
-__device__ void sel_advance(const SelState* st, int prev, int shift, long long (*cum)[256],
-                            unsigned long long* sp, unsigned long long* sm, long long* sk) {
-    const int b = threadIdx.x;
+// Digit state of both searches after pass `prev`, into LDS: the bin whose
+// cumulative count first exceeds k.  Called by all kSelThreads threads,
+// kSelOwn neighbouring bins each; ends with a barrier.
+__device__ void sel_advance(const SelState* st, int prev, unsigned long long* sp,
+                            unsigned long long* sm, long long* sk) {
+    __shared__ unsigned int waves[2][kSelThreads / 64];
+    const int t = threadIdx.x, lane = t & 63;
     const int sb = prev & 1, hb = prev % 3;
-    cum[0][b] = st->hist[hb][0][b];
-    cum[1][b] = st->hist[hb][1][b];
-    if (b < 2) {
-        sp[b] = st->prefix[sb][b];
-        sm[b] = st->mask[sb][b];
-        sk[b] = st->k[sb][b];
-    }
-    __syncthreads();
-    // read both ranks before any thread updates them (the scan's barriers
-    // order these reads before the single writer below)
-    const long long kk[2] = {sk[0], sk[1]};
-    for (int off = 1; off < 256; off <<= 1) {
-        const long long a0 = b >= off ? cum[0][b - off] : 0;
-        const long long a1 = b >= off ? cum[1][b - off] : 0;
-        __syncthreads();
-        cum[0][b] += a0;
-        cum[1][b] += a1;
-        __syncthreads();
-    }
+    const int same = st->prefix[sb][0] == st->prefix[sb][1];
+    unsigned int c[2][kSelOwn], before[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        const long long k = kk[s];
-        const long long before = b > 0 ? cum[s][b - 1] : 0;
-        // exactly one bin has before <= k < cum (k < total always holds)
-        if (before <= k && k < cum[s][b]) {
-            sk[s] = k - before;
-            sp[s] |= static_cast<unsigned long long>(b) << shift;
-            sm[s] |= 0xffull << shift;
+        unsigned int x = 0;
+#pragma unroll
+        for (int q = 0; q < kSelOwn; ++q) {
+            c[s][q] = st->hist[hb][same ? 0 : s][kSelOwn * t + q];
+            x += c[s][q];
+        }
+        before[s] = x;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned int y = __shfl_up(x, off);
+            if (lane >= off) x += y;
+        }
+        before[s] = x - before[s];
+        if (lane == 63) waves[s][t >> 6] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        for (int w = 0; w < (t >> 6); ++w) before[s] += waves[s][w];
+        const long long k = st->k[sb][s];
+        long long at = before[s];
+#pragma unroll
+        for (int q = 0; q < kSelOwn; ++q) {
+            // exactly one bin has at <= k < at + count (k < total always holds)
+            if (at <= k && k < at + c[s][q]) {
+                sk[s] = k - at;
+                sp[s] = st->prefix[sb][s] |
+                        static_cast<unsigned long long>(kSelOwn * t + q) << sel_shift(prev);
+                sm[s] = st->mask[sb][s] |
+                        static_cast<unsigned long long>(sel_digit(prev)) << sel_shift(prev);
+            }
+            at += c[s][q];
         }
     }
     __syncthreads();
 }
 
-// Pass `pass` (digit at bits 56 - 8*pass) of both searches.
-__global__ __launch_bounds__(256) void k_sel_hist(const double* __restrict__ f, int64_t n,
-                                                  SelState* st, int pass) {
-    __shared__ unsigned int h[2][256];
-    __shared__ unsigned int nans;
-    __shared__ long long cum[2][256];
+// h[bin] += 1 for the lanes with `on`, the first lane's bin in one step: the
+// leading digits of a smooth field agree over most of a wavefront, and 64
+// atomics on one LDS word take 64 turns.
+__device__ __forceinline__ void sel_count(unsigned int* h, unsigned int bin, bool on) {
+    const uint64_t m = __ballot(on);
+    if (m == 0) return;
+    const int first = __builtin_ctzll(m);
+    const unsigned int b0 = __builtin_amdgcn_readlane(bin, first);
+    const uint64_t same = __ballot(on && bin == b0);
+    if (static_cast<int>(threadIdx.x & 63) == first)
+        atomicAdd(&h[b0], static_cast<unsigned int>(__popcll(same)));
+    else if (on && bin != b0)
+        atomicAdd(&h[bin], 1u);
+}
+
+// Pass `pass` of both searches.  Passes 0 to 2 read the array; pass 2 also
+// lists the keys that match either prefix (22 bits: some thousands of 8 M
+// values of an FTLE field), and the later passes read that list.  Where it
+// overflows (many values equal in 22 bits) they read the array again.
+// Bound by the reads (13 us of the 17 to 21 a pass over 8 M values takes; then
+// 5.5 us a pass over the list): the whole percentile 156 -> 84 us, with digits of
+// 8 bits and every pass over the array before.
+__global__ __launch_bounds__(kSelThreads) void k_sel_hist(const double* __restrict__ f, int64_t n,
+                                                          SelState* st, int pass,
+                                                          unsigned long long* held,
+                                                          int64_t room) {
+    __shared__ unsigned int h[2][kSelBins];
     __shared__ unsigned long long sp[2], sm[2];
     __shared__ long long sk[2];
+    __shared__ unsigned long long own[kSelStage];
+    __shared__ unsigned int staged, fits, out;
     const int t = threadIdx.x;
-    const int shift = 56 - 8 * pass;
-    h[0][t] = 0;
-    h[1][t] = 0;
-    if (t == 0) nans = 0;
+    const int shift = sel_shift(pass);
+    if (t == 0) {
+        staged = 0;
+        fits = kSelStage;
+    }
+    for (int b = t; b < 2 * kSelBins; b += kSelThreads) h[0][b] = 0;
     if (pass == 0) {
         if (t < 2) {
             sp[t] = st->prefix[0][t];
@@ -158,7 +202,7 @@ __global__ __launch_bounds__(256) void k_sel_hist(const double* __restrict__ f, 
         }
         __syncthreads();
     } else {
-        sel_advance(st, pass - 1, shift + 8, cum, sp, sm, sk);
+        sel_advance(st, pass - 1, sp, sm, sk);
     }
     if (blockIdx.x == 0) {
         if (pass > 0 && t < 2) {
@@ -166,34 +210,85 @@ __global__ __launch_bounds__(256) void k_sel_hist(const double* __restrict__ f, 
             st->mask[pass & 1][t] = sm[t];
             st->k[pass & 1][t] = sk[t];
         }
-        st->hist[(pass + 1) % 3][0][t] = 0;
-        st->hist[(pass + 1) % 3][1][t] = 0;
+        unsigned int* next = st->hist[(pass + 1) % 3][0];
+        for (int b = t; b < 2 * kSelBins; b += kSelThreads) next[b] = 0;
     }
-    const unsigned long long p0 = sp[0], m0 = sm[0];
-    const unsigned long long p1 = sp[1], m1 = sm[1];
-    for (int64_t k = blockIdx.x * static_cast<int64_t>(blockDim.x) + t; k < n;
-         k += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const double v = f[k];
-        if (pass == 0 && v != v) atomicAdd(&nans, 1u);
-        const unsigned long long key = order_key(v);
-        const unsigned int bin = static_cast<unsigned int>((key >> shift) & 0xffu);
-        if ((key & m0) == p0) atomicAdd(&h[0][bin], 1u);
-        if ((key & m1) == p1) atomicAdd(&h[1][bin], 1u);
+    const unsigned long long p0 = sp[0], p1 = sp[1], mask = sm[0];  // one mask: equal digits
+    const bool one = p0 == p1;
+    const bool listed = pass > 2 && st->held <= room;
+    const int64_t count = listed ? st->held : n;
+    const unsigned long long* from =
+        listed ? held : reinterpret_cast<const unsigned long long*>(f);
+    bool room_left = pass == 2;
+    unsigned int nans = 0;
+    for (int64_t base = blockIdx.x * static_cast<int64_t>(4 * kSelThreads); base < count;
+         base += static_cast<int64_t>(gridDim.x) * (4 * kSelThreads)) {
+        unsigned long long key[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t k = base + q * kSelThreads + t;
+            key[q] = from[k < count ? k : count - 1];
+        }
+        if (!listed) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) key[q] = order_key(__longlong_as_double(key[q]));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool in = base + q * kSelThreads + t < count;
+            const double v = key_value(key[q]);
+            if (pass == 0 && in && v != v) ++nans;
+            const unsigned int bin =
+                static_cast<unsigned int>(key[q] >> shift) & sel_digit(pass);
+            const bool on0 = in && (key[q] & mask) == p0;
+            const bool on1 = in && !one && (key[q] & mask) == p1;
+            sel_count(h[0], bin, on0);
+            if (!one) sel_count(h[1], bin, on1);
+            if (!room_left) continue;
+            const uint64_t m = __ballot(on0 || on1);
+            if (m == 0) continue;
+            const int lane = t & 63, first = __builtin_ctzll(m);
+            const unsigned int c = __popcll(m), rank = __popcll(m & ((1ull << lane) - 1));
+            unsigned int at = 0;
+            if (lane == first) at = atomicAdd(&staged, c);
+            at = __builtin_amdgcn_readlane(at, first);
+            if (at + c <= kSelStage) {
+                if (on0 || on1) own[at + rank] = key[q];
+                continue;
+            }
+            // the block's own list is full (and stays so: staged only grows, and
+            // what fitted ends where the first that did not began): straight to
+            // memory
+            if (lane == first) {
+                atomicMin(&fits, at);
+                at = atomicAdd(&st->held, c);
+            }
+            at = __builtin_amdgcn_readlane(at, first);
+            room_left = at + c <= room;
+            if (room_left && (on0 || on1)) held[at + rank] = key[q];
+        }
     }
     __syncthreads();
+    const unsigned int list = staged < fits ? staged : fits;
+    if (list) {  // pass 2 only
+        if (t == 0) out = atomicAdd(&st->held, list);
+        __syncthreads();
+        for (unsigned int b = t; b < list; b += kSelThreads)
+            if (out + b < room) held[out + b] = own[b];
+    }
     unsigned int* gh = st->hist[pass % 3][0];
-    if (h[0][t]) atomicAdd(&gh[t], h[0][t]);
-    if (h[1][t]) atomicAdd(&gh[256 + t], h[1][t]);
-    if (t == 0 && nans) atomicAdd(&st->nan_count, nans);
+    for (int b = t; b < 2 * kSelBins; b += kSelThreads)
+        if (h[0][b]) atomicAdd(&gh[b], h[0][b]);
+    if (nans) atomicAdd(&st->nan_count, nans);
 }
 
-// The last digit (pass 7, bits 0-7), then numpy's _lerp: a + (b-a)*g, or
-// b - (b-a)*(1-g) when g >= 0.5.
-__global__ __launch_bounds__(256) void k_sel_finish(SelState* st, double gamma, double* out) {
-    __shared__ long long cum[2][256];
+// The last digit, then numpy's _lerp: a + (b-a)*g, or b - (b-a)*(1-g) when
+// g >= 0.5.
+__global__ __launch_bounds__(kSelThreads) void k_sel_finish(SelState* st, double gamma,
+                                                            double* out) {
     __shared__ unsigned long long sp[2], sm[2];
     __shared__ long long sk[2];
-    sel_advance(st, 7, 0, cum, sp, sm, sk);
+    sel_advance(st, kSelPasses - 1, sp, sm, sk);
     if (threadIdx.x != 0) return;
     const double a = key_value(sp[0]);
     const double b = key_value(sp[1]);
@@ -204,8 +299,9 @@ __global__ __launch_bounds__(256) void k_sel_finish(SelState* st, double gamma, 
     if (out) *out = r;
 }
 
-int percentile_device(const double* f, int64_t n, double q, SelState* st, double* out,
-                      hipStream_t s) {
+// held: room for min(n, kSelHeld) keys
+int percentile_device(const double* f, int64_t n, double q, SelState* st,
+                      unsigned long long* held, double* out, hipStream_t s) {
     NBX_REQUIRE(n >= 1, "percentile of an empty array");
     NBX_REQUIRE(q >= 0 && q <= 100, "percentile must be in [0, 100]");
     // numpy 'linear': virtual index (n-1) * (q/100); neighbours clamped to the
@@ -219,66 +315,70 @@ int percentile_device(const double* f, int64_t n, double q, SelState* st, double
     const double gamma = vi - lo;
     k_sel_init<<<1, 256, 0, s>>>(st, klo, khi);
     NBX_LAUNCHED("sel_init");
-    // about 8 keys per thread: every block adds its nonzero bins to the same
-    // 512 global counters, and on the first passes nearly all keys share a
-    // few bins, so fewer blocks serialise fewer atomics on each counter
-    unsigned nb = blocks_for(n, 256 * 8);
-    if (nb > 1024) nb = 1024;
-    for (int pass = 0; pass < 8; ++pass) {
-        k_sel_hist<<<nb, 256, 0, s>>>(f, n, st, pass);
+    // about 16 keys per thread, at most a block a CU: every block adds its
+    // nonzero bins to the same global counters (8 M values: 75 us for the passes;
+    // 512 blocks 77, of half the threads 83)
+    unsigned nb = blocks_for(n, kSelThreads * 16);
+    if (nb > 256) nb = 256;
+    for (int pass = 0; pass < kSelPasses; ++pass) {
+        k_sel_hist<<<nb, kSelThreads, 0, s>>>(f, n, st, pass, held, n < kSelHeld ? n : kSelHeld);
         NBX_LAUNCHED("sel_hist");
     }
-    k_sel_finish<<<1, 256, 0, s>>>(st, gamma, out);
+    k_sel_finish<<<1, kSelThreads, 0, s>>>(st, gamma, out);
     NBX_LAUNCHED("sel_finish");
     return 0;
 }
 
 // ---------------------------------------------------------------------------
-// Ridge predicate (ridges.py:52-74): flag[k] = 1 and pts[k] = sub-pixel ridge
-// point where the test passes, flag[k] = 0 elsewhere.
-__global__ __launch_bounds__(256) void k_ridge_predicate(
-    const double* __restrict__ f, const double2* __restrict__ evec, const double* __restrict__ xs,
-    const double* __restrict__ ys, int nx, int ny, double dx, double dy, double sdd_thresh,
-    const double* __restrict__ fmin_dev, int32_t* __restrict__ flag, double2* __restrict__ pts,
-    double* __restrict__ sdd_out, int32_t* __restrict__ uf_par) {
+// Ridge predicate (ridges.py:52-74) at grid point (i, j): whether the test
+// passes, then pts[k] = the sub-pixel ridge point and sdd = the second
+// derivative.
+__device__ __forceinline__ bool ridge_test(const double* __restrict__ f,
+                                           const double2* __restrict__ evec,
+                                           const double* __restrict__ xs,
+                                           const double* __restrict__ ys, int nx, int ny, int i,
+                                           int j, double f0, double dx, double dy,
+                                           double sdd_thresh, double f_min,
+                                           double2* __restrict__ pts, double& sdd) {
     // the reference's expressions in its source order, uncontracted: ridge
     // points and second derivatives equal the oracle's bit for bit, so the
     // ordered-ridge linking (which compares them) takes the same decisions
 #pragma clang fp contract(off)
+    if (i < 2 || i >= nx - 2 || j < 2 || j >= ny - 2) return false;
+    if (!(f0 > f_min)) return false;
+    const long k = static_cast<long>(i) * ny + j;
+    const double fe = f[k + ny], fw = f[k - ny], fn = f[k + 1], fs = f[k - 1];
+    const double fx = (fe - fw) / (2 * dx);
+    const double fy = (fn - fs) / (2 * dy);
+    const double fxx = (fe - 2 * f0 + fw) / (dx * dx);
+    const double fyy = (fn - 2 * f0 + fs) / (dy * dy);
+    const double fxy =
+        (f[k + ny + 1] - f[k + ny - 1] - f[k - ny + 1] + f[k - ny - 1]) / (4 * dx * dy);
+    const double2 e = evec[k];
+    const double ex = e.x, ey = e.y;
+    const double c2 = ex * (fxx * ex + fxy * ey) + ey * (fxy * ex + fyy * ey);
+    if (!(c2 < -sdd_thresh)) return false;
+    const double t = -(fx * ex + fy * ey) / c2;
+    if (!(fabs(t * ex) <= dx / 2 && fabs(t * ey) <= dy / 2)) return false;
+    pts[k] = make_double2(xs[i] + t * ex, ys[j] + t * ey);
+    sdd = c2;
+    return true;
+}
+
+// flag[k] = 1 where the test passes, 0 elsewhere
+__global__ __launch_bounds__(256) void k_ridge_predicate(
+    const double* __restrict__ f, const double2* __restrict__ evec, const double* __restrict__ xs,
+    const double* __restrict__ ys, int nx, int ny, double dx, double dy, double sdd_thresh,
+    const double* __restrict__ fmin_dev, int32_t* __restrict__ flag, double2* __restrict__ pts,
+    double* __restrict__ sdd_out) {
     const int j = blockIdx.x * 64 + threadIdx.x;
     const int i = blockIdx.y * 4 + threadIdx.y;
     if (i >= nx || j >= ny) return;
     const long k = static_cast<long>(i) * ny + j;
-    int32_t hit = 0;
     double sdd = 0.0;
-    if (i >= 2 && i < nx - 2 && j >= 2 && j < ny - 2) {
-        const double f_min = fmin_dev ? *fmin_dev : 0.0;
-        const double f0 = f[k];
-        if (f0 > f_min) {
-            const double fe = f[k + ny], fw = f[k - ny], fn = f[k + 1], fs = f[k - 1];
-            const double fx = (fe - fw) / (2 * dx);
-            const double fy = (fn - fs) / (2 * dy);
-            const double fxx = (fe - 2 * f0 + fw) / (dx * dx);
-            const double fyy = (fn - 2 * f0 + fs) / (dy * dy);
-            const double fxy = (f[k + ny + 1] - f[k + ny - 1] - f[k - ny + 1] + f[k - ny - 1]) /
-                               (4 * dx * dy);
-            const double2 e = evec[k];
-            const double ex = e.x, ey = e.y;
-            const double c2 = ex * (fxx * ex + fxy * ey) + ey * (fxy * ex + fyy * ey);
-            if (c2 < -sdd_thresh) {
-                const double t = -(fx * ex + fy * ey) / c2;
-                if (fabs(t * ex) <= dx / 2 && fabs(t * ey) <= dy / 2) {
-                    pts[k] = make_double2(xs[i] + t * ex, ys[j] + t * ey);
-                    hit = 1;
-                    sdd = c2;
-                }
-            }
-        }
-    }
-    flag[k] = hit;
+    flag[k] = ridge_test(f, evec, xs, ys, nx, ny, i, j, f[k], dx, dy, sdd_thresh,
+                         fmin_dev ? *fmin_dev : 0.0, pts, sdd);
     if (sdd_out != nullptr) sdd_out[k] = sdd;
-    // union-find start (each ridge point its own root), when labelling follows
-    if (uf_par != nullptr) uf_par[k] = hit ? static_cast<int32_t>(k) : -1;
 }
 
 // ---------------------------------------------------------------------------
@@ -295,28 +395,40 @@ __device__ __forceinline__ I2& operator+=(I2& x, I2 y) {
     return x;
 }
 
+__device__ __forceinline__ int32_t lane_up(int32_t x, int off) { return __shfl_up(x, off); }
+__device__ __forceinline__ I2 lane_up(I2 x, int off) {
+    return I2{__shfl_up(x.a, off), __shfl_up(x.b, off)};
+}
+
+// over the block's kScanThreads values; sh holds one value per wavefront
 template <class T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T* sh, T* total) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanThreads; off <<= 1) {
-        const T add = t >= off ? sh[t - off] : T{};
-        __syncthreads();
-        sh[t] += add;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    T x = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const T y = lane_up(x, off);
+        if (lane >= off) x += y;
     }
-    const T ex = t > 0 ? sh[t - 1] : T{};
-    *total = sh[kScanThreads - 1];
+    if (lane == 63) sh[w] = x;
+    const T prev = lane_up(x, 1);
+    T ex = lane > 0 ? prev : T{};
+    __syncthreads();
+    T sum{};
+#pragma unroll
+    for (int q = 0; q < kScanThreads / 64; ++q) {
+        if (q == w) ex += sum;
+        sum += sh[q];
+    }
+    *total = sum;
     __syncthreads();
     return ex;
 }
 
 template <class T>
-__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const T* __restrict__ in, int64_t n,
-                                                             T* __restrict__ out,
+__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const T* in, int64_t n, T* out,
                                                              T* __restrict__ tile_sums) {
-    __shared__ T sh[kScanThreads];
+    __shared__ T sh[kScanThreads / 64];
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
     T v[kScanItems];
     T sum{};
@@ -339,14 +451,23 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const T* __restrict
 template <class T>
 __global__ __launch_bounds__(kScanThreads) void k_scan_sums(T* __restrict__ sums, int64_t m,
                                                             T* __restrict__ total) {
-    __shared__ T sh[kScanThreads];
+    __shared__ T sh[kScanThreads / 64];
+    constexpr int kItems = 8;
     T carry{};
-    for (int64_t base = 0; base < m; base += kScanThreads) {
-        const int64_t k = base + threadIdx.x;
-        const T v = k < m ? sums[k] : T{};
-        T chunk;
-        const T ex = block_exclusive_scan(v, sh, &chunk);
-        if (k < m) sums[k] = carry + ex;
+    for (int64_t base = 0; base < m; base += kScanThreads * kItems) {
+        const int64_t k = base + threadIdx.x * kItems;
+        T v[kItems], sum{}, chunk;
+#pragma unroll
+        for (int q = 0; q < kItems; ++q) {
+            v[q] = k + q < m ? sums[k + q] : T{};
+            sum += v[q];
+        }
+        T run = carry + block_exclusive_scan(sum, sh, &chunk);
+#pragma unroll
+        for (int q = 0; q < kItems; ++q) {
+            if (k + q < m) sums[k + q] = run;
+            run += v[q];
+        }
         carry += chunk;
     }
     if (threadIdx.x == 0) *total = carry;
@@ -402,17 +523,12 @@ int exclusive_scan_tiled(const T* in, int64_t n, T* out, T* tile_off, T* total, 
 }
 
 // ---------------------------------------------------------------------------
-// Compaction of flagged points in raveled order.
-// pos is a complete exclusive scan, or with tile_off the tiled form.
+// Compaction of flagged points in raveled order (pos: the flags' scan).
 __global__ void k_compact(const int32_t* __restrict__ flag, const int32_t* __restrict__ pos,
                           const double2* __restrict__ pts_dense, int64_t n,
-                          double2* __restrict__ pts_out, int32_t* __restrict__ idx_out,
-                          const int32_t* __restrict__ tile_off) {
+                          double2* __restrict__ pts_out) {
     const int64_t k = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (k >= n || !flag[k]) return;
-    const int32_t p = pos[k] + (tile_off ? tile_off[k / kScanTile] : 0);
-    if (pts_out) pts_out[p] = pts_dense[k];
-    if (idx_out) idx_out[p] = static_cast<int32_t>(k);
+    if (k < n && flag[k]) pts_out[pos[k]] = pts_dense[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -492,187 +608,319 @@ __global__ void k_label_out(const int32_t* __restrict__ par, const int32_t* __re
 }
 
 // ---------------------------------------------------------------------------
-// Bitonic sort of 64-bit keys; N is a power of two and a multiple of
-// kSortChunk.
+// The grouped pipeline's labelling: par[k] = -1 off the ridges.
 
-__device__ __forceinline__ void cmp_swap(unsigned long long& a, unsigned long long& b, bool up) {
-    if ((a > b) == up) {
-        const unsigned long long t = a;
-        a = b;
-        b = t;
+constexpr int kTileRows = 16, kTileCols = 64;
+
+__device__ __forceinline__ int tile_root(const int* par, int a) {
+    int p = __hip_atomic_load(par + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (p != a) {
+        a = p;
+        p = __hip_atomic_load(par + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    return a;
+}
+
+__device__ __forceinline__ void tile_unite(int* par, int a, int b) {
+    for (;;) {
+        a = tile_root(par, a);
+        b = tile_root(par, b);
+        if (a == b) return;
+        const int hi = a > b ? a : b, lo = a > b ? b : a;
+        const int old = atomicMin(par + hi, lo);
+        if (old == hi) return;
+        a = old;
+        b = lo;
     }
 }
 
-// all stages k <= kSortChunk inside one chunk
-__global__ __launch_bounds__(kSortThreads) void k_bitonic_chunk_full(unsigned long long* keys) {
-    __shared__ unsigned long long sh[kSortChunk];
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kSortChunk;
-    const int t = threadIdx.x;
-    sh[t] = keys[base + t];
-    sh[t + kSortThreads] = keys[base + t + kSortThreads];
+// Ridge predicate and the components within one 16 x 64 tile, linked in LDS:
+// a global link is a chain of loads past the caches, so those are left to the
+// tiles' borders (k_border_union), 8% of the points.  Position order within a
+// tile is raveled order, so a tile's root is its component's smallest raveled
+// index there.  The points above the threshold are listed first, so the test and
+// the links run on full wavefronts.  Bound by memory (f, and the scattered lines
+// of evec and pts at a tenth of the points): 2001 x 4001 points 62 us (predicate)
+// + 80 us (every link global) -> 59 + 15 us.  Tiles of 8 and 32 rows are no
+// faster.
+__global__ __launch_bounds__(256) void k_ridge_label(
+    const double* __restrict__ f, const double2* __restrict__ evec, const double* __restrict__ xs,
+    const double* __restrict__ ys, int nx, int ny, double dx, double dy, double sdd_thresh,
+    const double* __restrict__ fmin_dev, double2* __restrict__ pts, int32_t* __restrict__ par) {
+    constexpr int kPoints = kTileRows * kTileCols, kRows = kTileRows / 4;
+    __shared__ int own[kPoints];
+    __shared__ uint16_t list[kPoints];  // points above the threshold
+    __shared__ int listed;
+    const int lj = threadIdx.x, t = threadIdx.y * kTileCols + lj;
+    const int j0 = blockIdx.x * kTileCols, i0 = blockIdx.y * kTileRows, j = j0 + lj;
+    const double f_min = fmin_dev ? *fmin_dev : 0.0;
+    if (t == 0) listed = 0;
+    double f0[kRows];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+        const int i = i0 + threadIdx.y + 4 * q;
+        f0[q] = i < nx && j < ny ? f[static_cast<int64_t>(i) * ny + j] : 0.0;
+    }
     __syncthreads();
-    for (int k = 2; k <= kSortChunk; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            const int lo = 2 * j * (t / j) + (t % j);
-            const bool up = (((base + lo) & k) == 0);
-            cmp_swap(sh[lo], sh[lo + j], up);
-            __syncthreads();
-        }
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+        const int i = i0 + threadIdx.y + 4 * q, at = (i - i0) * kTileCols + lj;
+        const bool on = i < nx && j < ny && f0[q] > f_min;
+        const uint64_t m = __ballot(on);
+        own[at] = -1;
+        if (m == 0) continue;
+        int first = 0;
+        if (lj == 0) first = atomicAdd(&listed, __popcll(m));
+        first = __builtin_amdgcn_readfirstlane(first);
+        if (on) list[first + __popcll(m & ((1ull << lj) - 1))] = static_cast<uint16_t>(at);
     }
-    keys[base + t] = sh[t];
-    keys[base + t + kSortThreads] = sh[t + kSortThreads];
-}
-
-// stage k (> kSortChunk), steps j < kSortChunk inside one chunk
-__global__ __launch_bounds__(kSortThreads) void k_bitonic_chunk_tail(unsigned long long* keys,
-                                                                     int64_t k) {
-    __shared__ unsigned long long sh[kSortChunk];
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kSortChunk;
-    const int t = threadIdx.x;
-    sh[t] = keys[base + t];
-    sh[t + kSortThreads] = keys[base + t + kSortThreads];
     __syncthreads();
-    const bool up = ((base & k) == 0);
-    for (int j = kSortChunk >> 1; j > 0; j >>= 1) {
-        const int lo = 2 * j * (t / j) + (t % j);
-        cmp_swap(sh[lo], sh[lo + j], up);
-        __syncthreads();
+    const int count = listed;
+    for (int c = t; c < count; c += 256) {
+        const int at = list[c], i = i0 + at / kTileCols, jj = j0 + at % kTileCols;
+        double sdd;
+        if (ridge_test(f, evec, xs, ys, nx, ny, i, jj, f[static_cast<int64_t>(i) * ny + jj], dx, dy,
+                       sdd_thresh, f_min, pts, sdd))
+            own[at] = at;
     }
-    keys[base + t] = sh[t];
-    keys[base + t + kSortThreads] = sh[t + kSortThreads];
-}
-
-__global__ void k_bitonic_global(unsigned long long* keys, int64_t N, int64_t k, int64_t j) {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= N / 2) return;
-    const int64_t lo = 2 * j * (t / j) + (t % j);
-    const bool up = ((lo & k) == 0);
-    unsigned long long a = keys[lo], b = keys[lo + j];
-    if ((a > b) == up) {
-        keys[lo] = b;
-        keys[lo + j] = a;
-    }
-}
-
-// Two global steps of stage k in one pass, j and h = j/2: thread t owns the
-// four keys lo, lo+h, lo+j, lo+j+h (lo with bits j and h clear), a set that
-// both steps map onto itself, and all four share the direction of bit k.
-__global__ void k_bitonic_global2(unsigned long long* keys, int64_t N, int64_t k, int64_t h) {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= N / 4) return;
-    const int64_t lo = 4 * h * (t / h) + (t % h);
-    const bool up = ((lo & k) == 0);
-    unsigned long long a0 = keys[lo], a1 = keys[lo + h], a2 = keys[lo + 2 * h],
-                       a3 = keys[lo + 3 * h];
-    cmp_swap(a0, a2, up);
-    cmp_swap(a1, a3, up);
-    cmp_swap(a0, a1, up);
-    cmp_swap(a2, a3, up);
-    keys[lo] = a0;
-    keys[lo + h] = a1;
-    keys[lo + 2 * h] = a2;
-    keys[lo + 3 * h] = a3;
-}
-
-int bitonic_sort(unsigned long long* keys, int64_t N, hipStream_t s) {
-    const unsigned chunks = static_cast<unsigned>(N / kSortChunk);
-    k_bitonic_chunk_full<<<chunks, kSortThreads, 0, s>>>(keys);
-    NBX_LAUNCHED("bitonic_chunk_full");
-    for (int64_t k = 2 * kSortChunk; k <= N; k <<= 1) {
-        int64_t j = k >> 1;
-        for (; j >= 2 * kSortChunk; j >>= 2) {
-            k_bitonic_global2<<<blocks_for(N / 4, 256), 256, 0, s>>>(keys, N, k, j >> 1);
-            NBX_LAUNCHED("bitonic_global2");
+    __syncthreads();
+    for (int c = t; c < count; c += 256) {
+        const int at = list[c], li = at / kTileCols, l = at % kTileCols, up = at - kTileCols;
+        if (own[at] < 0) continue;
+        // with the point above set, the other neighbours are linked to it by
+        // their own links; likewise the upper left one to the left one
+        if (li > 0 && own[up] >= 0) {
+            tile_unite(own, at, up);
+            continue;
         }
-        if (j == kSortChunk) {
-            k_bitonic_global<<<blocks_for(N / 2, 256), 256, 0, s>>>(keys, N, k, j);
-            NBX_LAUNCHED("bitonic_global");
-        }
-        k_bitonic_chunk_tail<<<chunks, kSortThreads, 0, s>>>(keys, k);
-        NBX_LAUNCHED("bitonic_chunk_tail");
+        if (l > 0 && own[at - 1] >= 0) tile_unite(own, at, at - 1);
+        else if (li > 0 && l > 0 && own[up - 1] >= 0) tile_unite(own, at, up - 1);
+        if (li > 0 && l < kTileCols - 1 && own[up + 1] >= 0) tile_unite(own, at, up + 1);
     }
-    return 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+        const int li = threadIdx.y + 4 * q, at = li * kTileCols + lj;
+        if (i0 + li >= nx || j >= ny) continue;
+        int32_t r = -1;
+        if (own[at] >= 0) {
+            const int a = tile_root(own, at);
+            r = (i0 + a / kTileCols) * ny + j0 + a % kTileCols;
+        }
+        par[static_cast<int64_t>(i0 + li) * ny + j] = r;
+    }
+}
+
+// Links across the tiles' borders: thread t < rows * ny is a point of a tile's
+// first row against the row above, the others are a row's pair across a border
+// between tile columns.
+__global__ __launch_bounds__(256) void k_border_union(int nx, int ny, int rows, int cols,
+                                                      int32_t* par) {
+    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    const int64_t across = static_cast<int64_t>(rows) * ny;
+    if (t < across) {
+        const int i = (static_cast<int>(t / ny) + 1) * kTileRows, j = static_cast<int>(t % ny);
+        const int32_t k = i * ny + j, up = k - ny;
+        if (uf_load(par + k) < 0) return;
+        if (uf_load(par + up) >= 0) {
+            uf_unite(par, k, up);
+            return;
+        }
+        if (j > 0 && uf_load(par + up - 1) >= 0) uf_unite(par, k, up - 1);
+        if (j + 1 < ny && uf_load(par + up + 1) >= 0) uf_unite(par, k, up + 1);
+        return;
+    }
+    const int64_t u = t - across;
+    if (u >= static_cast<int64_t>(cols) * nx) return;
+    const int i = static_cast<int>(u / cols), j = (static_cast<int>(u % cols) + 1) * kTileCols;
+    const int32_t k = i * ny + j;
+    const bool right = uf_load(par + k) >= 0, left = uf_load(par + k - 1) >= 0;
+    if (right && left) {
+        uf_unite(par, k, k - 1);
+    } else if (i > 0) {
+        if (right && uf_load(par + k - ny - 1) >= 0) uf_unite(par, k, k - ny - 1);
+        if (left && uf_load(par + k - ny) >= 0) uf_unite(par, k - 1, k - ny);
+    }
+}
+
+// Path flattening, and per kScanTile points the numbers of (ridge points,
+// roots).
+__global__ __launch_bounds__(kScanThreads) void k_flatten_count(int64_t n, int32_t* par,
+                                                                I2* __restrict__ sums) {
+    __shared__ I2 sh[kScanThreads / 64];
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x;
+    I2 c{0, 0};
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+        const int64_t k = base + q * kScanThreads;
+        const int32_t p = k < n ? uf_load(par + k) : -1;
+        if (p < 0) continue;
+        const int32_t r = uf_root(par, p);
+        if (r != p) __hip_atomic_store(par + k, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        c += I2{1, r == k ? 1 : 0};
+    }
+    I2 total;
+    block_exclusive_scan(c, sh, &total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// Ridge points in raveled order, and each root's number: components are
+// numbered by root, i.e. by first pixel.
+__global__ __launch_bounds__(kScanThreads) void k_compact_roots(
+    const int32_t* __restrict__ par, int64_t n, const I2* __restrict__ tile_off,
+    int32_t* __restrict__ idx, int32_t* __restrict__ number) {
+    __shared__ I2 sh[kScanThreads / 64];
+    const int64_t base =
+        static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
+    int32_t p[kScanItems];
+    I2 c{0, 0}, total;
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+        p[q] = base + q < n ? par[base + q] : -1;
+        c += I2{p[q] >= 0 ? 1 : 0, p[q] == base + q ? 1 : 0};
+    }
+    I2 at = block_exclusive_scan(c, sh, &total);
+    if (total.a == 0) return;
+    at += tile_off[blockIdx.x];
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+        if (p[q] < 0) continue;
+        idx[at.a++] = static_cast<int32_t>(base + q);
+        if (p[q] == base + q) number[base + q] = at.b++;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Stable radix sort of the ridge points by component number.  They come in
+// raveled order, so after it each component's points are together and in that
+// order.  A block takes kRadixTile points; a pass counts its digits (counts
+// [digit][block]), scans the counts, and moves the points: each wavefront its
+// own quarter, 64 at a time, a point's rank among the equal digits of its row
+// from ballots.  Two passes cover 4 M components: 37 us at a capacity of 800,000
+// points, and 19 us for the counts' scans (a bitonic sort of 2^20 64-bit keys
+// took 280 us).  A tile of 4096 points leaves CUs idle (63 us), one of 512
+// doubles the counts to scan.
+constexpr int kRadixTile = 1024, kRadixBits = 11, kRadixWaves = kScanThreads / 64;
+
+// FIRST: the numbers come from the labelling and are stored to comp
+template <bool FIRST>
+__global__ __launch_bounds__(kScanThreads) void k_radix_count(
+    const int32_t* __restrict__ idx, const int32_t* __restrict__ par,
+    const int32_t* __restrict__ number, const I2* __restrict__ total, int64_t m, int shift,
+    int bits, int32_t* __restrict__ comp, int32_t* __restrict__ counts) {
+    __shared__ int32_t h[1 << kRadixBits];
+    const int bins = 1 << bits;
+    for (int b = threadIdx.x; b < bins; b += kScanThreads) h[b] = 0;
+    __syncthreads();
+    const int64_t count = total->a < m ? total->a : m;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kRadixTile;
+    for (int64_t t = base + threadIdx.x; t < base + kRadixTile && t < count; t += kScanThreads) {
+        const int32_t c = FIRST ? number[par[idx[t]]] : comp[t];
+        if (FIRST) comp[t] = c;
+        atomicAdd(&h[(c >> shift) & (bins - 1)], 1);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < bins; b += kScanThreads)
+        counts[static_cast<int64_t>(b) * gridDim.x + blockIdx.x] = h[b];
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_radix_move(
+    const int32_t* __restrict__ idx, const int32_t* __restrict__ comp,
+    const I2* __restrict__ total, int64_t m, int shift, int bits,
+    const int32_t* __restrict__ starts, const int32_t* __restrict__ start_tile,
+    int32_t* __restrict__ idx_out, int32_t* __restrict__ comp_out) {
+    __shared__ int32_t next[kRadixWaves][1 << kRadixBits];
+    const int64_t count = total->a < m ? total->a : m;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kRadixTile;
+    if (first >= count) return;
+    const int bins = 1 << bits, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int b = threadIdx.x; b < bins; b += kScanThreads)
+#pragma unroll
+        for (int q = 0; q < kRadixWaves; ++q) next[q][b] = 0;
+    __syncthreads();
+    constexpr int kQuarter = kRadixTile / kRadixWaves;
+    const int64_t base = first + w * kQuarter;
+    for (int r = 0; r < kQuarter; r += 64) {
+        const int64_t t = base + r + lane;
+        if (t < count) atomicAdd(&next[w][(comp[t] >> shift) & (bins - 1)], 1);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < bins; b += kScanThreads) {
+        const int64_t at = static_cast<int64_t>(b) * gridDim.x + blockIdx.x;
+        int32_t run = starts[at] + start_tile[at / kScanTile];
+#pragma unroll
+        for (int q = 0; q < kRadixWaves; ++q) {
+            const int32_t c = next[q][b];
+            next[q][b] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    for (int r = 0; r < kQuarter && base + r < count; r += 64) {
+        const int64_t t = base + r + lane;
+        const bool in = t < count;
+        const int32_t c = in ? comp[t] : 0, k = in ? idx[t] : 0;
+        const int d = (c >> shift) & (bins - 1);
+        uint64_t same = __ballot(in);
+        for (int q = 0; q < bits; ++q) {
+            const uint64_t set = __ballot(d >> q & 1);
+            same &= d >> q & 1 ? set : ~set;
+        }
+        const int rank = __popcll(same & ((1ull << lane) - 1));
+        if (in) {
+            const int32_t to = next[w][d] + rank;
+            idx_out[to] = k;
+            comp_out[to] = c;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (in && rank == 0) next[w][d] += static_cast<int32_t>(__popcll(same));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
 }
 
 __global__ void k_offsets_zero(int64_t* __restrict__ offsets) { offsets[0] = 0; }
 
-__global__ void k_make_keys(const int32_t* __restrict__ idx, const int32_t* __restrict__ par,
-                            const int32_t* __restrict__ count_dev, int64_t N,
-                            unsigned long long* __restrict__ keys) {
+// seg_first[c] = position of component c's first point in the sorted list;
+// seg_first[nseg] = its length
+__global__ void k_seg_first(const int32_t* __restrict__ comp, const I2* __restrict__ total,
+                            int64_t cap, int32_t* __restrict__ seg_first) {
     const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= N) return;
-    const int32_t cnt = *count_dev;
-    if (t < cnt) {
-        const int32_t k = idx[t];
-        keys[t] = (static_cast<unsigned long long>(static_cast<uint32_t>(par[k])) << 32) |
-                  static_cast<uint32_t>(k);
-    } else {
-        keys[t] = ~0ull;
-    }
-}
-
-// seg_start[t] = 1 where a new component begins in the sorted keys
-__global__ void k_seg_start(const unsigned long long* __restrict__ keys,
-                            const int32_t* __restrict__ count_dev, int64_t cap,
-                            int32_t* __restrict__ seg_start) {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= cap) return;
-    const int32_t cnt = *count_dev;
-    int32_t v = 0;
-    if (t < cnt) v = (t == 0 || (keys[t] >> 32) != (keys[t - 1] >> 32)) ? 1 : 0;
-    seg_start[t] = v;
-}
-
-// seg_first[s] = position of the first key of segment s; seg_first[nseg] = cnt
-// seg_ex/seg_tile: the tiled exclusive scan of seg_start
-__global__ void k_seg_first(const int32_t* __restrict__ seg_start,
-                            const int32_t* __restrict__ seg_ex,
-                            const int32_t* __restrict__ seg_tile,
-                            const int32_t* __restrict__ count_dev,
-                            const int32_t* __restrict__ nseg_dev, int64_t cap,
-                            int32_t* __restrict__ seg_first) {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t < cap && t < *count_dev && seg_start[t])
-        seg_first[seg_ex[t] + seg_tile[t / kScanTile]] = static_cast<int32_t>(t);
-    if (t == 0) seg_first[*nseg_dev] = *count_dev;
+    if (t < cap && t < total->a && (t == 0 || comp[t] != comp[t - 1]))
+        seg_first[comp[t]] = static_cast<int32_t>(t);
+    if (t == 0) seg_first[total->b] = total->a;
 }
 
 // kept ridge sizes: len or 0
-__global__ void k_seg_keep(const int32_t* __restrict__ seg_first, const int32_t* __restrict__ nseg_dev,
+__global__ void k_seg_keep(const int32_t* __restrict__ seg_first, const I2* __restrict__ total,
                            int64_t cap, int min_pts, I2* __restrict__ kept) {
     const int64_t s = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (s >= cap) return;
     int32_t len = 0;
-    if (s < *nseg_dev) len = seg_first[s + 1] - seg_first[s];
+    if (s < total->b) len = seg_first[s + 1] - seg_first[s];
     const bool keep = len >= min_pts && len > 0;
     kept[s] = I2{keep ? len : 0, keep ? 1 : 0};
 }
 
-__global__ void k_group_scatter(const unsigned long long* __restrict__ keys,
-                                const int32_t* __restrict__ seg_start,
-                                const int32_t* __restrict__ seg_ex,
-                                const int32_t* __restrict__ seg_tile,
+__global__ void k_group_scatter(const int32_t* __restrict__ idx, const int32_t* __restrict__ comp,
                                 const int32_t* __restrict__ seg_first,
                                 const I2* __restrict__ kept,
                                 const I2* __restrict__ out_off_idx,
                                 const I2* __restrict__ out_tile,
                                 const I2* __restrict__ totals,
                                 const double2* __restrict__ pts_dense,
-                                const int32_t* __restrict__ count_dev, int64_t cap,
+                                const I2* __restrict__ all, int64_t cap,
                                 double2* __restrict__ pts_out, int64_t* __restrict__ offsets) {
     const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (t == 0) {
         const I2 tot = *totals;  // (points kept, ridges kept)
         offsets[tot.b] = tot.a;
     }
-    if (t >= cap || t >= *count_dev) return;
-    // segment of t: inclusive count of starts up to t, minus one
-    const int32_t s = seg_ex[t] + seg_tile[t / kScanTile] + seg_start[t] - 1;
+    if (t >= cap || t >= all->a) return;
+    const int32_t s = comp[t];
     if (!kept[s].b) return;
     const I2 o = out_off_idx[s] + out_tile[s / kScanTile];  // output offset, ridge number
-    const int32_t k = static_cast<int32_t>(keys[t] & 0xffffffffull);
     const int32_t r = o.a + (static_cast<int32_t>(t) - seg_first[s]);
-    pts_out[r] = pts_dense[k];
+    pts_out[r] = pts_dense[idx[t]];
     if (t == seg_first[s]) offsets[o.b] = o.a;
 }
 
@@ -704,22 +952,30 @@ int read_counts(const int32_t* dev, int count, int32_t* host, hipStream_t s) {
     return 0;
 }
 
-// Ridge predicate + optional percentile; leaves flag/pts_dense in the arena.
+// The percentile threshold, left at st->result (fmin_dev set to it); without
+// one fmin_dev is NULL.
+int ridge_threshold(const double* f, int64_t n, double percentile, SelState* st,
+                    unsigned long long* held, const double** fmin_dev, hipStream_t s) {
+    *fmin_dev = nullptr;
+    if (percentile == 0) return 0;
+    *fmin_dev = &st->result;
+    return percentile_device(f, n, percentile, st, held, nullptr, s);
+}
+
+// Optional percentile + ridge predicate into flag and pts_dense (which holds
+// the percentile's key list until then).
 int run_predicate(const double* f, const double* evec, const double* x, const double* y, int nx,
                   int ny, double dx, double dy, double sdd_thresh, double percentile,
                   SelState* st, int32_t* flag, double2* pts_dense, hipStream_t s,
-                  double* sdd = nullptr, int32_t* uf_par = nullptr) {
-    const int64_t n = static_cast<int64_t>(nx) * ny;
-    const double* fmin_dev = nullptr;
-    if (percentile != 0) {
-        int rc = percentile_device(f, n, percentile, st, nullptr, s);
-        if (rc) return rc;
-        fmin_dev = &st->result;
-    }
+                  double* sdd = nullptr) {
+    const double* fmin_dev;
+    if (int rc = ridge_threshold(f, static_cast<int64_t>(nx) * ny, percentile, st,
+                                 reinterpret_cast<unsigned long long*>(pts_dense), &fmin_dev, s))
+        return rc;
     const dim3 block(64, 4), grid((ny + 63) / 64, (nx + 3) / 4);
     k_ridge_predicate<<<grid, block, 0, s>>>(f, reinterpret_cast<const double2*>(evec), x, y, nx,
                                              ny, dx, dy, sdd_thresh, fmin_dev, flag, pts_dense,
-                                             sdd, uf_par);
+                                             sdd);
     NBX_LAUNCHED("ridge_predicate");
     return 0;
 }
@@ -774,34 +1030,43 @@ int scratch_address(char** out) {
 // Scratch layout of the grouped-ridge pipeline for n grid points.
 struct RidgeLayout {
     SelState* st;
-    // total[0..1] = the pair scan's (points, ridges) total, total[2] = count,
-    // the number of ridge points: one read-back fetches all three
-    int32_t *flag, *pos, *tmp, *count, *par, *idx, *seg_start, *seg_ex, *seg_first, *nseg,
-        *total;
+    int32_t *par, *number, *idx[2], *comp[2], *seg_first, *tmp, *counts;
+    // total[0..1] = the pair scan's (points, ridges) total, total[2..3] = (ridge
+    // points, components): one read-back fetches the first three
+    int32_t* total;
     I2 *kept, *out_off_idx, *tmp2;
     double2* dense;
-    unsigned long long* keys;
     void carve(Arena& A, int64_t n) {
         const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-        int64_t N = kSortChunk;
-        while (N < n) N <<= 1;
         st = A.take<SelState>(1);
-        flag = A.take<int32_t>(n);
-        pos = A.take<int32_t>(n);
-        dense = A.take<double2>(n);
-        tmp = A.take<int32_t>(tiles + 1);   // tile offsets: compaction, then segments
-        tmp2 = A.take<I2>(tiles + 1);       // tile offsets of the pair scan
+        dense = A.take<double2>(n);  // first the percentile's key list
         par = A.take<int32_t>(n);
-        idx = A.take<int32_t>(n);
-        keys = A.take<unsigned long long>(N);
-        seg_start = A.take<int32_t>(n);
-        seg_ex = A.take<int32_t>(n);
+        number = A.take<int32_t>(n);  // component number, at its root
+        for (int q = 0; q < 2; ++q) {
+            idx[q] = A.take<int32_t>(n);  // ridge points and their components, in turn
+            comp[q] = A.take<int32_t>(n);
+        }
         seg_first = A.take<int32_t>(n + 1);
-        kept = A.take<I2>(n);         // (kept length, kept flag) per segment
+        kept = A.take<I2>(n);         // (kept length, kept flag) per component
         out_off_idx = A.take<I2>(n);  // their exclusive scans
-        nseg = A.take<int32_t>(1);
-        total = A.take<int32_t>(3);
-        count = total + 2;
+        tmp2 = A.take<I2>(tiles + 1);  // tile offsets of the pair scans
+        // digit counts (scanned in place) and their tile offsets
+        const int64_t digits = radix_counts(n);
+        counts = A.take<int32_t>(digits);
+        tmp = A.take<int32_t>((digits + kScanTile - 1) / kScanTile + 1);
+        total = A.take<int32_t>(4);
+    }
+    // passes and bits a pass for component numbers below m
+    static int radix_passes(int64_t m, int* bits) {
+        int width = 1;
+        while ((static_cast<int64_t>(1) << width) < m) ++width;
+        const int passes = (width + kRadixBits - 1) / kRadixBits;
+        *bits = (width + passes - 1) / passes;
+        return passes;
+    }
+    static int64_t radix_counts(int64_t m) {
+        // (the widest digit: a smaller m may take more bits a pass than n does)
+        return (static_cast<int64_t>(1) << kRadixBits) * ((m + kRadixTile - 1) / kRadixTile);
     }
     static size_t bytes(int64_t n) {
         RidgeLayout L;
@@ -810,6 +1075,19 @@ struct RidgeLayout {
         return measure.used;
     }
 };
+
+// What a grid of n points counts against the fixed scratch: 60 bytes a point
+// and 8 of the power of two that holds them, the stated limit of about 980,000
+// points.  It covers RidgeLayout::bytes (68 bytes a point and 60 KB) wherever
+// that could pass 64 MiB: the power of two is well above 980,000 there.
+size_t noalloc_need(int64_t n) {
+    const size_t p = static_cast<size_t>(n), tiles = (p + kScanTile - 1) / kScanTile;
+    size_t pow2 = 1024;
+    while (pow2 < p) pow2 <<= 1;
+    return 6400 + 6 * align256(4 * p) + align256(16 * p) +
+           align256(4 * (tiles + 1)) + align256(8 * (tiles + 1)) + align256(8 * pow2) +
+           align256(4 * (p + 1)) + 2 * align256(8 * p) + 512;
+}
 
 // Count read-back without the pinned staging buffer (for callers that must
 // not allocate): a copy into pageable host memory, then a wait.
@@ -858,27 +1136,32 @@ int ridges_run(const double* f, const double* evec, const double* x, int nx, con
     RidgeLayout L;
     Arena A{arena, 0};
     L.carve(A, n);
-    SelState* st = L.st;
-    int32_t *flag = L.flag, *pos = L.pos, *tmp = L.tmp, *count = L.count, *par = L.par,
-            *idx = L.idx, *seg_start = L.seg_start, *seg_ex = L.seg_ex,
-            *seg_first = L.seg_first, *nseg = L.nseg, *total = L.total;
-    double2* dense = L.dense;
-    unsigned long long* keys = L.keys;
-
-    if (int rc = run_predicate(f, evec, x, y, nx, ny, dx, dy, sdd_thresh, percentile, st, flag,
-                               dense, s, nullptr, par))
+    int32_t *par = L.par, *total = L.total;
+    I2* const all = reinterpret_cast<I2*>(total + 2);
+    const double* fmin_dev;
+    if (int rc = ridge_threshold(f, n, percentile, L.st,
+                                 reinterpret_cast<unsigned long long*>(L.dense), &fmin_dev, s))
         return rc;
-    // label components (the predicate started the union-find)
-    const unsigned nb = blocks_for(n, 256);
-    const dim3 block(64, 4), grid((ny + 63) / 64, (nx + 3) / 4);
-    k_uf_union<<<grid, block, 0, s>>>(flag, nx, ny, par);
-    NBX_LAUNCHED("uf_union");
-    k_uf_flatten<<<nb, 256, 0, s>>>(flag, n, par);
-    NBX_LAUNCHED("uf_flatten");
-    // compact ridge points (raveled order)
-    if (int rc = exclusive_scan_tiled(flag, n, pos, tmp, count, s)) return rc;
-    k_compact<<<nb, 256, 0, s>>>(flag, pos, dense, n, nullptr, idx, tmp);
-    NBX_LAUNCHED("compact");
+    // ridge points and their components
+    const int rows = (nx - 1) / kTileRows, cols = (ny - 1) / kTileCols;  // borders between tiles
+    k_ridge_label<<<dim3(cols + 1, rows + 1), dim3(kTileCols, 4), 0, s>>>(
+        f, reinterpret_cast<const double2*>(evec), x, y, nx, ny, dx, dy, sdd_thresh, fmin_dev,
+        L.dense, par);
+    NBX_LAUNCHED("ridge_label");
+    const int64_t border = static_cast<int64_t>(rows) * ny + static_cast<int64_t>(cols) * nx;
+    if (border > 0) {
+        k_border_union<<<blocks_for(border, 256), 256, 0, s>>>(nx, ny, rows, cols, par);
+        NBX_LAUNCHED("border_union");
+    }
+    // compact ridge points (raveled order) and number the components
+    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    k_flatten_count<<<static_cast<unsigned>(tiles), kScanThreads, 0, s>>>(n, par, L.tmp2);
+    NBX_LAUNCHED("flatten_count");
+    k_scan_sums<<<1, kScanThreads, 0, s>>>(L.tmp2, tiles, all);
+    NBX_LAUNCHED("scan_sums");
+    k_compact_roots<<<static_cast<unsigned>(tiles), kScanThreads, 0, s>>>(par, n, L.tmp2, L.idx[0],
+                                                                         L.number);
+    NBX_LAUNCHED("compact_roots");
     // The grouping stage works on the ridge points only (typically a few
     // percent of the grid), sized by a bound on their count; its kernels read
     // the exact count on the device.  With a percentile threshold q the bound
@@ -896,7 +1179,7 @@ int ridges_run(const double* f, const double* evec, const double* x, int nx, con
         m = n;
     } else {
         int32_t cnt = 0;
-        if (int rc = read(count, 1, &cnt)) return rc;
+        if (int rc = read(&all->a, 1, &cnt)) return rc;
         m = cnt;
     }
     if (m == 0) {
@@ -911,29 +1194,38 @@ int ridges_run(const double* f, const double* evec, const double* x, int nx, con
         NBX_HIP(hipStreamSynchronize(s));
         return 0;
     }
-    int64_t Ns = kSortChunk;
-    while (Ns < m) Ns <<= 1;
     const unsigned nbm = blocks_for(m, 256);
-    // order by (component root, raveled index)
-    k_make_keys<<<blocks_for(Ns, 256), 256, 0, s>>>(idx, par, count, Ns, keys);
-    NBX_LAUNCHED("make_keys");
-    if (int rc = bitonic_sort(keys, Ns, s)) return rc;
+    // order by (component, raveled index)
+    int bits = 0;
+    const int passes = RidgeLayout::radix_passes(m, &bits);
+    const int64_t radix_blocks = (m + kRadixTile - 1) / kRadixTile;
+    const unsigned rb = static_cast<unsigned>(radix_blocks);
+    for (int q = 0; q < passes; ++q) {
+        int32_t *idx = L.idx[q & 1], *comp = L.comp[q & 1];
+        auto* count = q == 0 ? &k_radix_count<true> : &k_radix_count<false>;
+        count<<<rb, kScanThreads, 0, s>>>(idx, par, L.number, all, m, q * bits, bits, comp,
+                                          L.counts);
+        NBX_LAUNCHED("radix_count");
+        if (int rc = exclusive_scan_tiled(L.counts, radix_blocks << bits, L.counts, L.tmp,
+                                          total, s))
+            return rc;
+        k_radix_move<<<rb, kScanThreads, 0, s>>>(idx, comp, all, m, q * bits, bits, L.counts,
+                                                 L.tmp, L.idx[~q & 1], L.comp[~q & 1]);
+        NBX_LAUNCHED("radix_move");
+    }
+    const int32_t *idx = L.idx[passes & 1], *comp = L.comp[passes & 1];
     // segments = components
-    k_seg_start<<<nbm, 256, 0, s>>>(keys, count, m, seg_start);
-    NBX_LAUNCHED("seg_start");
-    if (int rc = exclusive_scan_tiled(seg_start, m, seg_ex, tmp, nseg, s)) return rc;
-    k_seg_first<<<nbm, 256, 0, s>>>(seg_start, seg_ex, tmp, count, nseg, m, seg_first);
+    k_seg_first<<<nbm, 256, 0, s>>>(comp, all, m, L.seg_first);
     NBX_LAUNCHED("seg_first");
-    k_seg_keep<<<nbm, 256, 0, s>>>(seg_first, nseg, m, min_ridge_pts, L.kept);
+    k_seg_keep<<<nbm, 256, 0, s>>>(L.seg_first, all, m, min_ridge_pts, L.kept);
     NBX_LAUNCHED("seg_keep");
     // total and nridges are adjacent: the pair scan's total lands in both
     I2* totals = reinterpret_cast<I2*>(total);
     if (int rc = exclusive_scan_tiled(L.kept, m, L.out_off_idx, L.tmp2, totals, s)) return rc;
-    // the segment scan's tile offsets (tmp) are still intact: the pair scan
-    // used tmp2; the scatter also writes offsets[nridges] = total
-    k_group_scatter<<<nbm, 256, 0, s>>>(keys, seg_start, seg_ex, tmp, seg_first, L.kept,
-                                        L.out_off_idx, L.tmp2, totals, dense, count, m,
-                                        reinterpret_cast<double2*>(pts), offsets);
+    // the scatter also writes offsets[nridges] = total
+    k_group_scatter<<<nbm, 256, 0, s>>>(idx, comp, L.seg_first, L.kept, L.out_off_idx, L.tmp2,
+                                        totals, L.dense, all, m, reinterpret_cast<double2*>(pts),
+                                        offsets);
     NBX_LAUNCHED("group_scatter");
     if (counts_dev) {
         k_counts_out<<<1, 64, 0, s>>>(total, m, 1, counts_dev);
@@ -961,9 +1253,12 @@ extern "C" {
 int nbx_percentile(const double* f, int64_t n, double q, double* result, nbx_stream stream) {
     NBX_REQUIRE(f != nullptr && result != nullptr, "NULL array");
     hipStream_t s = as_stream(stream);
-    Workspace ws(s, 2, sizeof(SelState));
+    const int64_t held = n < 0 ? 0 : n < kSelHeld ? n : kSelHeld;
+    Workspace ws(s, 2, align256(sizeof(SelState)) + 8 * held);
     if (ws.error()) return ws.error();
-    return percentile_device(f, n, q, reinterpret_cast<SelState*>(ws.get()), result, s);
+    Arena A{ws.get(), 0};
+    auto* st = A.take<SelState>(1);
+    return percentile_device(f, n, q, st, A.take<unsigned long long>(held), result, s);
 }
 
 int nbx_ridge_pts(const double* f, const double* evec, const double* x, int nx, const double* y,
@@ -993,7 +1288,7 @@ int nbx_ridge_pts(const double* f, const double* evec, const double* x, int nx, 
         return rc;
     if (int rc = exclusive_scan(flag, n, pos, tmp, total, s)) return rc;
     k_compact<<<blocks_for(n, 256), 256, 0, s>>>(flag, pos, dense, n,
-                                                 reinterpret_cast<double2*>(pts), nullptr, nullptr);
+                                                 reinterpret_cast<double2*>(pts));
     NBX_LAUNCHED("compact");
     int32_t cnt = 0;
     if (int rc = read_counts(total, 1, &cnt, s)) return rc;
@@ -1051,7 +1346,7 @@ int nbx_ridges_noalloc(const double* f, const double* evec, const double* x, int
     *npts_host = 0;
     if (n == 0) return 0;
     NBX_REQUIRE(f && evec && x && y && pts && offsets, "NULL array");
-    const size_t need = RidgeLayout::bytes(n);
+    const size_t need = noalloc_need(n);
     if (need > kNoAllocScratchBytes) {
         set_error("nbx_ridges_noalloc: a grid of " + std::to_string(n) + " points needs " +
                   std::to_string(need) + " bytes of scratch, above its fixed " +

@@ -150,3 +150,65 @@ def test_fused_inference_where_rounding_is_undecided(n, kind):
     a, b = net.predict_device(inp), net.predict_device_unfused(inp)
     assert torch.equal(torch.isnan(a), torch.isnan(b))
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+@pytest.mark.parametrize("kind", ["constant", "low bits", "two values", "infinite", "wide"])
+@pytest.mark.parametrize("n", [1, 2, 2049, 65536, 65537, 300001])
+def test_percentile_key_list(n, kind):
+    """The percentile's list of keys that share the leading 22 bits: short,
+    exactly full, and overflowing (all keys equal there, decided by the low
+    digits over the whole array).  Exact: order statistics and numpy's lerp,
+    which the device rounds once per step (fused multiply-add)."""
+    from fractions import Fraction
+
+    from numbacs_amd import _lib
+
+    def reference(f, q):
+        vi = (n - 1) * (q / 100.0)
+        lo = min(int(vi), n - 1)
+        part = np.sort(f)
+        a, b, g = float(part[lo]), float(part[min(lo + 1, n - 1)]), vi - int(vi)
+        if not (np.isfinite(a) and np.isfinite(b)):
+            with np.errstate(invalid="ignore"):
+                return np.percentile(f, q)
+        d = Fraction(b - a)
+        return float(Fraction(b) - d * Fraction(1 - g) if g >= 0.5 else Fraction(a) + d * Fraction(g))
+
+    rng = np.random.default_rng(n)
+    f = {"constant": lambda: np.full(n, -0.25),
+         "low bits": lambda: 1.0 + rng.integers(0, 1 << 30, n) * 2.0 ** -52,
+         "two values": lambda: rng.choice([1.0, 1.0 + 2.0 ** -52], n),
+         "infinite": lambda: rng.choice([-np.inf, -1.0, 0.0, -0.0, 5e-324], n),
+         "wide": lambda: rng.standard_normal(n) * 10.0 ** rng.integers(-300, 300, n)}[kind]()
+    fd, out = _lib.to_dev(f), _lib.empty((1,))
+    for q in (0.0, 37.3, 50.0, 90.0, 100.0):
+        _lib.check(_lib.load().nbx_percentile(_lib.ptr(fd), n, q, _lib.ptr(out),
+                                              _lib.stream_ptr()))
+        got = _lib.to_host(out)[0]
+        ref = reference(f, q)
+        assert got == ref or (np.isnan(got) and np.isnan(ref))
+
+
+@pytest.mark.parametrize("shape", [(5, 5), (16, 64), (17, 65), (16, 200), (300, 64), (33, 129),
+                                   (130, 257)])
+@pytest.mark.parametrize("gaps", [0.0, 0.3, 0.6])
+def test_ridge_components_across_tiles(shape, gaps):
+    """Half the grid is ridge points that touch diagonally (every second point
+    of a checkerboard), with gaps: one component over all tiles, many that
+    cross their borders, thousands of single points.  Equal to the oracle."""
+    from numbacs_amd.extraction import ftle_ridges
+
+    nx, ny = shape
+    rng = np.random.default_rng(nx * ny)
+    x, y = np.arange(nx) / 8.0, np.arange(ny) / 8.0
+    i, j = np.indices(shape)
+    f = 1.0 + 0.5 * (-1.0) ** (i + j) + 0.01 * rng.random(shape)
+    f[rng.random(shape) < gaps] = 0.0
+    ev = np.zeros(shape + (2,))
+    ev[..., 0] = 1.0
+    for least, q in ((1, 0), (3, 0), (1, 60)):
+        got = ftle_ridges(f, ev, x, y, percentile=q, min_ridge_pts=least)
+        ref = oracle.ridges(f, ev, x, y, percentile_=q, min_ridge_pts=least)
+        assert len(got) == len(ref)
+        for a, b in zip(got, ref):
+            assert np.array_equal(a, b)
