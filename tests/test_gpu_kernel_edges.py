@@ -212,3 +212,72 @@ def test_ridge_components_across_tiles(shape, gaps):
         assert len(got) == len(ref)
         for a, b in zip(got, ref):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (128, 64, 96), (64, 192, 128), (192, 128, 160),
+                                   (64, 64, 288)])
+def test_gemm_turns(M, N, K):
+    """All four forms of the GEMM where its turns of 128 k end: one slab of 32,
+    remainders of one to three slabs, several turns.  FP32 results: each is a sum
+    of K products of bf16 values (exact in float) rounded K times, so within
+    K ulps of the sum of magnitudes; the bf16 outputs within one bf16 ulp more."""
+    import torch
+    from numbacs_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(M + N + K)
+
+    def bf16(*shape):
+        return torch.tensor(rng.standard_normal(shape), dtype=torch.bfloat16, device="cuda")
+
+    def run(mode, A, B, c32=None, c16=None, bias=None, pre=None):
+        ptr = lambda v: None if v is None else _lib.ptr(v)
+        _lib.check(lib.nbx_mlp_gemm(mode, ptr(A), ptr(B), M, N, K, ptr(c32), ptr(c16), ptr(bias),
+                                    ptr(pre), _lib.stream_ptr()))
+
+    def out(dtype):
+        return torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
+
+    d = lambda v: v.double().cpu()
+    eps = K * 2.0 ** -23
+    A, B, At, Bt = bf16(M, K), bf16(K, N), bf16(K, M), bf16(N, K)
+    bias = torch.tensor(rng.standard_normal(N), dtype=torch.float32, device="cuda")
+    pre = torch.tensor(rng.standard_normal((M, N)), dtype=torch.float32, device="cuda")
+
+    def inner(a):
+        return 0.7978845608028654 * (a + 0.044715 * a ** 3)
+
+    for mode, left, right in ((3, d(A), d(B)), (2, d(At).T, d(B))):
+        c = out(torch.float32)
+        run(mode, A if mode == 3 else At, B, c32=c)
+        assert ((d(c) - left @ right).abs() <= eps * (left.abs() @ right.abs())).all()
+    c, h = out(torch.float32), out(torch.bfloat16)
+    run(0, A, B, c32=c, c16=h, bias=bias)
+    ref = d(A) @ d(B) + d(bias)
+    assert ((d(c) - ref).abs() <= eps * (d(A).abs() @ d(B).abs() + d(bias).abs())).all()
+    g = 0.5 * d(c) * (1 + torch.tanh(inner(d(c))))
+    assert ((d(h) - g).abs() <= 2.0 ** -8 * g.abs() + 1e-6 * (1 + d(c).abs())).all()
+    h = out(torch.bfloat16)
+    run(1, A, Bt, c16=h, pre=pre)
+    dh, t = d(A) @ d(Bt).T, torch.tanh(inner(d(pre)))
+    slope = 0.5 * (1 + t) + 0.5 * d(pre) * (1 - t ** 2) * 0.7978845608028654 * (
+        1 + 3 * 0.044715 * d(pre) ** 2)
+    # two roundings to bf16, and eps of the product's magnitudes
+    err = (2.0 ** -7 * dh.abs() + 2 * eps * (d(A).abs() @ d(Bt).abs().T)) * slope.abs() + 1e-5 * dh.abs()
+    assert ((d(h) - dh * slope).abs() <= err).all()
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 127, 129, 1000])
+@pytest.mark.parametrize("width", [64, 256, 320])
+def test_column_sums_of_partial_groups(n, width):
+    """Column sums where a block's row groups are cut short or empty, and for
+    more columns than a group has threads; within n ulps of the magnitudes."""
+    import torch
+    from numbacs_amd import _lib
+
+    rng = np.random.default_rng(n + width)
+    da = torch.tensor(rng.standard_normal((n, width)), dtype=torch.bfloat16, device="cuda")
+    gb = torch.full((width,), float("nan"), dtype=torch.float32, device="cuda")
+    _lib.check(_lib.load().nbx_mlp_colsum(_lib.ptr(da), n, width, _lib.ptr(gb), _lib.stream_ptr()))
+    ref = da.double()
+    assert ((gb.double() - ref.sum(0)).abs() <= n * 2.0 ** -23 * ref.abs().sum(0)).all()
