@@ -374,6 +374,10 @@ int nbx_mlp_out_backward(const float* dy, const uint16_t* h, const float* pre, i
                          nbx_stream stream);
 /* gb (width) = column sums of da (n x width). */
 int nbx_mlp_colsum(const uint16_t* da, int64_t n, int width, float* gb, nbx_stream stream);
+/* A hidden layer's weight and bias gradients in two launches: gW (M x N) as
+ * nbx_mlp_gemm's mode 2 of h (K x M) and da (K x N), gb (N) = column sums of da. */
+int nbx_mlp_weight_grad(const uint16_t* h, const uint16_t* da, int M, int N, int K, float* gW,
+                        float* gb, nbx_stream stream);
 /* Adam (bias-corrected, decoupled weight decay) on fp32 master weights w;
  * w16 (nullable) receives the bf16 copy. */
 int nbx_mlp_adam(float* w, const float* g, float* m, float* v, uint16_t* w16, int64_t n,

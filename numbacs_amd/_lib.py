@@ -65,6 +65,7 @@ SIGNATURES = {
     "nbx_mlp_out_backward": (_c_i, [_c_p, _c_p, _c_p, _c_i64, _c_i, _c_p, _c_p, _c_p, _c_p,
                                     _c_p]),
     "nbx_mlp_colsum": (_c_i, [_c_p, _c_i64, _c_i, _c_p, _c_p]),
+    "nbx_mlp_weight_grad": (_c_i, [_c_p, _c_p, _c_i, _c_i, _c_i, _c_p, _c_p, _c_p]),
     "nbx_mlp_adam": (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, ctypes.c_float, ctypes.c_float,
                             ctypes.c_float, ctypes.c_float, _c_i, ctypes.c_float, _c_p]),
     "nbx_mlp_adam_sched": (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, ctypes.c_float,

@@ -129,6 +129,15 @@ struct TurnLoad {
             }
         }
     }
+    // !KC: sums[i] += the thread's rows 8 (t & 7) + i over its k
+    __device__ __forceinline__ void add_columns(float (&sums)[8], int ks) const {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (64 * (q >> 1) + 2 * static_cast<int>(threadIdx.x >> 3) + (q & 1) >= ks) continue;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sums[i] += bf2f(v[q][i]);
+        }
+    }
     __device__ __forceinline__ void store(uint16_t* __restrict__ tile) const {
         const int t = threadIdx.x;
 #pragma unroll
@@ -153,7 +162,7 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t* __restrict__ A, lo
                                               long ldc, uint16_t* __restrict__ C16, long ldc16,
                                               const float* __restrict__ bias,
                                               const float* __restrict__ pre, long ldp,
-                                              int ksplit) {
+                                              int ksplit, float* __restrict__ colsum) {
     static_assert(BM == 64 && BN == 64 && BK == 32, "a turn's loads are laid out for these");
     __shared__ __attribute__((aligned(16))) uint16_t As[BM * kTurn];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[BN * kTurn];
@@ -191,7 +200,12 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t* __restrict__ A, lo
                     slope[i][j][q] = pre[(m0 + 32 * wm + 16 * i + r16) * ldp + n0 + 32 * wn +
                                          16 * j + 4 * (lane >> 4) + q];
     }
+    // column sums of B by the blocks of the first row of tiles, from the
+    // registers that B passes through
+    constexpr bool kSums = !AK && !BKC;
+    float sums[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int k0 = kb; k0 < ke; k0 += kTurn) {
+        if (kSums && colsum && blockIdx.y == 0) lb.add_columns(sums, ke - k0);
         la.store(As);
         lb.store(Bs);
         __syncthreads();
@@ -219,6 +233,22 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t* __restrict__ A, lo
         __syncthreads();
     }
 
+    if (kSums && colsum && blockIdx.y == 0) {
+        // one addition a column and block, 64 neighbours in one instruction
+        // (additions to memory from each wavefront, eight apart, took 15 us more)
+        float* const part = reinterpret_cast<float*>(As);  // (read no more)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            float s = sums[i];
+            s += __shfl_xor(s, 8);
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (lane < 8) part[64 * w + 8 * lane + i] = s;
+        }
+        __syncthreads();
+        if (t < 64)
+            atomicAdd(&colsum[n0 + t], part[t] + part[64 + t] + part[128 + t] + part[192 + t]);
+    }
     const int rq = 4 * (lane >> 4);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -722,6 +752,32 @@ int check_gemm_shape(int M, int N, int K) {
     return 0;
 }
 
+// gW = A^T @ B with A stored (K x M), B stored (K x N); with gb also B's column
+// sums, which the product's blocks take on the way (8192 x 256: four launches of
+// 1.8 + 11.6 + 1.3 + 4.5 us apart from it, two of 1.9 + 10.4 us with it).
+void weight_grad(const uint16_t* A, const uint16_t* B, int M, int N, int K, float* gW, float* gb,
+                 hipStream_t s) {
+    // K is the batch: split it over blocks when the output has few tiles (a
+    // 256 x 256 weight is 16 tiles on 256 CUs), each block adding its partial
+    // tile into gW
+    const int tiles = (M / BM) * (N / BN);
+    const int64_t size = static_cast<int64_t>(M) * N;
+    int splits = 256 / tiles;
+    if (splits > K / 256) splits = K / 256;
+    if (splits <= 1) {
+        if (gb) k_fill_f32<<<blocks_for(N, 256), 256, 0, s>>>(gb, N, 0.f);
+        k_gemm<false, false, EPI_F32><<<dim3(N / BN, M / BM), 256, 0, s>>>(
+            A, 1, M, B, N, 1, M, N, K, gW, N, nullptr, 0, nullptr, nullptr, 0, K, gb);
+        return;
+    }
+    const int ksplit = (K / splits + BK - 1) / BK * BK;
+    const dim3 grid(N / BN, M / BM, (K + ksplit - 1) / ksplit);
+    k_fill2_f32<<<blocks_for(size + N, 256), 256, 0, s>>>(gW, size, gb, gb ? N : 0);
+    k_gemm<false, false, EPI_F32_ADD><<<grid, 256, 0, s>>>(A, 1, M, B, N, 1, M, N, K, gW, N,
+                                                           nullptr, 0, nullptr, nullptr, 0, ksplit,
+                                                           gb);
+}
+
 }  // namespace
 }  // namespace nbx
 
@@ -741,47 +797,38 @@ int nbx_mlp_gemm(int mode, const uint16_t* A, const uint16_t* B, int M, int N, i
             NBX_REQUIRE(C16 != nullptr && bias != nullptr, "forward needs C16 and bias");
             k_gemm<true, false, EPI_BIAS_GELU><<<grid, 256, 0, s>>>(A, K, 1, B, N, 1, M, N, K, C32,
                                                                     N, C16, N, bias, nullptr, 0,
-                                                                    K);
+                                                                    K, nullptr);
             break;
         case 1:  // backward data: C16 = bf16(bf16(A (MxK) @ B^T) * gelu'(pre)), B stored (N x K)
             NBX_REQUIRE(C16 != nullptr && pre != nullptr, "backward-data needs C16 and pre");
             k_gemm<true, true, EPI_GELU_GRAD><<<grid, 256, 0, s>>>(A, K, 1, B, 1, K, M, N, K,
                                                                    nullptr, 0, C16, N, nullptr,
-                                                                   pre, N, K);
+                                                                   pre, N, K, nullptr);
             break;
-        case 2: {  // backward weight: C32 = A^T @ B with A stored (K x M), B stored (K x N)
+        case 2:  // backward weight: C32 = A^T @ B with A stored (K x M), B stored (K x N)
             NBX_REQUIRE(C32 != nullptr, "backward-weight needs C32");
-            // K is the batch: split it over blocks when the output has few
-            // tiles (a 256 x 256 weight is 16 tiles on 256 CUs), each block
-            // adding its partial tile into C32
-            const int tiles = (M / BM) * (N / BN);
-            int splits = 256 / tiles;
-            if (splits > K / 256) splits = K / 256;
-            if (splits <= 1) {
-                k_gemm<false, false, EPI_F32><<<grid, 256, 0, s>>>(A, 1, M, B, N, 1, M, N, K, C32,
-                                                                   N, nullptr, 0, nullptr, nullptr,
-                                                                   0, K);
-            } else {
-                const int ksplit = (K / splits + BK - 1) / BK * BK;
-                const dim3 g3(N / BN, M / BM, (K + ksplit - 1) / ksplit);
-                k_fill_f32<<<blocks_for(static_cast<int64_t>(M) * N, 256), 256, 0, s>>>(
-                    C32, static_cast<int64_t>(M) * N, 0.f);
-                k_gemm<false, false, EPI_F32_ADD><<<g3, 256, 0, s>>>(A, 1, M, B, N, 1, M, N, K,
-                                                                     C32, N, nullptr, 0, nullptr,
-                                                                     nullptr, 0, ksplit);
-            }
+            weight_grad(A, B, M, N, K, C32, nullptr, s);
             break;
-        }
         case 3:  // plain: C32 = A (MxK) @ B (KxN)
             NBX_REQUIRE(C32 != nullptr, "plain GEMM needs C32");
             k_gemm<true, false, EPI_F32><<<grid, 256, 0, s>>>(A, K, 1, B, N, 1, M, N, K, C32, N,
-                                                              nullptr, 0, nullptr, nullptr, 0, K);
+                                                              nullptr, 0, nullptr, nullptr, 0, K,
+                                                              nullptr);
             break;
         default:
             set_error("unknown GEMM mode");
             return -2;
     }
     NBX_LAUNCHED("mlp_gemm");
+    return 0;
+}
+
+int nbx_mlp_weight_grad(const uint16_t* h, const uint16_t* da, int M, int N, int K, float* gW,
+                        float* gb, nbx_stream stream) {
+    if (int rc = check_gemm_shape(M, N, K)) return rc;
+    NBX_REQUIRE(h && da && gW && gb, "NULL array");
+    weight_grad(h, da, M, N, K, gW, gb, as_stream(stream));
+    NBX_LAUNCHED("mlp_weight_grad");
     return 0;
 }
 

@@ -113,10 +113,9 @@ class MLPSurrogate:
                                           _lib.ptr(gb[-1]), _lib.ptr(da), s))
         for l in range(self.layers - 1, -1, -1):
             K = self.F if l == 0 else self.width
-            # weight gradient: gW_l = h_l^T da_l  (K x width)
-            _lib.check(L.nbx_mlp_gemm(2, _lib.ptr(h[l]), _lib.ptr(da), K, self.width, n,
-                                      _lib.ptr(gW[l]), None, None, None, s))
-            _lib.check(L.nbx_mlp_colsum(_lib.ptr(da), n, self.width, _lib.ptr(gb[l]), s))
+            # gW_l = h_l^T da_l  (K x width), gb_l = column sums of da_l
+            _lib.check(L.nbx_mlp_weight_grad(_lib.ptr(h[l]), _lib.ptr(da), K, self.width, n,
+                                             _lib.ptr(gW[l]), _lib.ptr(gb[l]), s))
             if l > 0:
                 da_prev = t.empty((n, self.width), dtype=t.bfloat16, device=dev)
                 _lib.check(L.nbx_mlp_gemm(1, _lib.ptr(da), _lib.ptr(self.W16[l]), n, self.width,

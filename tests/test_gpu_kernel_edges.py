@@ -281,3 +281,25 @@ def test_column_sums_of_partial_groups(n, width):
     _lib.check(_lib.load().nbx_mlp_colsum(_lib.ptr(da), n, width, _lib.ptr(gb), _lib.stream_ptr()))
     ref = da.double()
     assert ((gb.double() - ref.sum(0)).abs() <= n * 2.0 ** -23 * ref.abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (64, 128, 224), (128, 64, 512), (64, 192, 1056),
+                                   (256, 256, 1024)])
+def test_weight_grad_with_column_sums(M, N, K):
+    """The fused weight and bias gradients, without and with a split batch and
+    with a last part that ends inside a turn; each within K ulps of the
+    magnitudes it sums."""
+    import torch
+    from numbacs_amd import _lib
+
+    rng = np.random.default_rng(M + N + K)
+    h, da = (torch.tensor(rng.standard_normal((K, w)), dtype=torch.bfloat16, device="cuda")
+             for w in (M, N))
+    gW = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    gb = torch.full((N,), float("nan"), dtype=torch.float32, device="cuda")
+    _lib.check(_lib.load().nbx_mlp_weight_grad(_lib.ptr(h), _lib.ptr(da), M, N, K, _lib.ptr(gW),
+                                               _lib.ptr(gb), _lib.stream_ptr()))
+    hd, dd = h.double().cpu(), da.double().cpu()
+    eps = K * 2.0 ** -23
+    assert ((gW.double().cpu() - hd.T @ dd).abs() <= eps * (hd.abs().T @ dd.abs())).all()
+    assert ((gb.double().cpu() - dd.sum(0)).abs() <= eps * dd.abs().sum(0)).all()
