@@ -294,7 +294,8 @@ __global__ void k_features(const float* __restrict__ inp, int64_t n, const float
                            uint16_t* __restrict__ h0) {
     const int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (idx >= n * half) return;
-    const int64_t r = idx / half;
+    // (a 64-bit division takes longer than the rest)
+    const int64_t r = idx >> 32 ? idx / half : static_cast<uint32_t>(idx) / static_cast<uint32_t>(half);
     const int c = static_cast<int>(idx - r * half);
     float z = 0.f;
 #pragma unroll
@@ -303,29 +304,55 @@ __global__ void k_features(const float* __restrict__ inp, int64_t n, const float
         z += u * Bf[d * half + c];
     }
     z *= 6.283185307179586f;
-    h0[r * 2 * half + c] = f2bf(sinf(z));
-    h0[r * 2 * half + half + c] = f2bf(cosf(z));
+    float sn, cs;
+    sincosf(z, &sn, &cs);
+    h0[r * 2 * half + c] = f2bf(sn);
+    h0[r * 2 * half + half + c] = f2bf(cs);
 }
 
-// y = h W_out + b_out for a 2-column output layer (one row per thread).
-__global__ void k_out_fwd(const uint16_t* __restrict__ h, int64_t n, int width,
-                          const uint16_t* __restrict__ W, const float* __restrict__ b,
-                          float* __restrict__ y) {
-    const int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (r >= n) return;
+// y = h W_out + b_out for a 2-column output layer: one row per thread, sums in
+// k order.  The rows come through LDS (64 x 256 bf16, chunks permuted by row), so
+// that the loads are whole lines, and the weights are floats there: read row by
+// row, 64 lines a load, 8192 x 256 took 9.8 us, now 7.7.
+constexpr int kOutThreads = 64, kOutChunk = 256;
+
+__global__ __launch_bounds__(kOutThreads) void k_out_fwd(const uint16_t* __restrict__ h, int64_t n,
+                                                         int width, const uint16_t* __restrict__ W,
+                                                         const float* __restrict__ b,
+                                                         float* __restrict__ y) {
+    __shared__ __attribute__((aligned(16))) uint16_t hs[kOutThreads * kOutChunk];
+    __shared__ float wf[2 * kOutChunk];
+    const int t = threadIdx.x;
+    const int64_t r0 = blockIdx.x * static_cast<int64_t>(kOutThreads);
     float s0 = 0.f, s1 = 0.f;
-    const uint16_t* hr = h + r * width;
-    // 16-byte loads of the row (width a multiple of 8), sums in k order
-    for (int k8 = 0; k8 < width; k8 += 8) {
-        const u16x8 hv = *reinterpret_cast<const u16x8*>(hr + k8);
+    for (int base = 0; base < width; base += kOutChunk) {
+        const int m = width - base < kOutChunk ? width - base : kOutChunk;
+        __syncthreads();
+        for (int i = t; i < 2 * m; i += kOutThreads) wf[i] = bf2f(W[2 * base + i]);
+        const int c8 = t & 31;
+        if (8 * c8 < m) {
+#pragma unroll 8
+            for (int row = t >> 5; row < kOutThreads; row += 2) {
+                const int64_t r = r0 + row < n ? r0 + row : n - 1;
+                *reinterpret_cast<u16x8*>(hs + row * kOutChunk + 8 * (c8 ^ (row & 31))) =
+                    *reinterpret_cast<const u16x8*>(h + r * width + base + 8 * c8);
+            }
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int k8 = 0; k8 < m; k8 += 8) {
+            const u16x8 hv = *reinterpret_cast<const u16x8*>(hs + t * kOutChunk +
+                                                             8 * ((k8 >> 3) ^ (t & 31)));
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int k = k8 + q;
-            const float a = bf2f(hv[q]);
-            s0 += a * bf2f(W[2 * k]);
-            s1 += a * bf2f(W[2 * k + 1]);
+            for (int q = 0; q < 8; ++q) {
+                const float a = bf2f(hv[q]);
+                s0 += a * wf[2 * (k8 + q)];
+                s1 += a * wf[2 * (k8 + q) + 1];
+            }
         }
     }
+    const int64_t r = r0 + t;
+    if (r >= n) return;
     y[2 * r] = s0 + b[0];
     y[2 * r + 1] = s1 + b[1];
 }
@@ -351,16 +378,30 @@ __global__ void k_loss(const float* __restrict__ y, const float* __restrict__ ta
     if (threadIdx.x == 0) atomicAdd(loss, part[0]);
 }
 
-// da = bf16(bf16(dy W_out^T) * gelu'(pre)) for the last hidden layer.
-__global__ void k_out_bwd_data(const float* __restrict__ dy, int64_t n, int width,
-                               const uint16_t* __restrict__ W, const float* __restrict__ pre,
-                               uint16_t* __restrict__ da) {
-    const int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (idx >= n * width) return;
-    const int64_t r = idx / width;
-    const int k = static_cast<int>(idx - r * width);
-    const float dh = bf2f(f2bf(dy[2 * r] * bf2f(W[2 * k]) + dy[2 * r + 1] * bf2f(W[2 * k + 1])));
-    da[idx] = f2bf(dh * gelu_grad(pre[idx]));
+// da = bf16(bf16(dy W_out^T) * gelu'(pre)) for the last hidden layer, kOutStep
+// rows' element of one column a thread: no division by the width, the column's
+// weights read once (8192 x 256: 7.6 -> 5 us).
+constexpr int kOutStep = 4;
+
+__global__ __launch_bounds__(256) void k_out_bwd_data(const float* __restrict__ dy, int64_t n,
+                                                      int width, const uint16_t* __restrict__ W,
+                                                      const float* __restrict__ pre,
+                                                      uint16_t* __restrict__ da) {
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kOutStep;
+    for (int k = threadIdx.x; k < width; k += blockDim.x) {
+        const float w0 = bf2f(W[2 * k]), w1 = bf2f(W[2 * k + 1]);
+        float p[kOutStep];
+#pragma unroll
+        for (int q = 0; q < kOutStep; ++q)
+            p[q] = pre[(r0 + q < n ? r0 + q : n - 1) * width + k];
+#pragma unroll
+        for (int q = 0; q < kOutStep; ++q) {
+            const int64_t r = r0 + q;
+            if (r >= n) break;
+            const float dh = bf2f(f2bf(dy[2 * r] * w0 + dy[2 * r + 1] * w1));
+            da[r * width + k] = f2bf(dh * gelu_grad(p[q]));
+        }
+    }
 }
 
 // The column-sum kernels: a block takes kSumRows rows, kSumGroups groups of 256
@@ -845,7 +886,8 @@ int nbx_mlp_features(const float* inp, int64_t n, const float* shift, const floa
 int nbx_mlp_out_forward(const uint16_t* h, int64_t n, int width, const uint16_t* W,
                         const float* b, float* y, nbx_stream stream) {
     if (n == 0) return 0;
-    k_out_fwd<<<blocks_for(n, 256), 256, 0, as_stream(stream)>>>(h, n, width, W, b, y);
+    k_out_fwd<<<blocks_for(n, kOutThreads), kOutThreads, 0, as_stream(stream)>>>(h, n, width, W, b,
+                                                                               y);
     NBX_LAUNCHED("mlp_out_fwd");
     return 0;
 }
@@ -868,7 +910,7 @@ int nbx_mlp_out_backward(const float* dy, const uint16_t* h, const float* pre, i
     k_fill2_f32<<<blocks_for(2 * width + 2, 256), 256, 0, s>>>(gW, 2 * width, gb, 2);
     k_out_bwd_weight<<<static_cast<unsigned>((n + kSumRows - 1) / kSumRows), kSumThreads, 0, s>>>(
         h, dy, n, width, gW, gb);
-    k_out_bwd_data<<<blocks_for(n * width, 256), 256, 0, s>>>(dy, n, width, W, pre, da);
+    k_out_bwd_data<<<blocks_for(n, kOutStep), 256, 0, s>>>(dy, n, width, W, pre, da);
     NBX_LAUNCHED("mlp_out_bwd");
     return 0;
 }

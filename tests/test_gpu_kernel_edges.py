@@ -303,3 +303,41 @@ def test_weight_grad_with_column_sums(M, N, K):
     eps = K * 2.0 ** -23
     assert ((gW.double().cpu() - hd.T @ dd).abs() <= eps * (hd.abs().T @ dd.abs())).all()
     assert ((gb.double().cpu() - dd.sum(0)).abs() <= eps * dd.abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("n", [1, 3, 63, 65, 130])
+@pytest.mark.parametrize("width", [8, 64, 256, 264, 512])
+def test_output_layer_of_any_width(n, width):
+    """The output layer forward and backward where its rows' blocks and its
+    chunks of 256 columns are cut short.  Sums within width (or n) ulps of the
+    magnitudes; the deltas two roundings to bf16 from float64."""
+    import torch
+    from numbacs_amd import _lib
+
+    lib, rng = _lib.load(), np.random.default_rng(n + width)
+
+    def dev(a, dtype):
+        return torch.tensor(a, dtype=dtype, device="cuda")
+
+    h, W = (dev(rng.standard_normal(s), torch.bfloat16) for s in ((n, width), (width, 2)))
+    b, dy, pre = (dev(rng.standard_normal(s), torch.float32) for s in ((2,), (n, 2), (n, width)))
+    y = torch.full((n, 2), float("nan"), device="cuda")
+    gW, gb = torch.full((width, 2), float("nan"), device="cuda"), torch.zeros(2, device="cuda")
+    da = torch.full((n, width), float("nan"), dtype=torch.bfloat16, device="cuda")
+    s = _lib.stream_ptr()
+    _lib.check(lib.nbx_mlp_out_forward(_lib.ptr(h), n, width, _lib.ptr(W), _lib.ptr(b),
+                                       _lib.ptr(y), s))
+    _lib.check(lib.nbx_mlp_out_backward(_lib.ptr(dy), _lib.ptr(h), _lib.ptr(pre), n, width,
+                                        _lib.ptr(W), _lib.ptr(gW), _lib.ptr(gb), _lib.ptr(da), s))
+    y, gW, gb, da, h, W, b, dy, pre = (v.double().cpu()
+                                       for v in (y, gW, gb, da, h, W, b, dy, pre))
+    ulp = 2.0 ** -23
+    assert ((y - (h @ W + b)).abs() <= (width + 1) * ulp * (h.abs() @ W.abs() + b.abs())).all()
+    assert ((gW - h.T @ dy).abs() <= (n + 1) * ulp * (h.abs().T @ dy.abs())).all()
+    assert ((gb - dy.sum(0)).abs() <= (n + 1) * ulp * dy.abs().sum(0)).all()
+    t = torch.tanh(0.7978845608028654 * (pre + 0.044715 * pre ** 3))
+    slope = 0.5 * (1 + t) + 0.5 * pre * (1 - t ** 2) * 0.7978845608028654 * (
+        1 + 3 * 0.044715 * pre ** 2)
+    dh, mag = dy @ W.T, dy.abs() @ W.abs().T
+    err = (2.0 ** -7 * dh.abs() + 4 * ulp * mag) * slope.abs() + 1e-5 * dh.abs()
+    assert ((da - dh * slope).abs() <= err).all()
