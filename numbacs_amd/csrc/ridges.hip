@@ -315,10 +315,10 @@ int percentile_device(const double* f, int64_t n, double q, SelState* st,
     const double gamma = vi - lo;
     k_sel_init<<<1, 256, 0, s>>>(st, klo, khi);
     NBX_LAUNCHED("sel_init");
-    // about 16 keys per thread, at most a block a CU: every block adds its
+    // one turn of 4 keys a thread, at most a block a CU: every block adds its
     // nonzero bins to the same global counters (8 M values: 75 us for the passes;
     // 512 blocks 77, of half the threads 83)
-    unsigned nb = blocks_for(n, kSelThreads * 16);
+    unsigned nb = blocks_for(n, kSelThreads * 4);
     if (nb > 256) nb = 256;
     for (int pass = 0; pass < kSelPasses; ++pass) {
         k_sel_hist<<<nb, kSelThreads, 0, s>>>(f, n, st, pass, held, n < kSelHeld ? n : kSelHeld);
