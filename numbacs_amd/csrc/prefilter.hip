@@ -193,8 +193,9 @@ int lines_per_block(int n) {
 }
 
 // ---------------------------------------------------------------------------
-// Lines too long for LDS: one thread per line in global memory, the samples
-// first scattered into the coefficient array.
+// Lines too long for LDS or too many for one launch of groups (2^29 of up to 253
+// samples): one thread per line in global memory, the samples first scattered
+// into the coefficient array.
 
 __device__ void prefilter_line(double* p, long stride, int n) {
     auto C = [&](int k) -> double& { return p[(static_cast<long>(k) + 1) * stride]; };
@@ -297,8 +298,13 @@ int launch_axis(const double* U, int nt, int nx, int ny, double* C, int axis, hi
 
 int prefilter_axis(const double* U, int nt, int nx, int ny, double* C, int axis, hipStream_t s) {
     const int n = axis == 2 ? ny : axis == 1 ? nx : nt;
+    const int64_t lines = axis == 2   ? static_cast<int64_t>(nt) * nx
+                          : axis == 1 ? ny + 2
+                                      : static_cast<int64_t>(nx + 2) * (ny + 2);
     int L = lines_per_block(n);
-    // (a grid's y extent holds 65535 slices)
+    // (a launch holds fewer than 2^32 threads -- past that its last blocks do not
+    // run, and no error says so -- and its grid's y extent 65535 slices)
+    if (L > 0 && (lines + L - 1) / L * kThreads >= int64_t(1) << 32) L = 0;
     if (axis == 1 && nt > 65535) L = 0;
     switch (L) {
         case 32: return launch_axis<32>(U, nt, nx, ny, C, axis, s);
@@ -315,10 +321,8 @@ int prefilter_axis(const double* U, int nt, int nx, int ny, double* C, int axis,
                                                                                     C);
         NBX_LAUNCHED("prefilter_scatter");
     }
-    const long lines = axis == 2   ? static_cast<long>(nt) * nx
-                       : axis == 1 ? static_cast<long>(nt) * (ny + 2)
-                                   : static_cast<long>(nx + 2) * (ny + 2);
-    k_prefilter_axis<<<blocks_for(lines, 128), 128, 0, s>>>(C, nt, nx, ny, axis);
+    k_prefilter_axis<<<blocks_for(axis == 1 ? nt * lines : lines, 128), 128, 0, s>>>(C, nt, nx, ny,
+                                                                                     axis);
     NBX_LAUNCHED("prefilter_axis");
     return 0;
 }
