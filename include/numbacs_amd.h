@@ -157,12 +157,14 @@ int nbx_flowmap_compose(const double* flowmaps, int nslots, int first, int nT, d
  * (0: one lane group per particle in one launch over the particle tiles;
  * n > 0: a persistent grid of n blocks per compute unit taking wavefront
  * tiles from a device queue, a tile going back to the queue every 16
- * steps while a particle of it is still running, unless the tiles do not
- * outnumber the grid's wavefronts, outnumber them more than 16 times or the
- * stream is capturing: then as 0; -1: spline coefficients
+ * steps while a particle of it is still running; -1: spline coefficients
  * staged through LDS per step, spline flows at 4 lanes and 64-thread
  * blocks; persistent and staged launches serve grid flow maps and batches,
- * other sources run the plain launch).  Process-wide; set by the autotuner
+ * other sources run the plain launch).  The Bickley jet's default is a queue
+ * (8 blocks per compute unit, 12 for NBX_FP32_DISP) that is left for the
+ * launch of 0 where the tiles do not outnumber the grid's wavefronts or
+ * outnumber them more than 16 times, and on a stream that is capturing; a
+ * queue set to other numbers runs as set.  Process-wide; set by the autotuner
  * (numbacs_amd.autotune).  No reference counterpart (the reference's
  * parallel loop has no tunables, integration.py:166). */
 int nbx_set_launch_config(int kind, int precision, int lanes_per_particle, int block_threads,

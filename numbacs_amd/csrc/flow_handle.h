@@ -31,11 +31,15 @@ namespace nbx {
 //   block       threads per block (64, 128 or 256);
 //   persistent  0: one group per particle, one launch covering all of them;
 //               n > 0: a persistent grid of n blocks per CU pulling
-//               particles from a device work queue.
+//               particles from a device work queue;
+//   requested   set to something else than the kind's default.  A requested
+//               launch is the one that runs; a default queue is a choice of
+//               the launcher, which leaves it where the grid launch is better.
 struct LaunchCfg {
     int lanes;
     int block;
     int persistent;
+    bool requested = false;
 };
 
 LaunchCfg launch_cfg(int kind, int precision);

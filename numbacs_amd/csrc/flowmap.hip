@@ -496,10 +496,14 @@ __global__ void k_flow_eval(Flow f, const double* __restrict__ t, const double2*
 // behind its last wavefronts, so it runs the tile queue at its kernels'
 // occupancy (2 and 3 wavefronts per SIMD): 401,401 particles 17.1 -> 14.0 ms,
 // float 10.0 -> 8.0; 1.6 M 49.6 -> 46.4 ms.
-LaunchCfg g_cfg[4][2] = {{{1, 64, 0}, {1, 64, 0}},
-                         {{1, 64, 8}, {1, 64, 12}},
-                         {{4, 128, 0}, {4, 128, 0}},
-                         {{1, 64, 0}, {1, 64, 0}}};
+constexpr LaunchCfg kDefaultCfg[4][2] = {{{1, 64, 0}, {1, 64, 0}},
+                                         {{1, 64, 8}, {1, 64, 12}},
+                                         {{4, 128, 0}, {4, 128, 0}},
+                                         {{1, 64, 0}, {1, 64, 0}}};
+LaunchCfg g_cfg[4][2] = {{kDefaultCfg[0][0], kDefaultCfg[0][1]},
+                         {kDefaultCfg[1][0], kDefaultCfg[1][1]},
+                         {kDefaultCfg[2][0], kDefaultCfg[2][1]},
+                         {kDefaultCfg[3][0], kDefaultCfg[3][1]}};
 // edge-first tile order of the spline grid launch, per precision
 int g_edge_first[2] = {1, 1};
 std::mutex g_cfg_mutex;
@@ -567,14 +571,17 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
             const int64_t want = (ntiles * 64 + block - 1) / block;
             const int64_t most = static_cast<int64_t>(cus) * cfg.persistent;
-            // With a wavefront for every tile there is nothing to hand on; from
-            // 16 rounds of them the tail is a few percent and not worth the
-            // states' memory.  A stream under capture takes the grid launch too
-            // (the queue's workspace may have to be allocated).
-            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-            (void)hipStreamIsCapturing(s, &capture);
-            if (want <= most || want > 16 * most || capture != hipStreamCaptureStatusNone)
-                return launch_grid<Flow, R, G>(f, src, a, block, s);
+            // The queue as a kind's default: with a wavefront for every tile
+            // there is nothing to hand on; from 16 rounds of them the tail is a
+            // few percent and not worth the states' memory.  A stream under
+            // capture takes the grid launch too (the queue's workspace may have
+            // to be allocated).
+            if (!cfg.requested) {
+                hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+                (void)hipStreamIsCapturing(s, &capture);
+                if (want <= most || want > 16 * most || capture != hipStreamCaptureStatusNone)
+                    return launch_grid<Flow, R, G>(f, src, a, block, s);
+            }
             const unsigned long long ring = chunk_ring(ntiles);
             const size_t state_off = ring * sizeof(unsigned long long) + 256;
             Workspace ws(s, 3, state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots));
@@ -587,7 +594,7 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
                                ring - 1, static_cast<unsigned long long>(ntiles)};
             k_chunk_init<<<blocks_for(static_cast<int64_t>(ring), 256), 256, 0, s>>>(q, ntiles);
             NBX_LAUNCHED("chunk_init");
-            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(most), block,
+            k_flowmap_chunks<Flow, R, G><<<static_cast<unsigned>(std::min(want, most)), block,
                                            solve_lds_bytes<Flow, R, G>(block), s>>>(
                 f, single_request(src, a), nullptr, nullptr, 1, q,
                 reinterpret_cast<decltype(Solve<Flow, R, G>::s)*>(w + state_off), a.rtol, a.atol,
@@ -1026,8 +1033,12 @@ int nbx_set_launch_config(int kind, int precision, int lanes_per_particle, int b
     NBX_REQUIRE(persistent_blocks_per_cu != -1 ||
                     (kind == NBX_FLOW_SPLINE3 && lanes_per_particle == 4 && block_threads == 64),
                 "the LDS-staged launch (-1) is for spline flows at 4 lanes, 64-thread blocks");
+    const LaunchCfg& d = kDefaultCfg[kind][precision];
+    const bool requested = lanes_per_particle != d.lanes || block_threads != d.block ||
+                           persistent_blocks_per_cu != d.persistent;
     std::lock_guard<std::mutex> lock(g_cfg_mutex);
-    g_cfg[kind][precision] = LaunchCfg{lanes_per_particle, block_threads, persistent_blocks_per_cu};
+    g_cfg[kind][precision] =
+        LaunchCfg{lanes_per_particle, block_threads, persistent_blocks_per_cu, requested};
     return 0;
 }
 

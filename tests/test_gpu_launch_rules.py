@@ -33,6 +33,73 @@ def configs(lib):
         autotune.set_order(p, o)
 
 
+class Capture:
+    """Capture of one stream of its own by the HIP runtime the library uses."""
+
+    def __init__(self, lib, mode):
+        self.hip = ctypes.CDLL(lib.LIB_PATH)
+        self.stream = lib.torch().cuda.Stream()
+        self.mode = mode
+
+    def __enter__(self):
+        lib_stream = ctypes.c_void_p(self.stream.cuda_stream)
+        assert self.hip.hipStreamBeginCapture(lib_stream, self.mode) == 0
+        return self
+
+    def __exit__(self, *exc):
+        graph, count = ctypes.c_void_p(), ctypes.c_size_t()
+        self.status = self.hip.hipStreamEndCapture(ctypes.c_void_p(self.stream.cuda_stream),
+                                                   ctypes.byref(graph))
+        self.nodes = 0
+        if self.status == 0 and graph.value:
+            assert self.hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+            self.nodes = count.value
+            self.hip.hipGraphDestroy(graph)
+
+
+def kernels_of(lib, call):
+    """Number of kernels that call() enqueues on the current stream, by a
+    capture; called once before it, so that its workspaces are there."""
+    capture = Capture(lib, RELAXED)
+    with lib.torch().cuda.stream(capture.stream):
+        call()
+        capture.stream.synchronize()
+        with capture:
+            call()
+    assert capture.status == 0
+    return capture.nodes
+
+
+def small_spline(extrap_mode="constant"):
+    from numbacs_amd.flows import get_flow_2D
+
+    n = (8, 20, 18)
+    C = np.random.default_rng(1).standard_normal((2,) + tuple(m + 2 for m in n))
+    return get_flow_2D(tuple((0.0, 1.0, m) for m in n), C[0], C[1], extrap_mode=extrap_mode)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("cfg", [(4, 64, 4), (2, 64, 4), (4, 128, 2), (1, 256, 8)])
+@pytest.mark.parametrize("shape", [(9, 33), (801, 501)])
+def test_requested_queue_is_what_runs(lib, configs, precision, cfg, shape):
+    """A queue launch is two kernels (the ring's start, the persistent grid),
+    also for fewer tiles than the grid has wavefronts and for more than 16
+    rounds of them; the map equals the grid launch's at the same lanes."""
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    f = small_spline("nearest")
+    xd, yd = (lib.to_dev(np.linspace(0.0, 1.0, n)) for n in shape)
+    out = lib.empty(shape + (2,))
+    call = lambda: flowmap_grid_2d_device(f, 0.0, 0.5, xd, yd, [1.0], precision=precision, out=out)
+    configs.set_config(2, precision, cfg)
+    assert kernels_of(lib, call) == 2
+    call()
+    got = lib.to_host(out)
+    configs.set_config(2, precision, cfg[:2] + (0,))
+    call()
+    assert np.array_equal(got, lib.to_host(out))
+
+
 @pytest.mark.parametrize("shape", [(1, 23170, 23170), (23171, 23171, 1)])
 def test_prefilter_of_more_lines_than_one_launch_holds(lib, shape):
     """Axes of one sample with 2^29 lines and more across them (8 threads of the
