@@ -84,10 +84,19 @@ struct nbx_batch {
 namespace nbx {
 namespace {
 
+// Whether a batch runs the tile queue: where the configuration asks for it.  A
+// kind's default queue is for single grids: a batch would have to keep a solver
+// state per slot for its lifetime (112 bytes; 1.1 GB for 10 M particles), could
+// not be run inside a capture without having run before, nor on two streams
+// at once.
+bool runs_queue(const LaunchCfg& cfg) {
+    return cfg.persistent != 0 && cfg.requested;
+}
+
 template <class Flow, class R, int G>
 int launch_batch_queue(nbx_batch* b, const Flow& f, const LaunchCfg& cfg, hipStream_t s) {
     const int block = cfg.block;
-    if (cfg.persistent == 0) {
+    if (!runs_queue(cfg)) {
         if (b->total_slots == 0) return 0;
         k_flowmap_tiles<Flow, R, G><<<blocks_for(b->total_slots * G, block), block,
                                     solve_lds_bytes<Flow, R, G>(block), s>>>(
@@ -125,16 +134,18 @@ int launch_batch_queue(nbx_batch* b, const Flow& f, const LaunchCfg& cfg, hipStr
 
 // Allocate (or grow) the queue launch's buffers for the current launch
 // configuration: before a run, and before a capture (no allocation may
-// happen inside one).  Sized for the FP64 state, the larger of the two.
+// happen inside one).  Sized for the FP64 states of the lane groups it runs.
 int ensure_chunk_buffers(nbx_batch* b) {
     const LaunchCfg cfg = launch_cfg(b->flow->kind, b->precision);
-    if (cfg.persistent <= 0 || b->total_slots == 0) return 0;
+    if (!runs_queue(cfg) || cfg.persistent < 0 || b->total_slots == 0) return 0;
     int G = (b->flow->kind == NBX_FLOW_SPLINE3 && b->flow->extrap != 1) ? cfg.lanes : 1;
-    if (pair_lanes<double>(b->flow, b->total)) G = 2;
+    if (b->precision == NBX_FP32_DISP ? pair_lanes<float>(b->flow, b->total)
+                                      : pair_lanes<double>(b->flow, b->total))
+        G = 2;
     const int64_t ntiles = b->total_slots / (64 / G);
     NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
     const size_t need = chunk_ring(ntiles) * sizeof(unsigned long long) + 256 +
-                        std::max(solve_state_bytes<double, 1>(), solve_state_bytes<double, 4>()) *
+                        (G == 1 ? solve_state_bytes<double, 1>() : solve_state_bytes<double, 4>()) *
                             static_cast<size_t>(b->total_slots);
     if (b->chunk_bytes >= need) return 0;
     if (b->d_chunk) (void)hipFree(b->d_chunk);

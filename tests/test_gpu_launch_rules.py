@@ -100,6 +100,55 @@ def test_requested_queue_is_what_runs(lib, configs, precision, cfg, shape):
     assert np.array_equal(got, lib.to_host(out))
 
 
+@pytest.mark.parametrize("kind,precision,n", [(0, 0, 90000), (0, 0, 150000), (0, 1, 150000),
+                                              (0, 1, 300000), (1, 0, 90000), (1, 1, 90000)])
+def test_requested_queue_batch(lib, configs, kind, precision, n):
+    """A requested queue holds the states of the lane groups that run: analytic
+    flows on both sides of the double gyre's pair limits."""
+    from numbacs_amd.batch import FTLEBatch
+    from numbacs_amd.flows import get_predefined_flow
+
+    flow, p, dom = get_predefined_flow(("double_gyre", "bickley_jet")[kind])
+    x, y = np.linspace(*dom[0], n // 100), np.linspace(*dom[1], 100)
+    b = FTLEBatch(flow, [dict(t0=0.0, T=0.5, x=x, y=y)], p, precision=("fp64", "fp32")[precision],
+                  ftle=False)
+    configs.set_config(kind, precision, (1, 64, 4))
+    assert kernels_of(lib, b.run) == 2
+    b.run()
+    got = b.results()[0]["flowmap"]
+    configs.set_config(kind, precision, (1, 64, 0))
+    assert kernels_of(lib, b.run) == 1
+    b.run()
+    assert np.array_equal(got, b.results()[0]["flowmap"])
+    b.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_default_bickley_batch_takes_no_memory(lib, precision):
+    """A batch keeps no solver states unless its launch shape was set to the
+    queue: 1.4 M particles would hold 150 MB and more.  Its maps equal the
+    single grids'."""
+    from numbacs_amd.batch import FTLEBatch
+    from numbacs_amd.flows import get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    flow, p, dom = get_predefined_flow("bickley_jet")
+    x, y = np.linspace(*dom[0], 1401), np.linspace(*dom[1], 1001)
+    b = FTLEBatch(flow, [dict(t0=0.0, T=0.5, x=x, y=y)], p, precision=("fp64", "fp32")[precision],
+                  ftle=False)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    b.run()
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < 64 << 20
+    got = b.results()[0]["flowmap"]
+    want = flowmap_grid_2d_device(flow, 0.0, 0.5, lib.to_dev(x), lib.to_dev(y), p,
+                                  precision=precision)
+    assert np.array_equal(got, lib.to_host(want))
+    b.close()
+
+
 @pytest.mark.parametrize("shape", [(1, 23170, 23170), (23171, 23171, 1)])
 def test_prefilter_of_more_lines_than_one_launch_holds(lib, shape):
     """Axes of one sample with 2^29 lines and more across them (8 threads of the
