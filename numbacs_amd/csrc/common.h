@@ -56,9 +56,12 @@ inline unsigned blocks_for(int64_t n, int threads) {
 // run concurrently, calls on one stream from several host threads take turns
 // (and their device work is ordered by the stream).  Growing frees the old
 // buffer with hipFree, which waits for the device work that used it.
+// apart: the buffer may be grown while other streams are being captured (in
+// the runtime's relaxed mode, or an allocation would invalidate their captures);
+// its stream itself must not be, and nothing captured may use the slot.
 class Workspace {
    public:
-    Workspace(hipStream_t stream, int slot, size_t bytes);
+    Workspace(hipStream_t stream, int slot, size_t bytes, bool apart = false);
     Workspace(const Workspace&) = delete;
     Workspace& operator=(const Workspace&) = delete;
     char* get() const { return ptr_; }

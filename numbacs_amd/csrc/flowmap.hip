@@ -41,7 +41,26 @@ std::map<std::tuple<int, hipStream_t, int>, std::unique_ptr<WsEntry>> g_ws;
 
 void set_error(const std::string& msg) { g_last_error = msg; }
 
-Workspace::Workspace(hipStream_t stream, int slot, size_t bytes) {
+namespace {
+// This thread's allocations in relaxed mode while it is in scope.
+class RelaxedCapture {
+   public:
+    explicit RelaxedCapture(bool on) : on_(on) {
+        if (on_) on_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess;
+    }
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+    ~RelaxedCapture() {
+        if (on_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+
+   private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool on_;
+};
+}  // namespace
+
+Workspace::Workspace(hipStream_t stream, int slot, size_t bytes, bool apart) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         set_error("hipGetDevice failed");
@@ -57,6 +76,7 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes) {
     }
     lock_ = std::unique_lock<std::mutex>(e->m);
     if (e->bytes < bytes) {
+        const RelaxedCapture relaxed(apart);
         if (e->ptr) {
             // hipFree waits for the device work still using the old buffer
             (void)hipFree(e->ptr);
@@ -65,6 +85,8 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes) {
         }
         const size_t want = bytes < 4096 ? 4096 : bytes;
         if (hipMalloc(&e->ptr, want) != hipSuccess) {
+            (void)hipGetLastError();
+            e->ptr = nullptr;
             set_error("workspace hipMalloc failed");
             err_ = -1;
             return;
@@ -575,7 +597,7 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             // there is nothing to hand on; from 16 rounds of them the tail is a
             // few percent and not worth the states' memory.  A stream under
             // capture takes the grid launch too (the queue's workspace may have
-            // to be allocated).
+            // to be allocated), and so does a call that cannot have it.
             if (!cfg.requested) {
                 hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
                 (void)hipStreamIsCapturing(s, &capture);
@@ -584,8 +606,15 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             }
             const unsigned long long ring = chunk_ring(ntiles);
             const size_t state_off = ring * sizeof(unsigned long long) + 256;
-            Workspace ws(s, 3, state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots));
-            if (ws.error()) return ws.error();
+            // (a slot of its own for the default: a captured queue's workspace
+            // is grown by requested queues only)
+            Workspace ws(s, cfg.requested ? 3 : 5,
+                         state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots),
+                         !cfg.requested);
+            if (ws.error()) {
+                if (cfg.requested) return ws.error();
+                return launch_grid<Flow, R, G>(f, src, a, block, s);
+            }
             char* w = ws.get();
             const ChunkQueue q{reinterpret_cast<unsigned long long*>(w),
                                reinterpret_cast<unsigned long long*>(w + state_off - 256),

@@ -149,6 +149,69 @@ def test_default_bickley_batch_takes_no_memory(lib, precision):
     b.close()
 
 
+def test_default_bickley_map_during_another_capture(lib):
+    """A default flow map on one stream while another is being captured, in
+    the mode that refuses allocations meanwhile and is invalidated by them: the
+    map runs and the capture goes on."""
+    from numbacs_amd.flows import get_predefined_flow
+
+    torch = lib.torch()
+    flow, p, dom = get_predefined_flow("bickley_jet")
+    nx, ny = 711, 333
+    xd, yd = lib.to_dev(np.linspace(*dom[0], nx)), lib.to_dev(np.linspace(*dom[1], ny))
+    out, want = lib.empty((nx, ny, 2)), lib.empty((nx, ny, 2))
+    p = np.ascontiguousarray(p, dtype=np.float64)
+    hip = ctypes.CDLL(lib.LIB_PATH)
+
+    def run(dst, stream):
+        return lib.load().nbx_flowmap_grid_2d(
+            flow.handle, 0.0, 2.0, lib.ptr(xd), nx, lib.ptr(yd), ny, p.ctypes.data, p.size, 1e-6,
+            1e-8, None, 100000, 0, lib.ptr(dst), None, None, stream)
+
+    torch.cuda.synchronize()
+    other = ctypes.c_void_p()  # a stream that has no workspace yet
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
+    with Capture(lib, GLOBAL) as capture:
+        rc = run(out, other.value)
+    assert rc == 0, lib.load().nbx_last_error()
+    assert capture.status == 0
+    assert hip.hipStreamSynchronize(other) == 0
+    assert run(want, lib.stream_ptr()) == 0
+    assert torch.equal(out, want)
+
+
+def test_captured_queue_keeps_its_workspace(lib, configs):
+    """A requested queue captured on a stream, then a larger map of the default
+    configuration on the same stream: the graph's workspace is not grown away
+    from under it.  Replayed several times, with eager maps between."""
+    from numbacs_amd.flows import get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    flow, p, dom = get_predefined_flow("bickley_jet")
+
+    def axes(*n):
+        return [lib.to_dev(np.linspace(*d, m)) for d, m in zip(dom, n)]
+
+    small, large = axes(301, 111), axes(801, 401)
+    out, eager, big = (lib.empty(s + (2,)) for s in ((301, 111), (301, 111), (801, 401)))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    default = configs.get(1, 0)
+    with torch.cuda.stream(stream):
+        configs.set_config(1, 0, (1, 64, 1))
+        flowmap_grid_2d_device(flow, 0.0, 5.0, *small, p, out=eager)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            flowmap_grid_2d_device(flow, 0.0, 5.0, *small, p, out=out)
+        configs.set_config(1, 0, default)
+        for _ in range(3):
+            flowmap_grid_2d_device(flow, 0.0, 5.0, *large, p, out=big)
+            out.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(out, eager)
+
+
 @pytest.mark.parametrize("shape", [(1, 23170, 23170), (23171, 23171, 1)])
 def test_prefilter_of_more_lines_than_one_launch_holds(lib, shape):
     """Axes of one sample with 2^29 lines and more across them (8 threads of the
