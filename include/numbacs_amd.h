@@ -163,8 +163,9 @@ int nbx_flowmap_compose(const double* flowmaps, int nslots, int first, int nT, d
  * other sources run the plain launch).  The Bickley jet's default is a queue
  * (8 blocks per compute unit, 12 for NBX_FP32_DISP) that is left for the
  * launch of 0 where the tiles do not outnumber the grid's wavefronts or
- * outnumber them more than 16 times, on a stream that is capturing and in
- * batches; a queue set to other numbers runs as set.  Process-wide; set by the autotuner
+ * outnumber them more than 16 times, on a stream that is capturing, for
+ * max_steps above 100000 and in batches; a queue set to other numbers runs
+ * as set.  Process-wide; set by the autotuner
  * (numbacs_amd.autotune).  No reference counterpart (the reference's
  * parallel loop has no tunables, integration.py:166). */
 int nbx_set_launch_config(int kind, int precision, int lanes_per_particle, int block_threads,

@@ -88,7 +88,8 @@ namespace {
 // kind's default queue is for single grids: a batch would have to keep a solver
 // state per slot for its lifetime (112 bytes; 1.1 GB for 10 M particles), could
 // not be run inside a capture without having run before, nor on two streams
-// at once.
+// at once (401,401 particles of the Bickley jet: 17.0 ms, in a requested queue
+// of 7 blocks a CU 14.6).
 bool runs_queue(const LaunchCfg& cfg) {
     return cfg.persistent != 0 && cfg.requested;
 }

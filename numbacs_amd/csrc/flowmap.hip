@@ -597,11 +597,13 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             // there is nothing to hand on; from 16 rounds of them the tail is a
             // few percent and not worth the states' memory.  A stream under
             // capture takes the grid launch too (the queue's workspace may have
-            // to be allocated), and so does a call that cannot have it.
+            // to be allocated), and so do a call that cannot have it and one
+            // that allows solves of any length.
             if (!cfg.requested) {
                 hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
                 (void)hipStreamIsCapturing(s, &capture);
-                if (want <= most || want > 16 * most || capture != hipStreamCaptureStatusNone)
+                if (want <= most || want > 16 * most || a.nmax > kDefaultQueueSteps ||
+                    capture != hipStreamCaptureStatusNone)
                     return launch_grid<Flow, R, G>(f, src, a, block, s);
             }
             const unsigned long long ring = chunk_ring(ntiles);

@@ -157,9 +157,13 @@ struct ChunkQueue {
     unsigned long long ntiles;
 };
 // Polls of an unfilled claim before a wavefront gives up waiting (about ten
-// seconds at ~1 us of sleep per poll): a safety bound, far beyond any solve
-// here; a wavefront that gives up drops its claim.
+// seconds at ~1 us of sleep per poll): a safety bound; a wavefront that gives
+// up drops its claim, and the tile later handed to it is lost.
 constexpr int kMaxPolls = 10 << 20;
+// Steps a particle may take in a queue that was not asked for: a wavefront that
+// ran out of tiles may wait as long as the longest solve lasts, and the jet's
+// 100,000 steps (the entry points' default limit) take 1.5 seconds.
+constexpr long long kDefaultQueueSteps = 100000;
 // payload bit 31: the tile has been started (its states are stored)
 constexpr unsigned kResume = 0x80000000u;
 

@@ -149,6 +149,33 @@ def test_default_bickley_batch_takes_no_memory(lib, precision):
     b.close()
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_default_bickley_map_of_long_solves(lib, precision):
+    """A wavefront waits in the queue for a bounded time, so a map that allows
+    more steps than the entry points' default takes the grid launch, which holds
+    no states; the queue's stream holds 112 bytes a slot."""
+    from numbacs_amd.flows import get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    flow, p, dom = get_predefined_flow("bickley_jet")
+    hip, stream = ctypes.CDLL(lib.LIB_PATH), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0  # without a workspace yet
+    xd, yd = (lib.to_dev(np.linspace(*d, n)) for d, n in zip(dom, (1401, 1001)))
+    out = [lib.empty((1401, 1001, 2)) for _ in range(2)]
+    held = []
+    with torch.cuda.stream(torch.cuda.ExternalStream(stream.value)):
+        for dst, steps in zip(out, (100001, 100000)):
+            torch.cuda.synchronize()
+            before = torch.cuda.mem_get_info()[0]
+            flowmap_grid_2d_device(flow, 0.0, 0.5, xd, yd, p, max_steps=steps, precision=precision,
+                                   out=dst)
+            torch.cuda.synchronize()
+            held.append(before - torch.cuda.mem_get_info()[0])
+    assert held[0] < 64 << 20 < held[1]
+    assert torch.equal(*out)
+
+
 def test_default_bickley_map_during_another_capture(lib):
     """A default flow map on one stream while another is being captured, in
     the mode that refuses allocations meanwhile and is invalidated by them: the
