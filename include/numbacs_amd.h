@@ -92,7 +92,12 @@ int nbx_flow_create_linear3(const double* grid9_host, const double* U, const dou
  * scale (the np.moveaxis(u, 1, 2) * 3.6 of plot_merra_ftle.py:37-41). */
 int nbx_ingest_xy(const double* U_xy, int nt, int ny, int nx, double scale, double* U_ij,
                   nbx_stream stream);
+/* The arrays of a closed gridded flow may be held for the next one: at most
+ * 256 MiB a device, while the device has another flow.  nbx_release_memory gives
+ * back what is held on the current device, and the workspaces of default queue
+ * launches that no call is using. */
 void nbx_flow_destroy(nbx_flow* flow);
+int nbx_release_memory(void);
 
 /* Natural cubic B-spline prefilter (get_interp_arrays_2D, flows.py:39-46):
  * U (nt, nx, ny) -> C (nt+2, nx+2, ny+2). */

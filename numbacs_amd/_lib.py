@@ -37,6 +37,7 @@ SIGNATURES = {
     "nbx_flow_create_linear3": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_i, _c_d, _c_p, _c_p]),
     "nbx_ingest_xy": (_c_i, [_c_p, _c_i, _c_i, _c_i, _c_d, _c_p, _c_p]),
     "nbx_flow_destroy": (None, [_c_p]),
+    "nbx_release_memory": (_c_i, []),
     "nbx_prefilter3": (_c_i, [_c_p, _c_i, _c_i, _c_i, _c_p, _c_p]),
     "nbx_flow_eval": (_c_i, [_c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_p, _c_p]),
     "nbx_flowmap_grid_2d": (_c_i, [_c_p, _c_d, _c_d, _c_p, _c_i, _c_p, _c_i, _c_p, _c_i, _c_d,

@@ -152,7 +152,7 @@ int ensure_chunk_buffers(nbx_batch* b) {
     if (b->d_chunk) (void)hipFree(b->d_chunk);
     b->d_chunk = nullptr;
     b->chunk_bytes = 0;
-    NBX_HIP(hipMalloc(&b->d_chunk, need));
+    NBX_HIP(device_malloc(&b->d_chunk, need));
     b->chunk_bytes = need;
     return 0;
 }
@@ -274,11 +274,11 @@ int nbx_batch_create(const nbx_flow* flow, const nbx_request* reqs, int nreq,
     b->total = offsets[nreq];
     b->total_slots = slot_off[nreq];
     b->ntiles = static_cast<int>(tiles.size());
-    bool ok = hipMalloc(&b->d_table, sizeof(ReqDev) * nreq) == hipSuccess &&
-              hipMalloc(&b->d_slot_off, sizeof(int64_t) * (nreq + 1)) == hipSuccess;
+    bool ok = device_malloc(&b->d_table, sizeof(ReqDev) * nreq) == hipSuccess &&
+              device_malloc(&b->d_slot_off, sizeof(int64_t) * (nreq + 1)) == hipSuccess;
     if (ok && !ftle.empty())
-        ok = hipMalloc(&b->d_ftle, sizeof(FtleReqDev) * ftle.size()) == hipSuccess &&
-             hipMalloc(&b->d_tiles, sizeof(TileDev) * tiles.size()) == hipSuccess;
+        ok = device_malloc(&b->d_ftle, sizeof(FtleReqDev) * ftle.size()) == hipSuccess &&
+             device_malloc(&b->d_tiles, sizeof(TileDev) * tiles.size()) == hipSuccess;
     if (ok)
         ok = hipMemcpy(b->d_table, table.data(), sizeof(ReqDev) * nreq, hipMemcpyHostToDevice) ==
                  hipSuccess &&

@@ -49,6 +49,14 @@ inline unsigned blocks_for(int64_t n, int threads) {
     return static_cast<unsigned>((n + threads - 1) / threads);
 }
 
+// hipMalloc; where it fails, the blocks held from closed flows are given back and
+// it is tried again.  Leaves no error behind.
+hipError_t device_malloc(void** p, size_t bytes);
+template <class T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
+
 // Grow-only device scratch owned by the library: one buffer per (device,
 // stream, slot), held until the process ends.  A Workspace keeps its buffer
 // locked from construction to destruction, i.e. for the whole entry-point

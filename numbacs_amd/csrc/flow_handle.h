@@ -15,6 +15,7 @@ struct nbx_flow {
                               // trilinear: (nt, nx, ny) interleaved samples; device
     float4* coef32 = nullptr; // FP32 copy, time-paired, for the FP32-displacement path
     size_t coef_bytes = 0, coef32_bytes = 0;  // of the arrays, as allocated
+    void* token = nullptr;    // freed first at the close (see flow_release)
     int dev = -1;             // device of the arrays (-1: none)
     int64_t ncoef = 0;
     double grid9[9] = {0};

@@ -10,18 +10,17 @@
 #include <cmath>
 #include <cstring>
 #include <algorithm>
-#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <tuple>
 #include <type_traits>
 #include <string>
-#include <utility>
 #include <vector>
 
 #include "common.h"
 #include "dop853.h"
+#include "flow_blocks.h"
 #include "flow_handle.h"
 #include "flows.h"
 #include "queue.h"
@@ -35,6 +34,8 @@ struct WsEntry {
     void* ptr = nullptr;
     size_t bytes = 0;
 };
+// workspace slot of the queue launches that were not requested (never captured)
+constexpr int kDefaultQueueSlot = 5;
 std::mutex g_ws_mutex;  // guards the map, not the buffers
 std::map<std::tuple<int, hipStream_t, int>, std::unique_ptr<WsEntry>> g_ws;
 }  // namespace
@@ -84,9 +85,7 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes, bool apart) {
             e->bytes = 0;
         }
         const size_t want = bytes < 4096 ? 4096 : bytes;
-        if (hipMalloc(&e->ptr, want) != hipSuccess) {
-            (void)hipGetLastError();
-            e->ptr = nullptr;
+        if (device_malloc(&e->ptr, want) != hipSuccess) {
             set_error("workspace hipMalloc failed");
             err_ = -1;
             return;
@@ -96,90 +95,77 @@ Workspace::Workspace(hipStream_t stream, int slot, size_t bytes, bool apart) {
     ptr_ = static_cast<char*>(e->ptr);
 }
 
-// Device memory of flow handles.  A program that follows a data set replaces
-// its flow over and over (the next handle made, then the old one closed), and
-// hipFree and hipMalloc of the 2 x 44 MB of a 96-frame field cost 330 us of a
-// 550 us set-up.  So a closed flow's arrays wait here for the next one -- at
-// most kHeldBytes per device, and only while the device still has another
-// flow: the last handle to close gives everything back.  As hipFree does, a
-// close waits for the device's work first, so held memory is idle whatever
-// streams used it; an allocation that fails gives the held blocks back and is
-// tried again.
+// Flow handles' memory: the blocks of closed flows (flow_blocks.h) per device.
 namespace {
-constexpr size_t kHeldBytes = size_t(1) << 30;
-struct FlowBlocks {
-    std::vector<std::pair<void*, size_t>> held;
-    size_t bytes = 0;
-    int flows = 0;  // live gridded flows
-    void give_back() {
-        for (auto& b : held) (void)hipFree(b.first);
-        held.clear();
-        bytes = 0;
+struct FlowMemory {
+    static void* alloc(size_t bytes) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
     }
+    static void release(void* p) { (void)hipFree(p); }
 };
+using Blocks = FlowBlocks<FlowMemory>;
 std::mutex g_blocks_mutex;
-std::map<int, FlowBlocks> g_blocks;  // per device
+std::map<int, Blocks> g_blocks;  // per device
 
-// a held block of at least `bytes` and at most an eighth more, or a new one;
-// `bytes` becomes the block's size
-void* flow_alloc(int dev, size_t& bytes) {
-    std::lock_guard<std::mutex> lock(g_blocks_mutex);
-    FlowBlocks& fb = g_blocks[dev];
-    for (size_t i = 0; i < fb.held.size(); ++i) {
-        const auto b = fb.held[i];
-        if (b.second < bytes || b.second > bytes + bytes / 8) continue;
-        fb.held.erase(fb.held.begin() + i);
-        fb.bytes -= b.second;
-        bytes = b.second;
-        return b.first;
-    }
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError();
-    if (fb.held.empty()) return nullptr;
-    fb.give_back();
-    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
-}
-
-// the arrays of a closing flow (sizes as allocated; null entries allowed)
-void flow_release(int dev, std::initializer_list<std::pair<void*, size_t>> blocks) {
-    int cur = dev;
+// A closing flow: its token is freed first, which waits for the device's work
+// as freeing the arrays did, so blocks are held only when idle, whatever streams
+// used them.  (hipDeviceSynchronize takes 20 us less, but invalidates every
+// capture under way, another thread's of a batch among them; a free does so only
+// where the capture's mode forbids frees.)
+void flow_release(nbx_flow* fl) {
+    int cur = fl->dev;
     (void)hipGetDevice(&cur);
-    if (cur != dev) (void)hipSetDevice(dev);
-    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    if (cur != fl->dev) (void)hipSetDevice(fl->dev);
+    const bool idle = fl->token != nullptr && hipFree(fl->token) == hipSuccess;
     if (!idle) (void)hipGetLastError();
     {
         std::lock_guard<std::mutex> lock(g_blocks_mutex);
-        FlowBlocks& fb = g_blocks[dev];
-        --fb.flows;
-        for (const auto& b : blocks) {
-            if (b.first == nullptr) continue;
-            if (idle && fb.flows > 0 && fb.bytes + b.second <= kHeldBytes) {
-                fb.held.push_back(b);
-                fb.bytes += b.second;
-            } else {
-                (void)hipFree(b.first);
-            }
-        }
-        if (fb.flows <= 0) fb.give_back();
+        g_blocks[fl->dev].close({{fl->coef, fl->coef_bytes}, {fl->coef32, fl->coef32_bytes}}, idle);
     }
-    if (cur != dev) (void)hipSetDevice(cur);
+    if (cur != fl->dev) (void)hipSetDevice(cur);
 }
 
-// device and block sizes of a new gridded flow, counted among the live ones
+// A new gridded flow on the current device, with its token: a small allocation
+// of its own, refused where the runtime refuses allocations (during a capture),
+// also when the arrays come from held blocks.
 int flow_register(nbx_flow* fl) {
     if (hipGetDevice(&fl->dev) != hipSuccess) return -1;
-    std::lock_guard<std::mutex> lock(g_blocks_mutex);
-    ++g_blocks[fl->dev].flows;
-    return 0;
+    {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        g_blocks[fl->dev].open();
+    }
+    return device_malloc(&fl->token, 256) == hipSuccess ? 0 : -1;
 }
 template <class T>
 bool flow_array(const nbx_flow* fl, T** p, size_t* bytes) {
-    *bytes = sizeof(T) * static_cast<size_t>(fl->ncoef);
-    *p = static_cast<T*>(flow_alloc(fl->dev, *bytes));
-    return *p != nullptr;
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    const auto b = g_blocks[fl->dev].take(sizeof(T) * static_cast<size_t>(fl->ncoef));
+    *p = static_cast<T*>(b.p);
+    *bytes = b.bytes;
+    return b.p != nullptr;
 }
 }  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    bool any = false;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        any = g_blocks[dev].give_back();
+    }
+    if (any) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
 
 // (u, v) pairs in FP64, and FP32 elements pairing time index t with t + 1
 // (slab = one time slice of coefficients; the last slice repeats itself).
@@ -610,7 +596,7 @@ int launch_solve(const Flow& f, const Src& src, const SolveArgs& a, const Launch
             const size_t state_off = ring * sizeof(unsigned long long) + 256;
             // (a slot of its own for the default: a captured queue's workspace
             // is grown by requested queues only)
-            Workspace ws(s, cfg.requested ? 3 : 5,
+            Workspace ws(s, cfg.requested ? 3 : kDefaultQueueSlot,
                          state_off + solve_state_bytes<R, G>() * static_cast<size_t>(slots),
                          !cfg.requested);
             if (ws.error()) {
@@ -960,9 +946,27 @@ int nbx_ingest_xy(const double* U_xy, int nt, int ny, int nx, double scale, doub
 
 void nbx_flow_destroy(nbx_flow* fl) {
     if (!fl) return;
-    if (fl->dev >= 0)
-        flow_release(fl->dev, {{fl->coef, fl->coef_bytes}, {fl->coef32, fl->coef32_bytes}});
+    if (fl->dev >= 0) flow_release(fl);
     delete fl;
+}
+
+int nbx_release_memory(void) {
+    int dev = 0;
+    NBX_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        (void)g_blocks[dev].give_back();
+    }
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    for (auto& w : g_ws) {
+        if (std::get<0>(w.first) != dev || std::get<2>(w.first) != kDefaultQueueSlot) continue;
+        const std::unique_lock<std::mutex> unused(w.second->m, std::try_to_lock);
+        if (!unused.owns_lock() || w.second->ptr == nullptr) continue;
+        (void)hipFree(w.second->ptr);  // (waits for the device work that uses it)
+        w.second->ptr = nullptr;
+        w.second->bytes = 0;
+    }
+    return 0;
 }
 
 int nbx_flow_eval(const nbx_flow* fl, const double* params, int np, const double* t,

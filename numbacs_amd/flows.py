@@ -47,6 +47,14 @@ class FlowHandle(int):
         raise TypeError("FlowHandle refers to device memory and cannot be pickled")
 
 
+def release_memory():
+    """Give back the device memory that the library holds on the current device
+    for later calls: arrays of closed flows (at most 256 MiB, held while
+    another flow is open) and workspaces of default launches that no call is using."""
+    _lib.torch()
+    _lib.check(_lib.load().nbx_release_memory())
+
+
 def _analytic(kind):
     out = ctypes.c_void_p()
     _lib.check(_lib.load().nbx_flow_create_analytic(kind, ctypes.byref(out)))

@@ -3,13 +3,14 @@ requested launch shapes are the ones that run, default ones take no memory
 that a caller cannot spare, and sizes past 32-bit launch or index limits give
 the results of the smaller ones."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-RELAXED, GLOBAL = 2, 0  # hipStreamCaptureMode
+GLOBAL, THREAD_LOCAL, RELAXED = 0, 1, 2  # hipStreamCaptureMode
 
 
 @pytest.fixture(scope="module")
@@ -237,6 +238,92 @@ def test_captured_queue_keeps_its_workspace(lib, configs):
             graph.replay()
             stream.synchronize()
             assert torch.equal(out, eager)
+
+
+def constant_flow(n, value):
+    from numbacs_amd.flows import get_flow_2D
+
+    torch = __import__("torch")
+    C = torch.full(tuple(m + 2 for m in n), value, dtype=torch.float64, device="cuda")
+    return get_flow_2D(tuple((0.0, 1.0, m) for m in n), C, -C)
+
+
+def test_closed_flows_memory_comes_back(lib):
+    """What a closed flow leaves behind while another is open (2 x 71 MB here)
+    is given back on request, and by closing the last one; a flow of more than
+    256 MiB leaves nothing."""
+    from numbacs_amd import flows
+
+    torch = lib.torch()
+
+    def free():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        return torch.cuda.mem_get_info()[0]
+
+    n = (64, 256, 256)
+    kept = constant_flow((4, 5, 6), 1.0)
+    flows.release_memory()
+    start = free()
+    a = constant_flow(n, 2.0)
+    assert start - free() > 128 << 20
+    a.close()
+    flows.release_memory()
+    assert start - free() < 8 << 20
+    constant_flow((256, 256, 256), 2.0).close()
+    assert start - free() < 8 << 20
+    b, c = constant_flow(n, 2.0), constant_flow(n, 3.0)
+    b.close()
+    c.close()
+    kept.close()
+    assert start - free() < 8 << 20
+
+
+def test_closing_waits_for_the_flow_s_work(lib):
+    """A flow closed while a map over it runs on a side stream, and a flow of its
+    size made at once: the map is the closed flow's."""
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    n, shape = (32, 96, 96), (1200, 900)
+    kept = constant_flow((4, 5, 6), 1.0)
+    # (0.3 to the right and down: inside the unit box all the way)
+    xd, yd = (lib.to_dev(np.linspace(a, a + 0.1, m)) for a, m in zip((0.2, 0.6), shape))
+    side, out = torch.cuda.Stream(), lib.empty(shape + (2,))
+    want = None
+    for turn in range(4):
+        a = constant_flow(n, 0.5)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(8):  # some milliseconds
+                flowmap_grid_2d_device(a, 0.0, 0.6, xd, yd, [1.0], rtol=1e-10, atol=1e-13, out=out)
+        a.close()
+        b = constant_flow(n, -0.5)
+        torch.cuda.synchronize()
+        got = lib.to_host(out)
+        want = got if want is None else want
+        assert np.abs(got[..., 0] - lib.to_host(xd)[:, None] - 0.3).max() < 1e-9
+        assert np.array_equal(got, want)
+        b.close()
+    kept.close()
+
+
+@pytest.mark.parametrize("mode", [THREAD_LOCAL, RELAXED])
+def test_closing_a_flow_during_a_capture(lib, mode):
+    """Where frees are allowed -- in another thread than the capture's (batches
+    are captured that way), or in the relaxed mode -- a flow may be closed
+    while a stream is being captured; the capture goes on."""
+    kept, flow = constant_flow((4, 5, 6), 1.0), constant_flow((8, 9, 10), 2.0)
+    lib.torch().cuda.synchronize()
+    with Capture(lib, mode) as capture:
+        if mode == RELAXED:
+            flow.close()
+        else:
+            other = threading.Thread(target=flow.close)
+            other.start()
+            other.join()
+    assert capture.status == 0
+    kept.close()
 
 
 @pytest.mark.parametrize("shape", [(1, 23170, 23170), (23171, 23171, 1)])
