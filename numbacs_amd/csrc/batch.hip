@@ -140,8 +140,8 @@ int ensure_chunk_buffers(nbx_batch* b) {
     const LaunchCfg cfg = launch_cfg(b->flow->kind, b->precision);
     if (!runs_queue(cfg) || cfg.persistent < 0 || b->total_slots == 0) return 0;
     int G = (b->flow->kind == NBX_FLOW_SPLINE3 && b->flow->extrap != 1) ? cfg.lanes : 1;
-    if (b->precision == NBX_FP32_DISP ? pair_lanes<float>(b->flow, b->total)
-                                      : pair_lanes<double>(b->flow, b->total))
+    if (b->precision == NBX_FP32_DISP ? pair_lanes<float>(b->flow, b->total, b->total_slots)
+                                      : pair_lanes<double>(b->flow, b->total, b->total_slots))
         G = 2;
     const int64_t ntiles = b->total_slots / (64 / G);
     NBX_REQUIRE(ntiles < (int64_t(1) << 31), "too many particle tiles for the queue");
@@ -175,14 +175,14 @@ int launch_batch_flow(nbx_batch* b, hipStream_t s) {
         if (cfg.lanes == 2) return launch_batch_queue<Spline3<R, 2>, R, 2>(b, regroup<2>(sp), cfg, s);
         return launch_batch_queue<Spline3<R, 1>, R, 1>(b, sp, cfg, s);
     }
+    const bool pair = pair_lanes<R>(fl, b->total, b->total_slots);
     if (fl->kind == NBX_FLOW_LINEAR3)
-        return pair_lanes<R>(fl, b->total) ? launch_batch_queue<Linear3Pair<R>, R, 2>(
-                                                 b, pair_linear(make_linear<R>(fl, p[0])), cfg, s)
-                                           : launch_batch_queue<Linear3<R>, R, 1>(
-                                                 b, make_linear<R>(fl, p[0]), cfg, s);
+        return pair ? launch_batch_queue<Linear3Pair<R>, R, 2>(
+                          b, pair_linear(make_linear<R>(fl, p[0])), cfg, s)
+                    : launch_batch_queue<Linear3<R>, R, 1>(b, make_linear<R>(fl, p[0]), cfg, s);
     if (fl->kind == NBX_FLOW_DOUBLE_GYRE) {
         const DoubleGyre<R> dg{p[0], p[1], p[2], p[3], p[4], p[5]};
-        if (pair_lanes<R>(fl, b->total))
+        if (pair)
             return launch_batch_queue<DoubleGyrePair<R>, R, 2>(b, DoubleGyrePair<R>{dg}, cfg, s);
         return launch_batch_queue<DoubleGyre<R>, R, 1>(b, dg, cfg, s);
     }

@@ -797,7 +797,9 @@ int dispatch_solve(const nbx_flow* fl, const double* params, int np, const Src& 
     }
     // (the auxiliary grid's one-lane kernels of these flows contract a few
     // operations differently from the grid's: they stay, for the same results)
-    const bool pair = !std::is_same<Src, AuxSource>::value && pair_lanes<R>(fl, a.P);
+    int64_t slots = a.P;
+    if constexpr (std::is_same<Src, GridSource>::value) slots = src.slots();
+    const bool pair = !std::is_same<Src, AuxSource>::value && pair_lanes<R>(fl, a.P, slots);
     if (fl->kind == NBX_FLOW_LINEAR3)
         return pair ? launch_solve<Linear3Pair<R>, R, 2>(
                           pair_linear(make_linear<R>(fl, params[0])), src, a, cfg, s)

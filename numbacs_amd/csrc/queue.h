@@ -95,13 +95,16 @@ struct IsSpline3<Spline3<R, G, L, S>> : std::true_type {};
 // work.  Trilinear maps are bound by their longest trajectories (518 steps
 // against 112 on average) at every size: 1,768 particles 4.8 -> 3.1 ms,
 // 169,676 7.3 -> 6.5, 676,851 14.1 -> 12.6; their pair indexes samples with
-// 32 bits.  The double gyre's pair spends a fifth more instructions, so it
+// 32 bits, and one launch holds fewer than 2^32 threads (slots: of the launch,
+// the particles in tile order).  The double gyre's pair spends a fifth more instructions, so it
 // stays below two (float: four) wavefronts per SIMD of the one-lane form:
 // FP64 3,321 particles 187 -> 120 us, 80,601 289 -> 240, 180,901 376 -> 394;
 // float 80,601 220 -> 179, 180,901 289 -> 286, 721,801 857 -> 880.
 template <class R>
-inline bool pair_lanes(const nbx_flow* fl, int64_t P) {
-    if (fl->kind == NBX_FLOW_LINEAR3) return fl->ncoef < (int64_t(1) << 31);
+inline bool pair_lanes(const nbx_flow* fl, int64_t P, int64_t slots) {
+    constexpr int64_t limit = int64_t(1) << 31;
+    if (fl->kind == NBX_FLOW_LINEAR3)  // (a block is up to 256 threads)
+        return fl->ncoef < limit && slots <= limit - 256;
     return fl->kind == NBX_FLOW_DOUBLE_GYRE &&
            P <= static_cast<int64_t>(device_cu_count()) * (sizeof(R) == 4 ? 1024 : 512);
 }

@@ -350,3 +350,25 @@ def test_prefilter_of_more_lines_than_one_launch_holds(lib, shape):
     assert float((c - u).abs().max()) < 64 * 2.0 ** -52 * 4.5
     del U, C, planes, c, u
     torch.cuda.empty_cache()
+
+
+def test_trilinear_map_of_more_threads_than_a_pair_launch_holds(lib):
+    """2^31 particles, all but one row masked: one lane each fits a launch, two
+    do not."""
+    from numbacs_amd.flows import get_flow_linear_2D
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    n = (4, 9, 8)
+    U = np.random.default_rng(2).standard_normal((2,) + n)
+    f = get_flow_linear_2D(tuple((0.0, 1.0, m) for m in n), U[0], U[1])
+    nx, ny, row = 65536, 32768, 40000
+    xd, yd = (torch.linspace(0, 1, m, dtype=torch.float64, device="cuda") for m in (nx, ny))
+    mask = torch.ones((nx, ny), dtype=torch.uint8, device="cuda")
+    mask[row] = 0
+    got = flowmap_grid_2d_device(f, 0.1, 0.3, xd, yd, [1.0], maskd=mask)
+    want = flowmap_grid_2d_device(f, 0.1, 0.3, xd[row:row + 1].contiguous(), yd, [1.0])
+    assert torch.equal(got[row], want[0])
+    assert not got[row - 1].any() and not got[row + 1].any() and not got[-1].any()
+    del got, mask
+    torch.cuda.empty_cache()
