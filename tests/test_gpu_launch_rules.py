@@ -372,3 +372,32 @@ def test_trilinear_map_of_more_threads_than_a_pair_launch_holds(lib):
     assert not got[row - 1].any() and not got[row + 1].any() and not got[-1].any()
     del got, mask
     torch.cuda.empty_cache()
+
+
+def test_output_layer_backward_of_many_narrow_rows(lib):
+    """2^26 rows of 8 columns: the deltas of the first and last rows against
+    two roundings to bf16 from float64."""
+    torch = lib.torch()
+    n, width = 1 << 26, 8
+    dev = dict(device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    h = torch.zeros((n, width), dtype=torch.bfloat16, **dev)
+    dy = torch.rand((n, 2), generator=gen, **dev)
+    pre = torch.rand((n, width), generator=gen, **dev)
+    W = torch.rand((width, 2), generator=gen, **dev).to(torch.bfloat16)
+    gW, gb = torch.empty((width, 2), **dev), torch.empty(2, **dev)
+    da = torch.full((n, width), float("nan"), dtype=torch.bfloat16, **dev)
+    lib.check(lib.load().nbx_mlp_out_backward(
+        lib.ptr(dy), lib.ptr(h), lib.ptr(pre), n, width, lib.ptr(W), lib.ptr(gW), lib.ptr(gb),
+        lib.ptr(da), lib.stream_ptr()))
+    assert not da.isnan().any() and not gW.any()
+    for part in (slice(0, 999), slice(n - 1001, n)):
+        p = pre[part].double()
+        t = torch.tanh(0.7978845608028654 * (p + 0.044715 * p ** 3))
+        slope = 0.5 * (1 + t) + 0.5 * p * (1 - t ** 2) * 0.7978845608028654 * (
+            1 + 3 * 0.044715 * p ** 2)
+        dh = dy[part].double() @ W.double().T
+        err = (2.0 ** -7 * dh + 2.0 ** -21 * dh) * slope.abs() + 1e-5 * dh
+        assert ((da[part].double() - dh * slope).abs() <= err).all()
+    del h, dy, pre, da
+    torch.cuda.empty_cache()
