@@ -394,6 +394,14 @@ __device__ __forceinline__ double clamped(double q, double lo, double hi) {
     return raw_min(raw_max(q, lo), hi);
 }
 
+// Byte offset of the element g past the key-th, in an array of up to 4 GiB: beyond
+// 2 GiB only unsigned arithmetic holds it.
+__host__ __device__ constexpr unsigned element_offset(double key, int g, unsigned size) {
+    return (static_cast<unsigned>(key) + static_cast<unsigned>(g)) * size;
+}
+static_assert(element_offset((1 << 28) - 4, 3, 16) == 0xfffffff0u,
+              "the last element below 4 GiB (a signed product overflows: no constant)");
+
 // A box of coefficient elements copied to LDS by a one-wavefront block for
 // the stencils of one DOP853 step (cells it0.., ix0.., iy0.. of the
 // coefficient array, bt x bx x by elements, y fastest): a stencil whose 4 x 4
@@ -488,10 +496,10 @@ struct Spline3 {
             const_cast<P*>(C), 0, static_cast<int>(cbytes), 0x00020000);
         // (time slices step the vector offset, x rows are the scalar offsets:
         // three live scalars, not sixteen)
-        const int vo = (static_cast<int>(key) + g) * static_cast<int>(sizeof(P));
-        const int tstep =
-            (sizeof(R) == sizeof(double) ? 1 : 2) * st * static_cast<int>(sizeof(P));
-        const int xstep = sx * static_cast<int>(sizeof(P));
+        const unsigned vo = element_offset(key, g, sizeof(P));
+        const unsigned tstep =
+            (sizeof(R) == sizeof(double) ? 1u : 2u) * static_cast<unsigned>(st) * sizeof(P);
+        const unsigned xstep = static_cast<unsigned>(sx) * sizeof(P);
 #pragma unroll
         for (int a = 0; a < kRows / 4; ++a)
 #pragma unroll

@@ -326,6 +326,38 @@ def test_closing_a_flow_during_a_capture(lib, mode):
     kept.close()
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_spline_arrays_above_2_gib(lib, precision):
+    """The 4-lane kernel's 32-bit offsets at the far end of a coefficient array
+    of 2.7 GB: a unit-spaced grid's last corner against a flow of that corner's
+    coefficients alone.  Cell positions are exact in both, so the bits are
+    equal."""
+    from numbacs_amd.flows import get_flow_2D
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    n, first = (18, 1022, 8190), (0, 1000, 8160)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    C = [torch.zeros(tuple(m + 2 for m in n), dtype=torch.float64, device="cuda")
+         for _ in range(2)]
+    corner = []
+    for c in C:
+        part = c[:, first[1]:, first[2]:]
+        part.copy_(torch.rand(part.shape, generator=gen, dtype=torch.float64, device="cuda") - 0.5)
+        corner.append(part.contiguous())
+    big = get_flow_2D(tuple((0.0, m - 1.0, m) for m in n), *C)
+    small = get_flow_2D(tuple((float(a), m - 1.0, m - a) for a, m in zip(first, n)), *corner)
+    del C, c, part
+    xd, yd = (lib.to_dev(np.linspace(a + 6.0, m - 5.0, 37)) for a, m in zip(first[1:], n[1:]))
+    got, want = (flowmap_grid_2d_device(f, 13.0, 3.5, xd, yd, [1.0], precision=precision)
+                 for f in (big, small))
+    assert float((got - torch.stack(torch.meshgrid(xd, yd, indexing="ij"), -1)).abs().max()) > 0.1
+    assert torch.equal(got, want)
+    big.close()
+    small.close()
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("shape", [(1, 23170, 23170), (23171, 23171, 1)])
 def test_prefilter_of_more_lines_than_one_launch_holds(lib, shape):
     """Axes of one sample with 2^29 lines and more across them (8 threads of the
