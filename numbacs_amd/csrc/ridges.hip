@@ -1253,12 +1253,14 @@ extern "C" {
 int nbx_percentile(const double* f, int64_t n, double q, double* result, nbx_stream stream) {
     NBX_REQUIRE(f != nullptr && result != nullptr, "NULL array");
     hipStream_t s = as_stream(stream);
-    const int64_t held = n < 0 ? 0 : n < kSelHeld ? n : kSelHeld;
-    Workspace ws(s, 2, align256(sizeof(SelState)) + 8 * held);
+    // (one size for every n: a stream's first call allocates, and no later one
+    // grows the buffer, so a call may be captured once any has run, and a captured
+    // one keeps its buffer)
+    Workspace ws(s, 2, align256(sizeof(SelState)) + 8 * kSelHeld);
     if (ws.error()) return ws.error();
     Arena A{ws.get(), 0};
     auto* st = A.take<SelState>(1);
-    return percentile_device(f, n, q, st, A.take<unsigned long long>(held), result, s);
+    return percentile_device(f, n, q, st, A.take<unsigned long long>(kSelHeld), result, s);
 }
 
 int nbx_ridge_pts(const double* f, const double* evec, const double* x, int nx, const double* y,

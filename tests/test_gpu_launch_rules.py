@@ -433,3 +433,37 @@ def test_output_layer_backward_of_many_narrow_rows(lib):
         assert ((da[part].double() - dh * slope).abs() <= err).all()
     del h, dy, pre, da
     torch.cuda.empty_cache()
+
+
+def test_captured_percentile_keeps_its_workspace(lib):
+    """Once any percentile has run on a stream a larger one may be captured there
+    without an allocation, and larger ones run after it do not grow the
+    workspace away from under the graph.  Replayed several times."""
+    torch = lib.torch()
+    rng = np.random.default_rng(4)
+    few, some, many = (lib.to_dev(rng.standard_normal(n)) for n in (100, 5000, 300001))
+    result, eager = lib.empty((2,)), lib.empty((2,))
+    hip, handle = ctypes.CDLL(lib.LIB_PATH), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(handle), 1) == 0  # without a workspace yet
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.ExternalStream(handle.value), torch.cuda.CUDAGraph()
+
+    def percentile(f, out):
+        lib.check(lib.load().nbx_percentile(lib.ptr(f), f.numel(), 90.0, lib.ptr(out),
+                                            lib.stream_ptr()))
+
+    with torch.cuda.stream(stream):
+        percentile(few, eager)
+        with torch.cuda.graph(graph, stream=stream):
+            percentile(some, result[:1])
+            percentile(many, result[1:])
+        for _ in range(3):
+            percentile(many, eager[1:])
+            result.zero_()
+            graph.replay()
+            percentile(some, eager[:1])
+            stream.synchronize()
+            assert torch.equal(result, eager)
+    for k, f in enumerate((some, many)):
+        ref = np.percentile(lib.to_host(f), 90.0)
+        assert abs(float(eager[k]) - ref) <= 4 * np.spacing(abs(ref))
