@@ -109,17 +109,21 @@ __global__ void k_sel_init(SelState* st, long long k_lo, long long k_hi) {
 
 // Digit state of both searches after pass `prev`, into LDS: the bin whose
 // cumulative count first exceeds k.  Called by all kSelThreads threads,
-// kSelOwn neighbouring bins each; ends with a barrier.
+// kSelOwn neighbouring bins each; ends with a barrier.  Sum holds the number of
+// keys: 32 bits below 2^32 of them, as every grid has (64 bits throughout: FTLE
+// and ridges of 8 M values 333 -> 337 us).
+template <class Sum>
 __device__ void sel_advance(const SelState* st, int prev, unsigned long long* sp,
                             unsigned long long* sm, long long* sk) {
-    __shared__ unsigned int waves[2][kSelThreads / 64];
+    __shared__ Sum waves[2][kSelThreads / 64];
     const int t = threadIdx.x, lane = t & 63;
     const int sb = prev & 1, hb = prev % 3;
     const int same = st->prefix[sb][0] == st->prefix[sb][1];
-    unsigned int c[2][kSelOwn], before[2];
+    unsigned int c[2][kSelOwn];
+    Sum before[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        unsigned int x = 0;
+        Sum x = 0;
 #pragma unroll
         for (int q = 0; q < kSelOwn; ++q) {
             c[s][q] = st->hist[hb][same ? 0 : s][kSelOwn * t + q];
@@ -128,7 +132,7 @@ __device__ void sel_advance(const SelState* st, int prev, unsigned long long* sp
         before[s] = x;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
-            const unsigned int y = __shfl_up(x, off);
+            const Sum y = __shfl_up(x, off);
             if (lane >= off) x += y;
         }
         before[s] = x - before[s];
@@ -139,7 +143,7 @@ __device__ void sel_advance(const SelState* st, int prev, unsigned long long* sp
     for (int s = 0; s < 2; ++s) {
         for (int w = 0; w < (t >> 6); ++w) before[s] += waves[s][w];
         const long long k = st->k[sb][s];
-        long long at = before[s];
+        long long at = static_cast<long long>(before[s]);
 #pragma unroll
         for (int q = 0; q < kSelOwn; ++q) {
             // exactly one bin has at <= k < at + count (k < total always holds)
@@ -178,6 +182,7 @@ __device__ __forceinline__ void sel_count(unsigned int* h, unsigned int bin, boo
 // Bound by the reads (13 us of the 17 to 21 a pass over 8 M values takes; then
 // 5.5 us a pass over the list): the whole percentile 156 -> 84 us, with digits of
 // 8 bits and every pass over the array before.
+template <class Sum>
 __global__ __launch_bounds__(kSelThreads) void k_sel_hist(const double* __restrict__ f, int64_t n,
                                                           SelState* st, int pass,
                                                           unsigned long long* held,
@@ -202,7 +207,7 @@ __global__ __launch_bounds__(kSelThreads) void k_sel_hist(const double* __restri
         }
         __syncthreads();
     } else {
-        sel_advance(st, pass - 1, sp, sm, sk);
+        sel_advance<Sum>(st, pass - 1, sp, sm, sk);
     }
     if (blockIdx.x == 0) {
         if (pass > 0 && t < 2) {
@@ -284,11 +289,12 @@ __global__ __launch_bounds__(kSelThreads) void k_sel_hist(const double* __restri
 
 // The last digit, then numpy's _lerp: a + (b-a)*g, or b - (b-a)*(1-g) when
 // g >= 0.5.
+template <class Sum>
 __global__ __launch_bounds__(kSelThreads) void k_sel_finish(SelState* st, double gamma,
                                                             double* out) {
     __shared__ unsigned long long sp[2], sm[2];
     __shared__ long long sk[2];
-    sel_advance(st, kSelPasses - 1, sp, sm, sk);
+    sel_advance<Sum>(st, kSelPasses - 1, sp, sm, sk);
     if (threadIdx.x != 0) return;
     const double a = key_value(sp[0]);
     const double b = key_value(sp[1]);
@@ -318,13 +324,16 @@ int percentile_device(const double* f, int64_t n, double q, SelState* st,
     // one turn of 4 keys a thread, at most a block a CU: every block adds its
     // nonzero bins to the same global counters (8 M values: 75 us for the passes;
     // 512 blocks 77, of half the threads 83)
+    const bool narrow = n < int64_t(1) << 32;
+    auto* hist = narrow ? &k_sel_hist<unsigned int> : &k_sel_hist<unsigned long long>;
+    auto* finish = narrow ? &k_sel_finish<unsigned int> : &k_sel_finish<unsigned long long>;
     unsigned nb = blocks_for(n, kSelThreads * 4);
     if (nb > 256) nb = 256;
     for (int pass = 0; pass < kSelPasses; ++pass) {
-        k_sel_hist<<<nb, kSelThreads, 0, s>>>(f, n, st, pass, held, n < kSelHeld ? n : kSelHeld);
+        hist<<<nb, kSelThreads, 0, s>>>(f, n, st, pass, held, n < kSelHeld ? n : kSelHeld);
         NBX_LAUNCHED("sel_hist");
     }
-    k_sel_finish<<<1, kSelThreads, 0, s>>>(st, gamma, out);
+    finish<<<1, kSelThreads, 0, s>>>(st, gamma, out);
     NBX_LAUNCHED("sel_finish");
     return 0;
 }

@@ -467,3 +467,19 @@ def test_captured_percentile_keeps_its_workspace(lib):
     for k, f in enumerate((some, many)):
         ref = np.percentile(lib.to_host(f), 90.0)
         assert abs(float(eager[k]) - ref) <= 4 * np.spacing(abs(ref))
+
+
+def test_percentile_of_more_than_2_to_the_32_values(lib):
+    """Counts past 32 bits: whole numbers around zero, of which no digit's bin
+    holds as many; those from 2^33 up have more below them."""
+    torch = lib.torch()
+    n, low = 3 << 31, -(3 << 30)
+    f, out = lib.empty((n,)), lib.empty((1,))
+    for a in range(0, n, 1 << 30):  # (one call makes fewer than 2^32)
+        torch.arange(low + a, low + a + (1 << 30), out=f[a:a + (1 << 30)]).mul_(4)
+    for q in (0.0, 25.0, 50.0, 75.0, 99.0, 100.0):
+        lib.check(lib.load().nbx_percentile(lib.ptr(f), n, q, lib.ptr(out), lib.stream_ptr()))
+        # numpy's virtual index from low; it and the lerp round some 2^33 a few times
+        assert abs(float(out[0]) / 4 - (low + (n - 1) * (q / 100.0))) <= 4 * np.spacing(2.0 ** 33)
+    del f
+    torch.cuda.empty_cache()
