@@ -327,29 +327,28 @@ __global__ void k_loss(const float* __restrict__ y, const float* __restrict__ ta
 
 // da = bf16(bf16(dy W_out^T) * gelu'(pre)) for the last hidden layer, kOutStep
 // rows' element of one column a thread: no division by the width, the column's
-// weights read once (8192 x 256: 7.6 -> 5 us).  Rows beyond kOutBlocks groups are
-// taken in further turns: a launch holds fewer than 2^32 threads.
-constexpr int kOutStep = 4, kOutBlocks = 1 << 23;
+// weights read once (8192 x 256: 7.6 -> 5 us).  Groups of rows beyond kOutBlocks lie
+// along the grid's y: a grid extent holds fewer than 2^32 threads.
+constexpr int kOutStep = 4;
+constexpr int64_t kOutBlocks = 1 << 23;
 
 __global__ __launch_bounds__(256) void k_out_bwd_data(const float* __restrict__ dy, int64_t n,
                                                       int width, const uint16_t* __restrict__ W,
                                                       const float* __restrict__ pre,
                                                       uint16_t* __restrict__ da) {
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.y) * kOutBlocks + blockIdx.x) * kOutStep;
     for (int k = threadIdx.x; k < width; k += blockDim.x) {
         const float w0 = bf2f(W[2 * k]), w1 = bf2f(W[2 * k + 1]);
-        for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kOutStep; r0 < n;
-             r0 += static_cast<int64_t>(gridDim.x) * kOutStep) {
-            float p[kOutStep];
+        float p[kOutStep];
 #pragma unroll
-            for (int q = 0; q < kOutStep; ++q)
-                p[q] = pre[(r0 + q < n ? r0 + q : n - 1) * width + k];
+        for (int q = 0; q < kOutStep; ++q)
+            p[q] = pre[(r0 + q < n ? r0 + q : n - 1) * width + k];
 #pragma unroll
-            for (int q = 0; q < kOutStep; ++q) {
-                const int64_t r = r0 + q;
-                if (r >= n) break;
-                const float dh = bf2f(f2bf(dy[2 * r] * w0 + dy[2 * r + 1] * w1));
-                da[r * width + k] = f2bf(dh * gelu_grad(p[q]));
-            }
+        for (int q = 0; q < kOutStep; ++q) {
+            const int64_t r = r0 + q;
+            if (r >= n) break;
+            const float dh = bf2f(f2bf(dy[2 * r] * w0 + dy[2 * r + 1] * w1));
+            da[r * width + k] = f2bf(dh * gelu_grad(p[q]));
         }
     }
 }
@@ -846,8 +845,9 @@ int nbx_mlp_out_backward(const float* dy, const uint16_t* h, const float* pre, i
     k_out_bwd_weight<<<static_cast<unsigned>((n + kSumRows - 1) / kSumRows), kSumThreads, 0, s>>>(
         h, dy, n, width, gW, gb);
     const int64_t groups = (n + kOutStep - 1) / kOutStep;
-    k_out_bwd_data<<<static_cast<unsigned>(groups < kOutBlocks ? groups : kOutBlocks), 256, 0, s>>>(
-        dy, n, width, W, pre, da);
+    const dim3 grid(static_cast<unsigned>(groups < kOutBlocks ? groups : kOutBlocks),
+                    static_cast<unsigned>((groups + kOutBlocks - 1) / kOutBlocks));
+    k_out_bwd_data<<<grid, 256, 0, s>>>(dy, n, width, W, pre, da);
     NBX_LAUNCHED("mlp_out_bwd");
     return 0;
 }
