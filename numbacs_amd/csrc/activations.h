@@ -53,8 +53,8 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 // It differs from gelu(a) by less than (d + 6) units in its last float place,
 // d = 1 + exp(-2 inner) (the library form's own rounding grows with d: 1 + tanh
 // cancels), so undecided is set where a bf16 rounding boundary (low half
-// 0x8000) is that near.  Checked for every float: where undecided is not set,
-// both round to the same bf16.
+// 0x8000) is that near.  Checked for every float (tests/native): where undecided
+// is not set, both round to the same bf16.
 __device__ __forceinline__ float gelu_near(float a, bool& undecided) {
     constexpr float c0 = -2.0f * 1.4426950408889634f * kGeluC, c1 = c0 * kGeluA;
     const float d = 1.0f + __builtin_amdgcn_exp2f(a * fmaf(c1, a * a, c0));

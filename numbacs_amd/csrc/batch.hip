@@ -1,8 +1,8 @@
 // Batched FTLE time series: many flow-map requests (each its own window
-// t0, T and particle grid) over one flow, integrated by one launch -- the
-// persistent queue of particle tiles, or one non-persistent launch over
-// every request's tiles (the launch configuration's persistent occupancy 0;
-// the autotuner picks the faster) -- followed by one batched FTLE launch over
+// t0, T and particle grid) over one flow, integrated by one launch -- one
+// non-persistent launch over every request's tiles, or, where the launch
+// configuration asks for it, the persistent queue of particle tiles (the
+// autotuner picks the faster) -- followed by one batched FTLE launch over
 // every request's grid.  The pair can be captured once into a HIP graph and
 // replayed.  Requests run longest window first (the tile launch dispatches
 // blocks in order, so the longest solves do not form the launch's tail).

@@ -28,7 +28,8 @@ namespace nbx {
 
 // Launch shape per (flow kind, precision), set by the autotuner through
 // nbx_set_launch_config:
-//   lanes       lanes per particle for spline flows (1, 2 or 4);
+//   lanes       lanes per particle for spline flows (1, 2 or 4; for the double
+//               gyre and trilinear flows see pair_lanes);
 //   block       threads per block (64, 128 or 256);
 //   persistent  0: one group per particle, one launch covering all of them;
 //               n > 0: a persistent grid of n blocks per CU pulling

@@ -2,9 +2,9 @@
 //
 // Reference path: flowmap_grid_2D (integration.py:123-182) runs one
 // numbalsoda.dop853 solve per grid point over a numba cfunc right-hand side.
-// Here one GPU thread owns one particle: the right-hand side is a device
-// functor inlined into the integrator, the state stays in registers for the
-// whole solve, and the final position is written once, coalesced.
+// Here a lane, or a group of two or four, owns one particle: the right-hand side
+// is a device functor inlined into the integrator, the state stays in registers
+// (and LDS) for the whole solve, and the final position is written once.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -284,8 +284,10 @@ struct AuxSource {
     __device__ __forceinline__ int64_t cell(int64_t p) const { return p / naux; }
 };
 
-// One solve per group of G lanes (G = 1 for analytic flows); the group's
-// lanes run identical solver arithmetic and split the spline gathers.
+// One solve per group of G lanes.  With G = 1 the lane holds both components;
+// in groups of 2 or 4 even lanes hold x and odd lanes y (Solve in dop853.h), and
+// the group's lanes split the right-hand side: the spline's gathers, the
+// trilinear flow's time slices, the double gyre's library calls.
 template <class Flow, class R, int G, class Src>
 __global__ __launch_bounds__(256, (flowmap_min_waves<Flow, R, G>())) void k_flowmap(
     Flow f, Src src, int64_t P, double s0, double s1, double rtol, double atol,

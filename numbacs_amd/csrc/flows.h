@@ -356,8 +356,9 @@ __device__ __forceinline__ R group_component(R u, R v, bool odd) {
 // the clamped point times the outward offset.  L says whether that gradient
 // path is compiled in: it is the register-heaviest code of the functor, and
 // kernels built without it (L = false) serve modes 0 and 2 with fewer
-// registers (FP32 4-lane flow map: 167 instead of 234 VGPRs, 3 waves per
-// SIMD instead of 2; FP64: 221 instead of 256).
+// registers (one lane per particle: FP64 142 instead of 250, FP32 192 instead
+// of 238).
+
 // A uniform double moved into a vector register pair.  The flow kernels hold
 // the spline's box and spacing for their whole solve; in scalar registers
 // (next to the solver's constants and the kernel's pointers) they spill to
@@ -964,7 +965,8 @@ struct Linear3 {
 // the even lane gathers and sums time slice it, the odd lane slice it + 1 (four
 // samples each instead of eight), and each finishes its own component.  By the
 // operations of Linear3, its three quotients by the grid steps taken with
-// their reciprocals (div_with: an IEEE division's result).
+// their reciprocals (div_with: an IEEE division's result, for offsets from the
+// box's edge down to 2^-969).
 template <class R>
 struct Linear3Pair {
     static constexpr bool kStagesInLds = false;

@@ -7,11 +7,12 @@
 //
 // GEMM tiling: a 256-thread block computes a 64x64 tile of C = A * B; each of
 // its four wavefronts owns a 32x32 quarter as 2x2 MFMA 16x16 tiles.  K runs
-// in steps of 32: the block stages a 64x32 slice of A and a 32x64 slice of B
-// in LDS with k contiguous (rows padded to 40 elements against bank
+// in turns of 128: the block stages a 64x128 slice of A and a 128x64 slice of B
+// in LDS with k contiguous (chunks of 8 k permuted by row against bank
 // conflicts), transposing on the way in when the operand is stored with the
 // other dimension contiguous, so forward (X W), backward-data (dY W^T) and
-// backward-weight (X^T dY) products all use the same kernel.
+// backward-weight (X^T dY) products all use the same kernel, and multiplies
+// them in steps of 32.
 //
 // MFMA operand layout (v_mfma_f32_16x16x32_bf16, wave64): lane l supplies
 // A[l % 16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l % 16]; it receives

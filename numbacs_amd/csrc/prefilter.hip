@@ -31,8 +31,9 @@ namespace {
 // The quotient by the k-th pivot p[k] = 4 - cp[k-1] uses cp[k] = 1/p[k], the
 // correctly rounded reciprocal the back substitution needs anyway: product,
 // exact remainder, correction (Markstein), equal to the IEEE quotient on 4e7
-// sampled dividends for each of the pivots; the fix-up keeps infinities and
-// NaN as a division gives them.  cp reaches its fixed point by k = 13.
+// sampled dividends for each of the pivots (dividends below 2^-969, whose
+// remainder underflows, aside); the fix-up keeps infinities and NaN as a
+// division gives them.  cp reaches its fixed point by k = 13.
 constexpr int kThreads = 256;
 constexpr int kPivots = 16;
 struct Pivots {
