@@ -120,6 +120,13 @@ def load():
             raise RuntimeError(
                 f"numbacs_amd: {LIB_PATH} is not built; run __graft_entry__.build() "
                 "(make -C numbacs_amd/csrc)")
+        try:
+            # torch carries a HIP runtime of its own: loaded first, it is the
+            # one that the library binds to as well (two in a process crash at
+            # the first tensor)
+            import torch  # noqa: F401
+        except ImportError:
+            pass
         L = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(L, name)

@@ -84,3 +84,22 @@ def test_pmc_dispatch_mean_parses_counter_csv(tmp_path):
             fh.write(f'{d},"{k}",FETCH_SIZE,{v}\n')
     assert bench.pmc_dispatch_mean(str(path), ("k_flowmap", "Spline3<double")) == (90.0, 2)
     assert bench.pmc_dispatch_mean(str(path), ("copyBuffer",)) is None
+
+
+def test_one_hip_runtime_in_the_process():
+    """A program whose first call loads the library, torch only afterwards: both
+    use the runtime that torch brings."""
+    import subprocess
+    import sys
+
+    from conftest import ROOT
+
+    program = (
+        "from numbacs_amd.flows import get_predefined_flow\n"
+        "get_predefined_flow('double_gyre')\n"
+        "import torch\n"
+        "maps = {line.split()[-1] for line in open('/proc/self/maps') if 'libamdhip64' in line}\n"
+        "print(len(maps))\n")
+    out = subprocess.run([sys.executable, "-c", program], cwd=ROOT, check=True,
+                         capture_output=True, text=True).stdout
+    assert out.split() == ["1"]
