@@ -365,6 +365,20 @@ __device__ __forceinline__ double pair_sumsq(double e) {
     return quad_move<kPairEven>(fma(e, e, quad_move<kPairOdd>(e * e)));
 }
 
+// The step's error norm from a pair's scaled errors of third and fifth order
+__device__ __forceinline__ double pair_norm(double e2, double e5, double h) {
+    const double err2 = pair_sumsq(e2), err = pair_sumsq(e5);
+    double deno = fma(0.01, err2, err);
+    if (deno <= 0.0) deno = 1.0;
+    return fabs(h) * err * sqrt(1.0 / (2 * deno));
+}
+// ... and from the errors by the divisions themselves, out of line
+[[maybe_unused]] __device__ __attribute__((noinline)) static double pair_norm_far(double n2, double n5,
+                                                                                 double sk,
+                                                                                 double h) {
+    return pair_norm(n2 / sk, n5 / sk, h);
+}
+
 template <class R>
 struct Dop853Lane {
     double x, xend, h, hmax, posneg;
@@ -516,14 +530,12 @@ __device__ __forceinline__ bool dop853_step_body(const Flow& f, Dop853Lane<R>& s
     const double pn = fma(h, k4n, y);
     const double sk = fma(rtol, fmax(fabs(y), fabs(pn)), atol);
     const double rsk = div_recip(sk);
-    const double e2 = div_with(
-        fma(-bhh3, K, fma(-bhh2, ks.get(6), fma(-bhh1, ks.get(0), k4n))), sk, rsk);
-    const double e5 = div_with(fma(er12, K, E), sk, rsk);
-    const double err2 = pair_sumsq(e2);
-    double err = pair_sumsq(e5);
-    double deno = fma(0.01, err2, err);
-    if (deno <= 0.0) deno = 1.0;
-    err = fabs(h) * err * sqrt(1.0 / (2 * deno));
+    const double n2 = fma(-bhh3, K, fma(-bhh2, ks.get(6), fma(-bhh1, ks.get(0), k4n)));
+    const double n5 = fma(er12, K, E);
+    double err = pair_norm(div_with(n2, sk, rsk), div_with(n5, sk, rsk), h);
+    // (no number: also where the scale is subnormal -- an absolute tolerance of
+    // zero and a coordinate near zero -- and has no reciprocal)
+    if (__builtin_expect(err != err, 0)) err = pair_norm_far(n2, n5, sk, h);
     const double fac = dop::root8(err) / safe;
     const bool accept = err <= 1.0;
     double hnew = h / (accept ? fmax(facc2, fmin(facc1, fac)) : fmin(facc1, fac));

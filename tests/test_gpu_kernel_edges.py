@@ -341,3 +341,45 @@ def test_output_layer_of_any_width(n, width):
     dh, mag = dy @ W.T, dy.abs() @ W.abs().T
     err = (2.0 ** -7 * dh.abs() + 4 * ulp * mag) * slope.abs() + 1e-5 * dh.abs()
     assert ((da - dh * slope).abs() <= err).all()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind", ["double_gyre", "spline", "trilinear"])
+def test_zero_absolute_tolerance_near_zero(kind, precision):
+    """Error norms whose scale rtol |y| is subnormal: the lane groups' quotients
+    by a shared reciprocal hand over to the division there.  The double gyre's
+    pair equals its one-lane form bit for bit; gridded flows of velocities
+    as small end every solve."""
+    from numbacs_amd import _lib
+    from numbacs_amd.flows import get_flow_2D, get_flow_linear_2D, get_predefined_flow
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    v = np.array([1e-310, -3e-308, 2e-303, 1e-300, -1e-285, 1e-270, 1e-200, 0.3])
+    rng = np.random.default_rng(8)
+    if kind == "double_gyre":
+        flow, p, _ = get_predefined_flow(kind, int_direction=-1.0)
+        T = 3.0
+    else:
+        n = (6, 9, 8)
+        U, V = rng.uniform(0.5, 1.5, (2,) + n) * 1e-300
+        grid = ((0.0, 5.0, n[0]), (-1.0, 1.0, n[1]), (-1.0, 1.0, n[2]))
+        if kind == "spline":
+            from numbacs_amd.flows import prefilter3_device
+
+            flow = get_flow_2D(grid, prefilter3_device(U), prefilter3_device(V))
+        else:
+            flow = get_flow_linear_2D(grid, U, V)
+        p, T = np.array([1.0]), 2.0
+
+    def run(xs, ys):
+        st, ns = (_lib.empty((len(xs), len(ys)), "i32") for _ in range(2))
+        fm = flowmap_grid_2d_device(flow, 0.5, T, _lib.to_dev(xs), _lib.to_dev(ys), p, atol=0.0,
+                                    precision=precision, status=st, nsteps=ns)
+        return [_lib.to_host(a) for a in (fm, st, ns)]
+
+    fm, status, steps = run(v, v)
+    assert (status == 1).all()
+    if kind == "double_gyre":
+        xs = np.concatenate([v, np.full(100000, 1.0)])  # one lane per particle
+        for a, b in zip((fm, status, steps), run(xs, v)):
+            assert np.array_equal(a, b[:len(v)])
