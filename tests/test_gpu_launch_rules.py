@@ -483,3 +483,40 @@ def test_percentile_of_more_than_2_to_the_32_values(lib):
         assert abs(float(out[0]) / 4 - (low + (n - 1) * (q / 100.0))) <= 4 * np.spacing(2.0 ** 33)
     del f
     torch.cuda.empty_cache()
+
+
+def test_releasing_memory_beside_running_maps(lib):
+    """A thread that keeps releasing the library's memory while another runs
+    default Bickley maps, whose queue's workspace it may take as soon as a launch
+    is enqueued: it waits for the work, and the maps stay the same."""
+    from numbacs_amd import flows
+    from numbacs_amd.integration import flowmap_grid_2d_device
+
+    torch = lib.torch()
+    flow, p, dom = flows.get_predefined_flow("bickley_jet")
+    xd, yd = (lib.to_dev(np.linspace(*d, n)) for d, n in zip(dom, (801, 401)))
+    want = flowmap_grid_2d_device(flow, 0.0, 3.0, xd, yd, p)
+    outs = [lib.empty((801, 401, 2)) for _ in range(12)]
+    torch.cuda.synchronize()
+    done, errors = threading.Event(), []
+
+    def release():
+        try:
+            while not done.is_set():
+                flows.release_memory()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    thread = threading.Thread(target=release)
+    thread.start()
+    try:
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for out in outs:
+                flowmap_grid_2d_device(flow, 0.0, 3.0, xd, yd, p, out=out)
+        torch.cuda.synchronize()
+    finally:
+        done.set()
+        thread.join()
+    assert not errors
+    for out in outs:
+        assert torch.equal(out, want)
