@@ -125,7 +125,7 @@ def load():
             # one that the library binds to as well (two in a process crash at
             # the first tensor)
             import torch  # noqa: F401
-        except ImportError:
+        except (ImportError, OSError):  # not there, or not loadable here
             pass
         L = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
